@@ -22,7 +22,7 @@ import kuqcd_amd.api as A
 
 DEV = "cuda"
 #: lowest and highest eigenvalue of -DD that the iteration counts of work() assume (weak links of the kind above)
-EIG_LOW, EIG_HIGH = 4e-3, 3.6
+EIG_LOW, EIG_HIGH = 4e-3, 4.2
 
 
 def listed():
