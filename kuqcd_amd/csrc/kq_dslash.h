@@ -8,7 +8,12 @@ namespace kq {
 enum DslashEpilogue {
     EPI_STORE = 0,     // dst = D src
     EPI_AXMY_DOT = 1,  // dst = sigma[r] * aux - D src ; partial[r][blk] = Re<aux, dst>
+    EPI_AXMY = 2,      // dst = sigma0 * aux - D src (operator entry points)
 };
+
+// Layout of a hopping term's vectors: the library's colour planes, or the caller's host layout
+// (v[3 s + c]) for the source (bit 0) or for the destination and aux (bit 1)
+enum DslashLayout { LAY_SOA = 0, LAY_HOST_SRC = 1, LAY_HOST_DST = 2, LAY_HOST = 3 };
 
 template <class LF, class LL, typename SR> struct DslashArgs {
     using R = typename LF::R;
@@ -19,6 +24,7 @@ template <class LF, class LL, typename SR> struct DslashArgs {
     LL lng;
     Vec<SR> src, dst, aux;
     const double *sigma;  // per right-hand side (EPI_AXMY_DOT)
+    double sigma0;        // for every right-hand side (EPI_AXMY)
     double *partial;      // [nrhs_total][nblk] (EPI_AXMY_DOT)
     const int *run;       // device flag; kernel does nothing when *run == 0 (may be null)
     const int *rlist;     // compact list of active right-hand sides (may be null = identity)
@@ -43,6 +49,21 @@ constexpr int kReproNT = 256;
 // neighbour vectors of the batched terms in L2 (measured up to 19 % faster at 32^4).
 template <class LF, class LL, typename SR>
 void launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStream_t st, int cap = 0);
+
+// The same on vectors of the loaded gauge's precision in the caller's host layout (device memory,
+// aligned to their reals): lay LAY_HOST with EPI_STORE (D src, nr right-hand sides per block), or
+// the two terms of sigma0 src - D D src on one right-hand side, LAY_HOST_SRC with EPI_STORE and
+// LAY_HOST_DST with EPI_AXMY, whose intermediate is in colour planes. The vectors of one launch
+// must not overlap, except that aux and dst may be the same vector.
+template <class LF, class LL, typename SR>
+void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int nr, hipStream_t st);
+
+// Workgroups of nt sites for Vh sites, rounded up to a multiple of the 8 XCDs so that tile_site can
+// give each XCD a contiguous range of sites on any lattice (the last ones may be empty)
+inline uint32_t dslash_grid(uint32_t Vh, int nt)
+{
+    return (uint32_t)(((uint64_t)Vh + 8u * (uint32_t)nt - 1) / (8u * (uint32_t)nt)) * 8u;
+}
 
 inline uint32_t dslash_nblk(uint32_t Vh, int nt)
 {

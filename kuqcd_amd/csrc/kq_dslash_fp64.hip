@@ -4,5 +4,6 @@
 namespace kq {
 
 template void launch_dslash<LinkD, LinkD, double>(DslashArgs<LinkD, LinkD, double>, int, int, int, hipStream_t, int);
+template void launch_dslash_host<LinkD, LinkD, double>(const DslashArgs<LinkD, LinkD, double> &, int, int, int, hipStream_t);
 
 }  // namespace kq

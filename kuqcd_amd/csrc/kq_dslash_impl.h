@@ -20,16 +20,21 @@
 
 namespace kq {
 
-// gather the colour vector at site n of right-hand side j (base pointer src[j])
-template <class V2>
+// gather the colour vector at site n of right-hand side j (base pointer src[j]); AOS: the caller's
+// host layout (a site's three colours together, kq_fields.h) instead of the library's colour planes
+template <bool AOS = false, class V2>
 __device__ __forceinline__ void gather(const V2 *src, uint32_t n, uint32_t Vh, V2 v[3])
 {
+    if constexpr (AOS) {
+        ld_site(src + (size_t)3 * n, v);
+    } else {
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
-        v[c] = src[(size_t)c * Vh + n];
+        for (int c = 0; c < 3; ++c)
+            v[c] = src[(size_t)c * Vh + n];
+    }
 }
 
-template <class A, class LK, int NR, int MU, int H>
+template <class A, class LK, int NR, int MU, int H, bool AOS = false>
 __device__ __forceinline__ void hop_fwd(const A &a, const LK &lk, uint32_t s, const SiteCoord &sc,
                                         const typename A::V2 *const src[NR], typename A::R acc[NR][6])
 {
@@ -40,12 +45,12 @@ __device__ __forceinline__ void hop_fwd(const A &a, const LK &lk, uint32_t s, co
 #pragma unroll
     for (int j = 0; j < NR; ++j) {
         typename A::V2 v[3];
-        gather(src[j], n, a.g.Vh, v);
+        gather<AOS>(src[j], n, a.g.Vh, v);
         umv_add(U, v, acc[j]);
     }
 }
 
-template <class A, class LK, int NR, int MU, int H>
+template <class A, class LK, int NR, int MU, int H, bool AOS = false>
 __device__ __forceinline__ void hop_bwd(const A &a, const LK &lk, uint32_t s, const SiteCoord &sc,
                                         const typename A::V2 *const src[NR], typename A::R acc[NR][6])
 {
@@ -56,7 +61,7 @@ __device__ __forceinline__ void hop_bwd(const A &a, const LK &lk, uint32_t s, co
 #pragma unroll
     for (int j = 0; j < NR; ++j) {
         typename A::V2 v[3];
-        gather(src[j], n, a.g.Vh, v);
+        gather<AOS>(src[j], n, a.g.Vh, v);
         udmv_sub(U, v, acc[j]);
     }
 }
@@ -184,9 +189,16 @@ template <class LF, class V2> __device__ __forceinline__ void put(V2 *p, V2 v)
         st_nt(p, v);
 }
 
-// Epilogue of the hopping term: store D src (EPI_STORE), or dst = sigma aux - D src with the
-// per-workgroup partial sums of <aux, dst> (EPI_AXMY_DOT)
-template <class LF, typename SR, int NR, int EPI, int NT, class A, typename R>
+// Entry of colour c of site s of a vector in colour planes or in the caller's host layout
+template <bool AOS> __device__ __forceinline__ size_t entry_of(uint32_t Vh, uint32_t s, int c)
+{
+    return AOS ? (size_t)3 * s + c : (size_t)c * Vh + s;
+}
+
+// Epilogue of the hopping term: store D src (EPI_STORE), dst = sigma0 aux - D src with dst and aux
+// in the caller's host layout (EPI_AXMY), or dst = sigma aux - D src with the per-workgroup partial
+// sums of <aux, dst> (EPI_AXMY_DOT).
+template <class LF, typename SR, int NR, int EPI, int NT, bool AOS = false, class A, typename R>
 __device__ __forceinline__ void dslash_epilogue(const A &a, const R (&acc)[NR][6], c2_t<SR> *const (&dst)[NR],
                                                 const c2_t<SR> *const (&aux)[NR], const int (&rr)[NR], int j0,
                                                 int nact, uint32_t s, bool valid, double *lds)
@@ -203,6 +215,17 @@ __device__ __forceinline__ void dslash_epilogue(const A &a, const R (&acc)[NR][6
                 for (int c = 0; c < 3; ++c)
                     put<LF>(&dst[j][(size_t)c * Vh + s], mk<V2>((SR)acc[j][2 * c], (SR)acc[j][2 * c + 1]));
             }
+        }
+    } else if constexpr (EPI == EPI_AXMY) {
+        static_assert(NR == 1 && AOS, "the operator entry points' last term: one vector, host layout");
+        if (valid) {
+            V2 p[3], o[3];
+            gather<true>(aux[0], s, Vh, p);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                o[c] = mk<V2>((SR)((R)a.sigma0 * (R)p[c].x - acc[0][2 * c]),
+                              (SR)((R)a.sigma0 * (R)p[c].y - acc[0][2 * c + 1]));
+            st_site(dst[0] + (size_t)3 * s, o);
         }
     } else {
 #pragma unroll
@@ -244,12 +267,13 @@ __device__ __forceinline__ void dslash_rhs(const A &a, int j0, int nact, int (&r
     }
 }
 
-template <class LF, class LL, typename SR, int NR, int EPI, int NT>
+template <class LF, class LL, typename SR, int NR, int EPI, int NT, int LAY = LAY_SOA>
 __global__ void __launch_bounds__(NT) k_dslash(const DslashArgs<LF, LL, SR> a)
 {
     using A = DslashArgs<LF, LL, SR>;
     using R = typename A::R;
     using V2 = c2_t<SR>;
+    constexpr bool SA = (LAY & LAY_HOST_SRC) != 0, DA = (LAY & LAY_HOST_DST) != 0;
     __shared__ double lds[NT / kWave];
     if (a.run != nullptr && *a.run == 0)
         return;  // uniform over the grid
@@ -261,7 +285,7 @@ __global__ void __launch_bounds__(NT) k_dslash(const DslashArgs<LF, LL, SR> a)
     const V2 *src[NR];
     V2 *dst[NR];
     const V2 *aux[NR];
-    dslash_rhs<NR>(a, j0, nact, rr, dst, src, aux, EPI == EPI_AXMY_DOT);
+    dslash_rhs<NR>(a, j0, nact, rr, dst, src, aux, EPI != EPI_STORE);
     bool valid;
     const uint32_t s = tile_site<NT>(a.g, blockIdx.x, gridDim.x, threadIdx.x, valid);
     R acc[NR][6];
@@ -272,24 +296,164 @@ __global__ void __launch_bounds__(NT) k_dslash(const DslashArgs<LF, LL, SR> a)
             acc[j][k] = 0;
     if (valid) {
         const SiteCoord sc = site_coords(a.g, s, a.dst_parity);
-        hop_fwd<A, LF, NR, 0, 1>(a, a.fat, s, sc, src, acc);
-        hop_fwd<A, LL, NR, 0, 3>(a, a.lng, s, sc, src, acc);
-        hop_fwd<A, LF, NR, 1, 1>(a, a.fat, s, sc, src, acc);
-        hop_fwd<A, LL, NR, 1, 3>(a, a.lng, s, sc, src, acc);
-        hop_fwd<A, LF, NR, 2, 1>(a, a.fat, s, sc, src, acc);
-        hop_fwd<A, LL, NR, 2, 3>(a, a.lng, s, sc, src, acc);
-        hop_fwd<A, LF, NR, 3, 1>(a, a.fat, s, sc, src, acc);
-        hop_fwd<A, LL, NR, 3, 3>(a, a.lng, s, sc, src, acc);
-        hop_bwd<A, LF, NR, 0, 1>(a, a.fat, s, sc, src, acc);
-        hop_bwd<A, LL, NR, 0, 3>(a, a.lng, s, sc, src, acc);
-        hop_bwd<A, LF, NR, 1, 1>(a, a.fat, s, sc, src, acc);
-        hop_bwd<A, LL, NR, 1, 3>(a, a.lng, s, sc, src, acc);
-        hop_bwd<A, LF, NR, 2, 1>(a, a.fat, s, sc, src, acc);
-        hop_bwd<A, LL, NR, 2, 3>(a, a.lng, s, sc, src, acc);
-        hop_bwd<A, LF, NR, 3, 1>(a, a.fat, s, sc, src, acc);
-        hop_bwd<A, LL, NR, 3, 3>(a, a.lng, s, sc, src, acc);
+        hop_fwd<A, LF, NR, 0, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_fwd<A, LL, NR, 0, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_fwd<A, LF, NR, 1, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_fwd<A, LL, NR, 1, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_fwd<A, LF, NR, 2, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_fwd<A, LL, NR, 2, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_fwd<A, LF, NR, 3, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_fwd<A, LL, NR, 3, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_bwd<A, LF, NR, 0, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_bwd<A, LL, NR, 0, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_bwd<A, LF, NR, 1, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_bwd<A, LL, NR, 1, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_bwd<A, LF, NR, 2, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_bwd<A, LL, NR, 2, 3, SA>(a, a.lng, s, sc, src, acc);
+        hop_bwd<A, LF, NR, 3, 1, SA>(a, a.fat, s, sc, src, acc);
+        hop_bwd<A, LL, NR, 3, 3, SA>(a, a.lng, s, sc, src, acc);
     }
-    dslash_epilogue<LF, SR, NR, EPI, NT>(a, acc, dst, aux, rr, j0, nact, s, valid, lds);
+    dslash_epilogue<LF, SR, NR, EPI, NT, DA>(a, acc, dst, aux, rr, j0, nact, s, valid, lds);
+}
+
+// ---- split hopping term: S waves per 64 sites, each with 16 / S of the 16 hops
+//
+// With one thread per site a small lattice leaves most of the chip idle (8^4 has 2048 sites of one
+// parity: 32 waves on 1024 SIMDs) and each wave walks a serial chain of 16 link and neighbour
+// loads, so the time is latency. Here the S waves of a workgroup take the hops of the same 64
+// sites, keep the links' coalesced loads (lane = site) and add their partial results through LDS,
+// in wave order: S times the waves in flight and 1/S of the chain. Consecutive threads then own
+// consecutive entries of the destination's layout, so the host layout is written coalesced.
+// Measured per FP64 term (LinkD, LinkD14, one right-hand side), one thread per site in workgroups
+// of 256 -> S = 8: 8^4 8.9 -> 4.5 us, 12^4 16.5 -> 6.8, 16^4 18.9 -> 12.4, 22x18x15x13
+// 20.6 -> 17.1; at 16^3x32 and above, where the one-thread form fills the chip, up to 10 % slower
+// (32^4 176 -> 195). S = 4 and 16 are up to 10 % slower than 8 at 8^4 to 16^4.
+
+// Hops of one wave: hop I = 4 mu + 2 (backward) + (3 hops)
+template <class A, class LF, class LL, int NR, bool SA, int I>
+__device__ __forceinline__ void split_hop(const A &a, uint32_t s, const SiteCoord &sc,
+                                          const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+{
+    constexpr int MU = I / 4;
+    if constexpr ((I & 3) == 0)
+        hop_fwd<A, LF, NR, MU, 1, SA>(a, a.fat, s, sc, src, acc);
+    else if constexpr ((I & 3) == 1)
+        hop_fwd<A, LL, NR, MU, 3, SA>(a, a.lng, s, sc, src, acc);
+    else if constexpr ((I & 3) == 2)
+        hop_bwd<A, LF, NR, MU, 1, SA>(a, a.fat, s, sc, src, acc);
+    else
+        hop_bwd<A, LL, NR, MU, 3, SA>(a, a.lng, s, sc, src, acc);
+}
+
+template <class A, class LF, class LL, int NR, bool SA, int I, int N>
+__device__ __forceinline__ void split_hops(const A &a, uint32_t s, const SiteCoord &sc,
+                                           const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+{
+    split_hop<A, LF, LL, NR, SA, I>(a, s, sc, src, acc);
+    if constexpr (N > 1)
+        split_hops<A, LF, LL, NR, SA, I + 1, N - 1>(a, s, sc, src, acc);
+}
+
+template <class A, class LF, class LL, int NR, bool SA, int S, int W>
+__device__ __forceinline__ void split_wave(int w, const A &a, uint32_t s, const SiteCoord &sc,
+                                           const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+{
+    if (w == W)
+        split_hops<A, LF, LL, NR, SA, W * (16 / S), 16 / S>(a, s, sc, src, acc);
+    else if constexpr (W + 1 < S)
+        split_wave<A, LF, LL, NR, SA, S, W + 1>(w, a, s, sc, src, acc);
+}
+
+template <class LF, class LL, typename SR, int NR, int EPI, int S, int LAY = LAY_SOA>
+__global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL, SR> a)
+{
+    using A = DslashArgs<LF, LL, SR>;
+    using R = typename A::R;
+    using V2 = c2_t<SR>;
+    constexpr bool SA = (LAY & LAY_HOST_SRC) != 0, DA = (LAY & LAY_HOST_DST) != 0;
+    constexpr int NT = 64 * S;
+    __shared__ R red[S][NR][6][64];
+    __shared__ uint32_t site[64];
+    __shared__ double lds[S];
+    if (a.run != nullptr && *a.run == 0)
+        return;  // uniform over the grid
+    const int nact = a.nact ? *a.nact : a.nrhs;
+    const int j0 = blockIdx.y * NR;
+    if (j0 >= nact)
+        return;  // uniform over the block
+    int rr[NR];
+    const V2 *src[NR];
+    V2 *dst[NR];
+    const V2 *aux[NR];
+    dslash_rhs<NR>(a, j0, nact, rr, dst, src, aux, EPI != EPI_STORE);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t Vh = a.g.Vh;
+    bool valid;
+    const uint32_t s = tile_site<64>(a.g, blockIdx.x, gridDim.x, lane, valid);
+    R acc[NR][6];
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            acc[j][k] = 0;
+    if (valid) {
+        const SiteCoord sc = site_coords(a.g, s, a.dst_parity);
+        split_wave<A, LF, LL, NR, SA, S, 0>(w, a, s, sc, src, acc);
+    }
+    if (w == 0)
+        site[lane] = valid ? s : 0xffffffffu;
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            red[w][j][k][lane] = acc[j][k];
+    __syncthreads();
+    // 192 complex results per right-hand side, summed over the waves in their order; consecutive
+    // threads take consecutive entries of the destination's layout
+    constexpr int DOTS = EPI == EPI_AXMY_DOT ? NR : 1;
+    double d[DOTS];
+#pragma unroll
+    for (int j = 0; j < DOTS; ++j)
+        d[j] = 0.0;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+        if (j0 + j >= nact)
+            continue;  // uniform over the block
+        for (int e = threadIdx.x; e < 192; e += NT) {
+            const int l = DA ? e / 3 : (e & 63), c = DA ? e - 3 * l : e >> 6;
+            const uint32_t sl = site[l];
+            if (sl == 0xffffffffu)
+                continue;
+            R x = red[0][j][2 * c][l], y = red[0][j][2 * c + 1][l];
+#pragma unroll
+            for (int k = 1; k < S; ++k) {
+                x += red[k][j][2 * c][l];
+                y += red[k][j][2 * c + 1][l];
+            }
+            const size_t o = entry_of<DA>(Vh, sl, c);
+            V2 v = mk<V2>((SR)x, (SR)y);
+            if constexpr (EPI != EPI_STORE) {
+                const R sg = (R)(EPI == EPI_AXMY ? a.sigma0 : a.sigma[rr[j]]);
+                const V2 p = DA ? ld_u(&aux[j][o]) : aux[j][o];
+                v = mk<V2>((SR)(sg * (R)p.x - x), (SR)(sg * (R)p.y - y));
+                if constexpr (EPI == EPI_AXMY_DOT)
+                    d[j] += (double)p.x * (double)v.x + (double)p.y * (double)v.y;
+            }
+            if constexpr (DA)
+                st_u(&dst[j][o], v);
+            else
+                put<LF>(&dst[j][o], v);
+        }
+    }
+    if constexpr (EPI == EPI_AXMY_DOT) {
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            const double tot = block_sum<NT>(d[j], lds);
+            if (threadIdx.x == 0 && j0 + j < nact)
+                a.partial[(size_t)rr[j] * a.nblk + blockIdx.x] = tot;
+            __syncthreads();
+        }
+    }
 }
 
 // The batched hopping term with the x and y neighbours read from LDS: the workgroup (256 sites,
@@ -463,6 +627,94 @@ static void launch_epi(const DslashArgs<LF, LL, SR> &a, int epi, int nt, int cap
         launch_nt<LF, LL, SR, NR, EPI_STORE>(a, nt, cap, st);
     else
         launch_nt<LF, LL, SR, NR, EPI_AXMY_DOT>(a, nt, cap, st);
+}
+
+// Hopping term on the caller's host layout (kq_dslash.h)
+template <class LF, class LL, typename SR, int NR, int S>
+static void launch_host_split(DslashArgs<LF, LL, SR> a, int lay, int epi, hipStream_t st)
+{
+    a.nblk = dslash_grid(a.g.Vh, 64);
+    const dim3 grid(a.nblk, (a.nrhs + NR - 1) / NR), blk(64 * S);
+    if (lay == LAY_HOST && epi == EPI_STORE)
+        hipLaunchKernelGGL((k_dslash_split<LF, LL, SR, NR, EPI_STORE, S, LAY_HOST>), grid, blk, 0, st, a);
+    else if constexpr (NR == 1) {
+        if (lay == LAY_HOST_SRC && epi == EPI_STORE)
+            hipLaunchKernelGGL((k_dslash_split<LF, LL, SR, 1, EPI_STORE, S, LAY_HOST_SRC>), grid, blk, 0, st, a);
+        else if (lay == LAY_HOST_DST && epi == EPI_AXMY)
+            hipLaunchKernelGGL((k_dslash_split<LF, LL, SR, 1, EPI_AXMY, S, LAY_HOST_DST>), grid, blk, 0, st, a);
+        else
+            throw std::logic_error("dslash: unsupported layout");
+    } else
+        throw std::logic_error("dslash: unsupported layout");
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
+template <class LF, class LL, typename SR, int NT>
+static void launch_host_nt(DslashArgs<LF, LL, SR> a, int lay, int epi, hipStream_t st)
+{
+    a.nblk = dslash_grid(a.g.Vh, NT);
+    if (lay == LAY_HOST_SRC && epi == EPI_STORE)
+        hipLaunchKernelGGL((k_dslash<LF, LL, SR, 1, EPI_STORE, NT, LAY_HOST_SRC>), dim3(a.nblk), dim3(NT), 0, st, a);
+    else if (lay == LAY_HOST_DST && epi == EPI_AXMY)
+        hipLaunchKernelGGL((k_dslash<LF, LL, SR, 1, EPI_AXMY, NT, LAY_HOST_DST>), dim3(a.nblk), dim3(NT), 0, st, a);
+    else
+        throw std::logic_error("dslash: unsupported layout");
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
+template <class LF, class LL, typename SR>
+void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int nr, hipStream_t st)
+{
+    constexpr bool kDouble = std::is_same<SR, double>::value;
+    if (a.g.Vh == 0 || a.nrhs <= 0)
+        return;
+    if (lay == LAY_HOST) {
+        // Source and destination in the host layout: the split form at every size. Its epilogue
+        // writes the 48- or 24-byte sites coalesced, where one thread per site writes them in
+        // strides. Per launch, one thread per site -> split: FP64, one right-hand side, 24^4
+        // 67.6 -> 65 us, 32^4 206 -> 196, 48^4 1087 -> 1015; FP32, 8 right-hand sides in blocks of
+        // 4, 24^4 110 -> 82, 48^4 1597 -> 1382; in one block of 8 (S = 4), 24^4 90 -> 63. FP64
+        // blocks above 2 spill, so larger ones run as blocks of 2.
+        if constexpr (kDouble) {
+            if (nr >= 2)
+                launch_host_split<LF, LL, SR, 2, 8>(a, lay, epi, st);
+            else
+                launch_host_split<LF, LL, SR, 1, 8>(a, lay, epi, st);
+        } else {
+            switch (nr) {
+            case 1:
+                launch_host_split<LF, LL, SR, 1, 8>(a, lay, epi, st);
+                break;
+            case 2:
+                launch_host_split<LF, LL, SR, 2, 8>(a, lay, epi, st);
+                break;
+            case 3:
+                launch_host_split<LF, LL, SR, 3, 8>(a, lay, epi, st);
+                break;
+            case 4:
+                launch_host_split<LF, LL, SR, 4, 8>(a, lay, epi, st);
+                break;
+            case 8:
+                launch_host_split<LF, LL, SR, 8, 4>(a, lay, epi, st);
+                break;
+            default:
+                throw std::runtime_error("dslash: unsupported RHS blocking " + std::to_string(nr));
+            }
+        }
+        return;
+    }
+    // One side in the host layout (A = sigma - D D, one right-hand side): split up to the size at
+    // which one thread per site fills the chip, measured per term, one thread -> split: FP64
+    // 22x18x15x13 18.6 -> 16.9 us, 20^4 39.4 -> 31.7 (but 29.4 in workgroups of 64), 24^4
+    // 61.4 -> 63.6, 32^4 182 -> 196; FP32 16^3x32 14.2 -> 12.2, 20^4 18.9 -> 15.7, 24^4
+    // 29.4 -> 30.2. Workgroups of 64 below 200 000 sites, where a grid of 256-thread ones ends in
+    // a partly filled round (24^4 64.4 -> 61.4 us; equal at 32^3x16).
+    if (a.g.Vh <= (kDouble ? 49152u : 98304u))
+        launch_host_split<LF, LL, SR, 1, 8>(a, lay, epi, st);
+    else if (a.g.Vh < 200000u)
+        launch_host_nt<LF, LL, SR, 64>(a, lay, epi, st);
+    else
+        launch_host_nt<LF, LL, SR, 256>(a, lay, epi, st);
 }
 
 template <class LF, class LL, typename SR>

@@ -57,6 +57,63 @@ __device__ inline float2 ld_nt(const float2 *p)
     return mk<float2>(v.x, v.y);
 }
 
+// One site's three colours in the caller's host layout (v[3 s + c]): 48 bytes in FP64 as three
+// 16-byte words, 24 bytes in FP32 as a 16- and an 8-byte word. The caller's arrays are only as
+// aligned as their reals, so the words are too.
+typedef double kq_v2d_u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float kq_v2f_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float kq_v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void ld_site(const double2 *p, double2 v[3])
+{
+    const kq_v2d_u *q = reinterpret_cast<const kq_v2d_u *>(p);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const kq_v2d_u t = q[c];
+        v[c] = mk<double2>(t.x, t.y);
+    }
+}
+__device__ __forceinline__ void ld_site(const float2 *p, float2 v[3])
+{
+    const kq_v4f_u t = *reinterpret_cast<const kq_v4f_u *>(p);
+    const kq_v2f_u u = *reinterpret_cast<const kq_v2f_u *>(p + 2);
+    v[0] = mk<float2>(t.x, t.y);
+    v[1] = mk<float2>(t.z, t.w);
+    v[2] = mk<float2>(u.x, u.y);
+}
+__device__ __forceinline__ double2 ld_u(const double2 *p)
+{
+    const kq_v2d_u t = *reinterpret_cast<const kq_v2d_u *>(p);
+    return mk<double2>(t.x, t.y);
+}
+__device__ __forceinline__ float2 ld_u(const float2 *p)
+{
+    const kq_v2f_u t = *reinterpret_cast<const kq_v2f_u *>(p);
+    return mk<float2>(t.x, t.y);
+}
+// streaming stores, as st_nt's
+__device__ __forceinline__ void st_u(double2 *p, double2 v)
+{
+    const kq_v2d_u t = {v.x, v.y};
+    __builtin_nontemporal_store(t, reinterpret_cast<kq_v2d_u *>(p));
+}
+__device__ __forceinline__ void st_u(float2 *p, float2 v)
+{
+    const kq_v2f_u t = {v.x, v.y};
+    __builtin_nontemporal_store(t, reinterpret_cast<kq_v2f_u *>(p));
+}
+__device__ __forceinline__ void st_site(double2 *p, const double2 v[3])
+{
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        st_u(p + c, v[c]);
+}
+__device__ __forceinline__ void st_site(float2 *p, const float2 v[3])
+{
+    const kq_v4f_u t = {v[0].x, v[0].y, v[1].x, v[1].y};
+    __builtin_nontemporal_store(t, reinterpret_cast<kq_v4f_u *>(p));
+    st_u(p + 2, v[2]);
+}
+
 // two 16-bit fixed-point reals (low half: real part) -> floats in units of the
 // stored scale: q / 32767 for |q| <= 32767
 __device__ inline float2 q2f(unsigned int u)

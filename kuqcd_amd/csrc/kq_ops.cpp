@@ -9,21 +9,71 @@
 
 namespace kq {
 
-// ---------------------------------------------------------------- dslash on host buffers
-template <class LF, class LL, typename VR, typename HR>
-static void apply_t(LF fat, LL lng, const Geom &g, int nrhs, const void *src, void *dst, int dst_parity, int nr, int nt,
-                    bool mdaggm, double sigma)
+// ---------------------------------------------------------------- dslash on the caller's buffers
+static bool overlap(const void *p, const void *q, size_t bytes)
+{
+    const char *a = static_cast<const char *>(p), *b = static_cast<const char *>(q);
+    return a < b + bytes && b < a + bytes;
+}
+
+// In the loaded precision the hopping terms read and write the caller's host layout themselves, so
+// device arrays are used in place: converting them to colour planes and back cost two kernels,
+// two device-to-device copies and their gaps around every vector (A at 8^4 to 32^4: see
+// k_dslash_split; 8 FP32 right-hand sides at 24^4: 290 us for a 98 us kernel). Arrays that a kernel
+// cannot use in place (host memory, another GPU's, addresses that are not a multiple of a real, a
+// source that overlaps the destination) go through a device buffer in the same layout.
+template <class LF, class LL, typename R>
+static void apply_host(LF fat, LL lng, const Geom &g, int nrhs, const void *src, void *dst, int dst_parity, int nr,
+                       bool mdaggm, double sigma)
+{
+    Context &c = ctx();
+    const size_t n3 = (size_t)3 * g.Vh, bytes = sizeof(c2_t<R>) * n3 * (size_t)nrhs;
+    const auto usable = [](const void *p) { return (uintptr_t)p % sizeof(R) == 0 && on_this_device(p); };
+    const bool put_back = !usable(dst);
+    DevBuf s, d, t;
+    if (overlap(src, dst, bytes) || !usable(src)) {
+        s.alloc(bytes);
+        copy_from_host(s.as<void>(), src, bytes, c.stream);
+    }
+    if (put_back)
+        d.alloc(bytes);
+    const R *from = s ? s.as<R>() : static_cast<const R *>(src);
+    R *to = d ? d.as<R>() : static_cast<R *>(dst);
+    if (mdaggm) {
+        t.alloc(bytes);
+        mdaggm_host<LF, LL, R>(fat, lng, g, from, to, t.as<c2_t<R>>(), dst_parity, sigma, c.stream);
+    } else {
+        DslashArgs<LF, LL, R> a{};
+        a.g = g;
+        a.fat = fat;
+        a.lng = lng;
+        a.nrhs = nrhs;
+        a.dst_parity = dst_parity;
+        a.src = Vec<R>{reinterpret_cast<c2_t<R> *>(const_cast<R *>(from)), g.Vh, n3};
+        a.dst = Vec<R>{reinterpret_cast<c2_t<R> *>(to), g.Vh, n3};
+        launch_dslash_host(a, LAY_HOST, EPI_STORE, nr, c.stream);
+    }
+    if (put_back)
+        copy_to_host(dst, to, bytes, c.stream);
+    else
+        KQ_HIP_CHECK(hipStreamSynchronize(c.stream));
+}
+
+// The mixed modes work on FP32 colour planes converted from the caller's FP64 vectors
+template <class LF, class LL>
+static void apply_mixed(LF fat, LL lng, const Geom &g, int nrhs, const void *src, void *dst, int dst_parity, int nr,
+                        int nt, bool mdaggm, double sigma)
 {
     Context &c = ctx();
     const size_t n3 = (size_t)3 * g.Vh, nh = (size_t)6 * g.Vh;
-    DevBuf s(sizeof(c2_t<VR>) * nrhs * n3), d(sizeof(c2_t<VR>) * nrhs * n3), stage(sizeof(HR) * nh);
-    Vec<VR> sv{s.as<c2_t<VR>>(), g.Vh, n3}, dv{d.as<c2_t<VR>>(), g.Vh, n3};
+    DevBuf s(sizeof(float2) * nrhs * n3), d(sizeof(float2) * nrhs * n3), stage(sizeof(double) * nh);
+    Vec<float> sv{s.as<float2>(), g.Vh, n3}, dv{d.as<float2>(), g.Vh, n3};
     for (int r = 0; r < nrhs; ++r) {
-        KQ_HIP_CHECK(hipMemcpyAsync(stage.as<void>(), static_cast<const HR *>(src) + r * nh, sizeof(HR) * nh,
+        KQ_HIP_CHECK(hipMemcpyAsync(stage.as<void>(), static_cast<const double *>(src) + r * nh, sizeof(double) * nh,
                                     hipMemcpyDefault, c.stream));
-        vec_host_to_soa<HR, VR>(stage.as<HR>(), sv, r, c.stream);
+        vec_host_to_soa<double, float>(stage.as<double>(), sv, r, c.stream);
     }
-    DslashArgs<LF, LL, VR> a{};
+    DslashArgs<LF, LL, float> a{};
     a.g = g;
     a.fat = fat;
     a.lng = lng;
@@ -34,11 +84,11 @@ static void apply_t(LF fat, LL lng, const Geom &g, int nrhs, const void *src, vo
         a.dst = dv;
         launch_dslash(a, EPI_STORE, nr, nt, c.stream);
     } else {
-        DevBuf t(sizeof(c2_t<VR>) * nrhs * n3), sig(sizeof(double) * nrhs);
+        DevBuf t(sizeof(float2) * nrhs * n3), sig(sizeof(double) * nrhs);
         DevBuf part(sizeof(double) * nrhs * dslash_nblk(g.Vh, nt));
         std::vector<double> sg(nrhs, sigma);
         KQ_HIP_CHECK(hipMemcpyAsync(sig.as<void>(), sg.data(), sizeof(double) * nrhs, hipMemcpyHostToDevice, c.stream));
-        Vec<VR> tv{t.as<c2_t<VR>>(), g.Vh, n3};
+        Vec<float> tv{t.as<float2>(), g.Vh, n3};
         a.dst_parity = 1 - dst_parity;
         a.src = sv;
         a.dst = tv;
@@ -53,8 +103,8 @@ static void apply_t(LF fat, LL lng, const Geom &g, int nrhs, const void *src, vo
         KQ_HIP_CHECK(hipStreamSynchronize(c.stream));
     }
     for (int r = 0; r < nrhs; ++r) {
-        vec_soa_to_host<VR, HR>(dv, r, stage.as<HR>(), c.stream);
-        KQ_HIP_CHECK(hipMemcpyAsync(static_cast<HR *>(dst) + r * nh, stage.as<void>(), sizeof(HR) * nh,
+        vec_soa_to_host<float, double>(dv, r, stage.as<double>(), c.stream);
+        KQ_HIP_CHECK(hipMemcpyAsync(static_cast<double *>(dst) + r * nh, stage.as<void>(), sizeof(double) * nh,
                                     hipMemcpyDefault, c.stream));
         KQ_HIP_CHECK(hipStreamSynchronize(c.stream));
     }
@@ -94,13 +144,13 @@ static KuQCDStatus apply(int nrhs, const void *src, void *dst, int parity, int m
     if (mode == KQ_MODE_REFERENCE || mode == KQ_MODE_FP64) {
         if (dbl)
             with_fp64_links(slot, [&](auto fat, auto lng) {
-                apply_t<decltype(fat), decltype(lng), double, double>(fat, lng, g, nrhs, src, dst, parity, nr, nt,
-                                                                      mdaggm, sigma);
+                apply_host<decltype(fat), decltype(lng), double>(fat, lng, g, nrhs, src, dst, parity, nr, mdaggm,
+                                                                 sigma);
             });
         else if (mode == KQ_MODE_REFERENCE)
             with_fp32_links(slot, [&](auto fat, auto lng) {
-                apply_t<decltype(fat), decltype(lng), float, float>(fat, lng, g, nrhs, src, dst, parity, nr, nt, mdaggm,
-                                                                    sigma);
+                apply_host<decltype(fat), decltype(lng), float>(fat, lng, g, nrhs, src, dst, parity, nr, mdaggm,
+                                                                sigma);
             });
         else {
             set_error("FP64 mode needs a double-precision gauge field");
@@ -114,8 +164,7 @@ static KuQCDStatus apply(int nrhs, const void *src, void *dst, int parity, int m
     }
     if (is_mixed_mode(mode)) {
         with_mixed_links(slot, mode, [&](auto fat, auto lng) {
-            apply_t<decltype(fat), decltype(lng), float, double>(fat, lng, g, nrhs, src, dst, parity, nr, nt, mdaggm,
-                                                                 sigma);
+            apply_mixed<decltype(fat), decltype(lng)>(fat, lng, g, nrhs, src, dst, parity, nr, nt, mdaggm, sigma);
         });
         return KUQCD_SUCCESS;
     }

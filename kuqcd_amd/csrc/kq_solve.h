@@ -2,6 +2,7 @@
 #pragma once
 
 #include "kq_context.h"
+#include "kq_dslash.h"
 #include "kuqcd_hip.h"
 
 namespace kq {
@@ -22,6 +23,34 @@ std::vector<double> reduce_host(const double *part_dev, uint32_t nblk, int n, hi
 void copy_to_host(void *h, const void *d, size_t bytes, hipStream_t st);
 // bytes from h (pageable host, pinned host or device memory) to device memory d, likewise
 void copy_from_host(void *d, const void *h, size_t bytes, hipStream_t st);
+
+// true for device memory of the current GPU (not host, managed or another GPU's memory)
+bool on_this_device(const void *p);
+
+// dst = sigma src - D D src on parity `parity`, src and dst in the caller's host layout in device
+// memory (not overlapping), tmp a device vector of the other parity: two launches, not waited for
+template <class LF, class LL, typename R>
+inline void mdaggm_host(LF fat, LL lng, const Geom &g, const R *src, R *dst, c2_t<R> *tmp, int parity, double sigma,
+                        hipStream_t st)
+{
+    const size_t n3 = (size_t)3 * g.Vh;
+    const Vec<R> sv{reinterpret_cast<c2_t<R> *>(const_cast<R *>(src)), g.Vh, n3}, tv{tmp, g.Vh, n3};
+    DslashArgs<LF, LL, R> a{};
+    a.g = g;
+    a.fat = fat;
+    a.lng = lng;
+    a.nrhs = 1;
+    a.dst_parity = 1 - parity;
+    a.src = sv;
+    a.dst = tv;
+    launch_dslash_host(a, LAY_HOST_SRC, EPI_STORE, 1, st);
+    a.dst_parity = parity;
+    a.src = tv;
+    a.dst = Vec<R>{reinterpret_cast<c2_t<R> *>(dst), g.Vh, n3};
+    a.aux = sv;
+    a.sigma0 = sigma;
+    launch_dslash_host(a, LAY_HOST_DST, EPI_AXMY, 1, st);
+}
 
 // caller vector (reference layout, HR; host or device memory) -> device SoA vector r of v
 template <typename HR, typename VR> inline void upload_vec(const void *h, Vec<VR> v, int r, DevBuf &stage, hipStream_t st)

@@ -140,6 +140,17 @@ bool pageable(const void *p)
 
 }  // namespace
 
+bool on_this_device(const void *p)
+{
+    hipPointerAttribute_t a{};
+    int dev = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && hipGetDevice(&dev) == hipSuccess && a.device == dev;
+}
+
 void copy_to_host(void *h, const void *d, size_t bytes, hipStream_t st)
 {
     PinnedChunks &pc = chunks();

@@ -1,0 +1,109 @@
+"""The operator entry points on the caller's own device arrays (host layout): hopping term and
+A = sigma - D D against the oracle on lattices with remainders of every tile (64 sites, 8 XCDs, 256
+sites), on both sides of the sizes at which the split and the one-thread kernels change over, for
+every right-hand-side blocking and with a padded last block; addresses aligned to one real only; and
+sources that overlap the destination."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import rel_err
+
+TOL = {8: 1e-13, 4: 1e-5}  # the path's parity bounds (FP64, FP32)
+
+
+def _load(kq, lat, prec, u3=False):
+    fat, lng = kq.gen_gauge(lat, kind=kq.KQ_GEN_WEAK, eps=0.3, seed_fat=21, seed_long=22)
+    if u3:  # a phase on every long link: the complex-scale forms
+        ph = np.exp(1j * np.random.default_rng(5).normal(size=lng.shape[:2]))[:, :, None]
+        lng = np.ascontiguousarray(((lng[..., 0] + 1j * lng[..., 1]) * ph).view(np.float64).reshape(lng.shape))
+    kq.kuqcd_gauge_free()
+    kq.load_gauge_pair(fat, lng, lat, prec=prec)
+    return fat, lng
+
+
+class _Dev:
+    """A device array of `nbytes` bytes starting `shift` bytes after an allocation's start."""
+
+    def __init__(self, kq, nbytes, shift=0):
+        self.kq, self.n = kq, nbytes
+        self.base = kq.L.lib().kq_device_alloc(nbytes + 64)
+        self.p = self.base + shift
+
+    def put(self, a):
+        assert self.kq.L.lib().kq_memcpy(self.p, a.ctypes.data, a.nbytes) == 0
+
+    def get(self, like):
+        out = np.empty_like(like)
+        assert self.kq.L.lib().kq_memcpy(out.ctypes.data, self.p, out.nbytes) == 0
+        return out
+
+    def free(self):
+        self.kq.L.lib().kq_device_free(self.base)
+
+
+# Vh = 180 (less than the 8 tiles), 2048, 38610 (ragged), 56000 (FP64 one-thread kernel in workgroups
+# of 64), 131072 (FP32 likewise), 262144 (workgroups of 256)
+LATS = [(6, 5, 4, 3), (8, 8, 8, 8), (22, 18, 15, 13), (20, 20, 20, 14), (32, 16, 16, 32), (32, 32, 32, 16)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [8, 4])
+@pytest.mark.parametrize("lat", LATS)
+def test_operator_on_device_arrays(gpu, lat, prec):
+    kq, L = gpu, gpu.L.lib()
+    dt = np.float64 if prec == 8 else np.float32
+    fat, lng = _load(kq, lat, prec, u3=lat[1] % 2 == 1)
+    fat, lng = (a.astype(dt).astype(np.float64) for a in (fat, lng))
+    sigma = 0.07
+    for parity in (0, 1):
+        print("case", lat, prec, parity, flush=True)
+        src = kq.gen_source(lat, parity, seed=31).astype(dt)
+        want = sigma * src.astype(np.float64) - oracle.mdaggm(fat, lng, src.astype(np.float64), lat, parity)
+        hop = oracle.dslash(fat, lng, src.astype(np.float64), lat, 1 - parity)
+        for shift in (0, prec):  # aligned, and to one real only
+            s, d = _Dev(kq, src.nbytes, shift), _Dev(kq, src.nbytes, shift)
+            try:
+                s.put(src)
+                assert L.kq_mdaggm(C.c_void_p(s.p), C.c_void_p(d.p), parity, sigma, 0) == 0, kq.last_error()
+                out = d.get(src)
+                assert rel_err(out, want) <= TOL[prec]
+                assert np.array_equal(s.get(src), src)
+                host = np.empty_like(src)
+                assert kq.mdaggm(src, host, parity, sigma, 0) == 0
+                assert np.array_equal(host, out)
+                assert L.kq_dslash(C.c_void_p(s.p), C.c_void_p(d.p), 1 - parity, 0) == 0, kq.last_error()
+                assert rel_err(d.get(src), hop) <= TOL[prec]
+                # in place
+                assert L.kq_mdaggm(C.c_void_p(s.p), C.c_void_p(s.p), parity, sigma, 0) == 0
+                assert np.array_equal(s.get(src), out)
+            finally:
+                s.free()
+                d.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,nrs", [(8, (1, 2, 4, 8)), (4, (1, 2, 3, 4, 8))])
+@pytest.mark.parametrize("lat", [(6, 5, 4, 3), (16, 12, 8, 8)])
+def test_block_of_vectors_on_device_arrays(gpu, lat, prec, nrs):
+    kq, L = gpu, gpu.L.lib()
+    dt = np.float64 if prec == 8 else np.float32
+    fat, lng = _load(kq, lat, prec)
+    fat, lng = (a.astype(dt).astype(np.float64) for a in (fat, lng))
+    for nrhs in (1, 5, 9):  # whole and padded blocks
+        src = np.stack([kq.gen_source(lat, 1, seed=40 + r) for r in range(nrhs)]).astype(dt)
+        want = np.stack([oracle.dslash(fat, lng, v.astype(np.float64), lat, 0) for v in src])
+        both = _Dev(kq, 2 * src.nbytes)
+        try:
+            for nr in nrs:
+                print("case", lat, prec, nrhs, nr, flush=True)
+                for at in (src.nbytes, src.nbytes // 2):  # apart; destination over the source's second half
+                    both.put(src)
+                    assert L.kq_dslash_batched(nrhs, C.c_void_p(both.p), C.c_void_p(both.p + at), 0, 0, nr, 256) == 0
+                    out = np.empty_like(src)
+                    assert L.kq_memcpy(out.ctypes.data, both.p + at, out.nbytes) == 0
+                    assert rel_err(out, want) <= TOL[prec]
+        finally:
+            both.free()
