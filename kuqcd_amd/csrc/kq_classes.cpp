@@ -359,7 +359,7 @@ static void hop(const kq::Geom &g, LF fat, LL lng, const void *src, void *dst, i
     a.src = kq::Vec<T>{static_cast<kq::c2_t<T> *>(const_cast<void *>(src)), g.Vh, (size_t)3 * g.Vh};
     a.dst = kq::Vec<T>{static_cast<kq::c2_t<T> *>(dst), g.Vh, (size_t)3 * g.Vh};
     a.nrhs = 1;
-    kq::launch_dslash(a, kq::EPI_STORE, 1, kq::kReproNT, st, 0);
+    kq::launch_dslash(a, kq::EPI_STORE, 1, kq::repro_nt(g.Vh), st, 0);
 }
 
 template <typename T, int NB, KuQCDReconstructType RS, KuQCDReconstructType RN>
@@ -497,7 +497,7 @@ int CGM<T, VecT>::Invert(int noShifts, T shifts[], const VecT &src, VecT *sol[],
         const RK lr{static_cast<char *>(const_cast<void *>(h->KernelLinks(2))), kq::nb64_of(g.Vh)};
         kq::RunnerTuning tune;
         tune.nr = 1;
-        tune.nt = kq::kReproNT;
+        tune.nt = kq::repro_nt(g.Vh);
         tune.chunk = 16;
         auto solve = [&](auto lng) {
             kq::CgmRunner<T, T, LK, decltype(lng)> run(g, parity, f, lng, 1, noShifts, st, tune);

@@ -37,18 +37,23 @@ template <class LF, class LL, typename SR> struct DslashArgs {
 constexpr int kMinDslashNT = 64;
 // Block size of the hopping terms whose partial sums feed the reference method, the plain
 // FP64 solve and the FP64 verification. One partial per workgroup, added in a fixed order,
-// makes a reduction deterministic for a given block size; fixing the block size (instead of
-// taking the autotuner's timing-dependent pick) makes these results bitwise reproducible from
-// one process to the next.
-constexpr int kReproNT = 256;
+// makes a reduction deterministic for a given block size; fixing the block size by the lattice
+// (instead of taking the autotuner's timing-dependent pick) makes these results bitwise
+// reproducible from one process to the next. Below 200 000 sites a grid of 256-thread workgroups
+// ends in a partly filled round (FP64 term at 20^4: 313 workgroups on 256 CUs, 37 us against 29 in
+// workgroups of 64; 24^4 62 against 59.5); above, 256 is 1-3 % faster (32^4 176 against 181 us).
+inline int repro_nt(uint32_t Vh) { return Vh < 200000u ? 64 : 256; }
 
 // Launch D over all sites of parity dst_parity for every right-hand side.
 // nr = right-hand sides handled per thread (1, 2, 3, 4 or 8), nt = threads per block,
 // cap = at most this many wavefronts per SIMD (0: as many as the registers allow). The
 // cap is imposed with unused dynamic LDS; fewer resident waves keep the gathered
-// neighbour vectors of the batched terms in L2 (measured up to 19 % faster at 32^4).
+// neighbour vectors of the batched terms in L2 (measured up to 19 % faster at 32^4). Where the
+// split or the LDS-staged kernel runs, nt (and for the split one cap) has no effect.
+// Returns the number of workgroups over the sites: the stride of the partial sums per right-hand
+// side, at most dslash_nblk(Vh, kMinDslashNT).
 template <class LF, class LL, typename SR>
-void launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStream_t st, int cap = 0);
+uint32_t launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStream_t st, int cap = 0);
 
 // The same on vectors of the loaded gauge's precision in the caller's host layout (device memory,
 // aligned to their reals): lay LAY_HOST with EPI_STORE (D src, nr right-hand sides per block), or
@@ -65,11 +70,7 @@ inline uint32_t dslash_grid(uint32_t Vh, int nt)
     return (uint32_t)(((uint64_t)Vh + 8u * (uint32_t)nt - 1) / (8u * (uint32_t)nt)) * 8u;
 }
 
-inline uint32_t dslash_nblk(uint32_t Vh, int nt)
-{
-    uint32_t nb = (Vh + nt - 1) / nt;
-    return nb;
-}
+inline uint32_t dslash_nblk(uint32_t Vh, int nt) { return dslash_grid(Vh, nt); }
 
 // Row length Lx/2 of the lattices whose batched hopping terms stage rows in LDS (Lx = 32, as at
 // 32^4): a compile-time row length gives the staged kernel a static LDS size
@@ -86,12 +87,35 @@ inline bool stage_enabled()
     return on;
 }
 
+// Lattices whose workgroups of 256 cover whole x-rows of one (x, y) plane of that row length
+inline bool stage_lattice(const Geom &g) { return g.lxh == kStageLxh && stage_rows(g, 256) > 0; }
+
 // Whether launch_dslash runs the LDS-staged kernel for nr right-hand sides per thread and block
 // size nt on this lattice (its NR * 3 * 352 staged colour entries, at most 67.6 KB for eight
 // FP32 or 33.8 KB for two FP64 right-hand sides, fit a workgroup's LDS on gfx950)
 inline bool dslash_staged(const Geom &g, int nr, int nt)
 {
-    return nr >= 2 && nt == 256 && g.lxh == kStageLxh && stage_enabled() && stage_rows(g, nt) > 0;
+    return nr >= 2 && nt == 256 && stage_enabled() && stage_lattice(g);
+}
+
+// Waves per 64 sites of the split hopping term (k_dslash_split) that launch_dslash uses for
+// `groups` groups of nr right-hand sides, or 0 where one thread per site serves better: when the
+// one-thread form's waves (Vh * groups / 64) already fill the chip. Measured per term, one
+// thread per site -> split: FP64 (blocks of 1) 8^4 8.9 -> 4.5 us, 16^4 18.9 -> 12.7, 22x18x15x13
+// 20.6 -> 17.1, 16^3x32 23.9 -> 25.2; FP32 (LinkF, LinkF12) blocks of 1: 16^4 12.1 -> 7.1, 16^3x32
+// 14.5 -> 12.6, 20^4 19.0 -> 16.4, 24^4 29.8 -> 31.2; blocks of 4: 16^4 21.8 -> 12.4, 16^3x32
+// 23.8 -> 21.1, but two groups of 4 there 33 -> 37, 24^4 50 -> 47 (47.6 in workgroups of 64).
+// Blocks of 8 FP32 right-hand sides leave the one-thread form one wave per SIMD, waiting for its
+// gathers: split into 4 waves at every size, 16^4 41 -> 18, 24^4 82 -> 75, 48^4 1316 -> 1118,
+// except where the larger lattices stage rows in LDS (32^4: 174 staged, 217 split).
+inline int dslash_split_waves(bool fp64, const Geom &g, int groups, int nr)
+{
+    const uint64_t work = (uint64_t)g.Vh * (uint64_t)groups;
+    if (fp64)
+        return nr <= 2 && work <= 49152u ? 8 : 0;
+    if (work <= 98304u)
+        return nr <= 2 ? 8 : 4;
+    return nr == 8 && !stage_lattice(g) ? 4 : 0;
 }
 
 }  // namespace kq

@@ -3,8 +3,8 @@
 
 namespace kq {
 
-template void launch_dslash<LinkF, LinkF, float>(DslashArgs<LinkF, LinkF, float>, int, int, int, hipStream_t, int);
-template void launch_dslash<LinkF, LinkF12, float>(DslashArgs<LinkF, LinkF12, float>, int, int, int, hipStream_t, int);
+template uint32_t launch_dslash<LinkF, LinkF, float>(DslashArgs<LinkF, LinkF, float>, int, int, int, hipStream_t, int);
+template uint32_t launch_dslash<LinkF, LinkF12, float>(DslashArgs<LinkF, LinkF12, float>, int, int, int, hipStream_t, int);
 template void launch_dslash_host<LinkF, LinkF, float>(const DslashArgs<LinkF, LinkF, float> &, int, int, int, hipStream_t);
 template void launch_dslash_host<LinkF, LinkF12, float>(const DslashArgs<LinkF, LinkF12, float> &, int, int, int, hipStream_t);
 

@@ -3,7 +3,7 @@
 
 namespace kq {
 
-template void launch_dslash<LinkD, LinkD, double>(DslashArgs<LinkD, LinkD, double>, int, int, int, hipStream_t, int);
+template uint32_t launch_dslash<LinkD, LinkD, double>(DslashArgs<LinkD, LinkD, double>, int, int, int, hipStream_t, int);
 template void launch_dslash_host<LinkD, LinkD, double>(const DslashArgs<LinkD, LinkD, double> &, int, int, int, hipStream_t);
 
 }  // namespace kq

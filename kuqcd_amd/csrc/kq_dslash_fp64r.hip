@@ -3,7 +3,7 @@
 
 namespace kq {
 
-template void launch_dslash<LinkD, LinkD14, double>(DslashArgs<LinkD, LinkD14, double>, int, int, int, hipStream_t,
+template uint32_t launch_dslash<LinkD, LinkD14, double>(DslashArgs<LinkD, LinkD14, double>, int, int, int, hipStream_t,
                                                     int);
 template void launch_dslash_host<LinkD, LinkD14, double>(const DslashArgs<LinkD, LinkD14, double> &, int, int, int, hipStream_t);
 

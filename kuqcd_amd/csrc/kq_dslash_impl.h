@@ -590,7 +590,7 @@ template <class LF, class LL, typename SR, int NR, int EPI>
 static void launch_nt(const DslashArgs<LF, LL, SR> &a, int nt, int cap, hipStream_t st)
 {
     const int nact_max = a.nrhs;
-    dim3 grid((a.g.Vh + nt - 1) / nt, (nact_max + NR - 1) / NR);
+    const dim3 grid(a.nblk, (nact_max + NR - 1) / NR);
     const size_t lds = cap_lds_bytes(cap, nt);
     if constexpr (NR >= 2) {
         // staged rows (static LDS of the kernel): NR * 3 colour entries for each of the
@@ -620,13 +620,35 @@ static void launch_nt(const DslashArgs<LF, LL, SR> &a, int nt, int cap, hipStrea
     KQ_HIP_CHECK(hipGetLastError());
 }
 
-template <class LF, class LL, typename SR, int NR>
-static void launch_epi(const DslashArgs<LF, LL, SR> &a, int epi, int nt, int cap, hipStream_t st)
+template <class LF, class LL, typename SR, int NR, int S>
+static void launch_split(const DslashArgs<LF, LL, SR> &a, int epi, hipStream_t st)
 {
+    const dim3 grid(a.nblk, (a.nrhs + NR - 1) / NR), blk(64 * S);
+    if (epi == EPI_STORE)
+        hipLaunchKernelGGL((k_dslash_split<LF, LL, SR, NR, EPI_STORE, S>), grid, blk, 0, st, a);
+    else
+        hipLaunchKernelGGL((k_dslash_split<LF, LL, SR, NR, EPI_AXMY_DOT, S>), grid, blk, 0, st, a);
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
+template <class LF, class LL, typename SR, int NR>
+static uint32_t launch_epi(DslashArgs<LF, LL, SR> a, int epi, int nt, int cap, hipStream_t st)
+{
+    constexpr bool kDouble = std::is_same<SR, double>::value;
+    if constexpr (!kDouble || NR <= 2) {
+        constexpr int S = NR <= 2 ? 8 : 4;
+        if (dslash_split_waves(kDouble, a.g, (a.nrhs + NR - 1) / NR, NR) == S) {
+            a.nblk = dslash_grid(a.g.Vh, 64);
+            launch_split<LF, LL, SR, NR, S>(a, epi, st);
+            return a.nblk;
+        }
+    }
+    a.nblk = dslash_grid(a.g.Vh, nt);
     if (epi == EPI_STORE)
         launch_nt<LF, LL, SR, NR, EPI_STORE>(a, nt, cap, st);
     else
         launch_nt<LF, LL, SR, NR, EPI_AXMY_DOT>(a, nt, cap, st);
+    return a.nblk;
 }
 
 // Hopping term on the caller's host layout (kq_dslash.h)
@@ -718,31 +740,24 @@ void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int n
 }
 
 template <class LF, class LL, typename SR>
-void launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStream_t st, int cap)
+uint32_t launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStream_t st, int cap)
 {
     if (a.g.Vh == 0 || a.nrhs <= 0)
-        return;
-    a.nblk = (a.g.Vh + nt - 1) / nt;
+        return 0;
     switch (nr) {
     case 1:
-        launch_epi<LF, LL, SR, 1>(a, epi, nt, cap, st);
-        break;
+        return launch_epi<LF, LL, SR, 1>(a, epi, nt, cap, st);
     case 2:
-        launch_epi<LF, LL, SR, 2>(a, epi, nt, cap, st);
-        break;
+        return launch_epi<LF, LL, SR, 2>(a, epi, nt, cap, st);
     case 3:
-        launch_epi<LF, LL, SR, 3>(a, epi, nt, cap, st);
-        break;
+        return launch_epi<LF, LL, SR, 3>(a, epi, nt, cap, st);
     case 4:
-        launch_epi<LF, LL, SR, 4>(a, epi, nt, cap, st);
-        break;
+        return launch_epi<LF, LL, SR, 4>(a, epi, nt, cap, st);
     case 8:
-        launch_epi<LF, LL, SR, 8>(a, epi, nt, cap, st);
-        break;
+        return launch_epi<LF, LL, SR, 8>(a, epi, nt, cap, st);
     default:
         throw std::runtime_error("dslash: unsupported RHS blocking " + std::to_string(nr));
     }
 }
-
 
 }  // namespace kq

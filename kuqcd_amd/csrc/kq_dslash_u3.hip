@@ -4,11 +4,11 @@
 
 namespace kq {
 
-template void launch_dslash<LinkF, LinkF12C, float>(DslashArgs<LinkF, LinkF12C, float>, int, int, int, hipStream_t,
+template uint32_t launch_dslash<LinkF, LinkF12C, float>(DslashArgs<LinkF, LinkF12C, float>, int, int, int, hipStream_t,
                                                     int);
-template void launch_dslash<LinkF, LinkH12C, float>(DslashArgs<LinkF, LinkH12C, float>, int, int, int, hipStream_t,
+template uint32_t launch_dslash<LinkF, LinkH12C, float>(DslashArgs<LinkF, LinkH12C, float>, int, int, int, hipStream_t,
                                                     int);
-template void launch_dslash<LinkH, LinkH12C, float>(DslashArgs<LinkH, LinkH12C, float>, int, int, int, hipStream_t,
+template uint32_t launch_dslash<LinkH, LinkH12C, float>(DslashArgs<LinkH, LinkH12C, float>, int, int, int, hipStream_t,
                                                     int);
 template void launch_dslash_host<LinkF, LinkF12C, float>(const DslashArgs<LinkF, LinkF12C, float> &, int, int, int, hipStream_t);
 

@@ -118,9 +118,11 @@ template <class LF, class LL, typename R> struct OpA {
     LL lng;
     int nt;
     int cap = 0;  // occupancy cap of the hopping term (waves per SIMD, 0 = none)
-    uint32_t nblk() const { return dslash_nblk(g.Vh, nt); }
-    // dst = sigma src - D D src (parity q), tmp on parity 1-q; part[nblk] = partials of Re<src, dst>
-    void apply(const V2 *src, V2 *tmp, V2 *dst, const double *sigma, double *part, const int *run,
+    // entries of part that any launch fits
+    uint32_t max_nblk() const { return dslash_nblk(g.Vh, kMinDslashNT); }
+    // dst = sigma src - D D src (parity q), tmp on parity 1-q; part = partials of Re<src, dst>, whose
+    // number is returned
+    uint32_t apply(const V2 *src, V2 *tmp, V2 *dst, const double *sigma, double *part, const int *run,
                hipStream_t st) const
     {
         DslashArgs<LF, LL, R> a{};
@@ -139,7 +141,7 @@ template <class LF, class LL, typename R> struct OpA {
         a.dst = Vec<R>{dst, g.Vh, 0};
         a.sigma = sigma;
         a.partial = part;
-        launch_dslash(a, EPI_AXMY_DOT, 1, nt, st, cap);
+        return launch_dslash(a, EPI_AXMY_DOT, 1, nt, st, cap);
     }
 };
 
@@ -149,7 +151,7 @@ void apply_a_f32(const Geom &g, int q, LF fat, LL lng, double sigma, const float
                  hipStream_t st)
 {
     const size_t n3 = (size_t)3 * g.Vh;
-    DevBuf t(sizeof(float2) * n3), sig(sizeof(double)), part(sizeof(double) * dslash_nblk(g.Vh, nt));
+    DevBuf t(sizeof(float2) * n3), sig(sizeof(double)), part(sizeof(double) * dslash_nblk(g.Vh, kMinDslashNT));
     KQ_HIP_CHECK(hipMemcpyAsync(sig.as<void>(), &sigma, sizeof(double), hipMemcpyHostToDevice, st));
     const OpA<LF, LL, float> A{g, q, fat, lng, nt};
     A.apply(x, t.as<float2>(), out, sig.as<double>(), part.as<double>(), nullptr, st);
@@ -193,7 +195,7 @@ FcgOut fcg_solve(const Geom &g, int q, AF af, AL al, PF pf, PL pl, LinkD df, Lin
     DevBuf vh16(cfg.learned ? sizeof(kq_v4u) * n3 : 0);
     DevBuf ax64(db), t64(db), r64(hook ? db : 0), xbest(cfg.learned ? db : 0);
     DevBuf part_qz(sizeof(double) * 2 * std::max(nbv, nbl)), part_pr(sizeof(double) * 2 * nbv),
-        part_pq(sizeof(double) * std::max(A.nblk(), D64.nblk())), part_rr(sizeof(double) * nbv);
+        part_pq(sizeof(double) * A.max_nblk()), part_rr(sizeof(double) * nbv);
     DevBuf sdev(sizeof(FcgState));
     Pinned<FcgState> sh(1);
     FcgState &H = *sh.get();
@@ -232,8 +234,9 @@ FcgOut fcg_solve(const Geom &g, int q, AF af, AL al, PF pf, PL pl, LinkD df, Lin
             fcg_beta(S, part_qz.as<double>(), nbv, st);
             fcg_p_update(S, vr.as<float2>(), vp.as<float2>(), vr.as<float2>(), n3, part_pr.as<double>(), st);
         }
-        A.apply(vp.as<float2>(), vt.as<float2>(), vq.as<float2>(), &S->sigma, part_pq.as<double>(), &S->run, st);
-        fcg_alpha(S, part_pq.as<double>(), A.nblk(), part_pr.as<double>(), nbv, st);
+        const uint32_t nbp = A.apply(vp.as<float2>(), vt.as<float2>(), vq.as<float2>(), &S->sigma, part_pq.as<double>(),
+                                     &S->run, st);
+        fcg_alpha(S, part_pq.as<double>(), nbp, part_pr.as<double>(), nbv, st);
         fcg_xr_update(S, vx.as<float2>(), vr.as<float2>(), vp.as<float2>(), vq.as<float2>(), n3,
                       part_rr.as<double>(), st);
         fcg_check(S, part_rr.as<double>(), nbv, st);
@@ -358,7 +361,7 @@ struct Work {
         gz.alloc(fb);
         gh.alloc(4 * fb);
         sig.alloc(sizeof(double));
-        part.alloc(sizeof(double) * dslash_nblk(Vh, nt));
+        part.alloc(sizeof(double) * dslash_nblk(Vh, kMinDslashNT));
     }
 };
 

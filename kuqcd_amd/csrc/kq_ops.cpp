@@ -85,7 +85,7 @@ static void apply_mixed(LF fat, LL lng, const Geom &g, int nrhs, const void *src
         launch_dslash(a, EPI_STORE, nr, nt, c.stream);
     } else {
         DevBuf t(sizeof(float2) * nrhs * n3), sig(sizeof(double) * nrhs);
-        DevBuf part(sizeof(double) * nrhs * dslash_nblk(g.Vh, nt));
+        DevBuf part(sizeof(double) * nrhs * dslash_nblk(g.Vh, kMinDslashNT));
         std::vector<double> sg(nrhs, sigma);
         KQ_HIP_CHECK(hipMemcpyAsync(sig.as<void>(), sg.data(), sizeof(double) * nrhs, hipMemcpyHostToDevice, c.stream));
         Vec<float> tv{t.as<float2>(), g.Vh, n3};
@@ -248,6 +248,9 @@ static double time_mode(int slot, int mode, int nrhs, int nr, int nt, int iters,
     return ms;
 }
 
+// Lattices whose single group of right-hand sides takes the split hopping term (dslash_split_waves)
+static bool small_lattice(const Geom &g) { return dslash_split_waves(false, g, 1, 1) > 0; }
+
 std::pair<int, int> tuned_launch(int slot, int mode, int nrhs)
 {
     Context &c = ctx();
@@ -266,6 +269,23 @@ std::pair<int, int> tuned_launch(int slot, int mode, int nrhs)
     // without an occupancy cap and with caps of 5..2 waves per SIMD; the best cap is kept
     // (tuned_cap).
     static const int kNr[5] = {1, 2, 3, 4, 8}, kNt[3] = {64, 128, 256}, kCap[5] = {0, 5, 4, 3, 2};
+    if (small_lattice(g)) {
+        // Groups of a small lattice share the chip, so the blockings are timed on all nrhs systems
+        // (8 FP32 systems at 8^4: one group of 8 11.5 us, 8 groups of 1 about half), without caps
+        double best = 1e30, bs = 0.0;
+        std::pair<int, int> pick{1, dslash_staged(g, 2, 256) ? 256 : 64};
+        for (int nr : kNr) {
+            if (nr > 1 && (nr >= 2 * nrhs || (mode == KQ_MODE_FP64 && nr > 2)))
+                continue;
+            const double t = time_mode(slot, mode, nrhs, nr, pick.second, 6, &bs);
+            if (t < best) {
+                best = t;
+                pick.first = nr;
+            }
+        }
+        c.tune[key] = pick;
+        return pick;
+    }
     auto &tg = c.tune_group[{mode, g.Vh}];
     if (tg[0] == 0.0)
         tg.fill(-1.0);
@@ -307,6 +327,8 @@ int tuned_cap(int slot, int mode, int nr, int nt)
 {
     Context &c = ctx();
     const Geom g = slot_geom(slot);
+    if (small_lattice(g))
+        return 0;
     if (mode == KQ_MODE_REFERENCE && c.fat[slot].prec == KUQCD_DOUBLE)
         mode = KQ_MODE_FP64;
     const auto key = std::make_tuple(mode, g.Vh, nr, nt);

@@ -92,7 +92,7 @@ static KuQCDStatus solve_ref_t(int slot, LF fat, LL lng, void **x, void *b, KuQC
     const int ns = p.num_shift;
     RunnerTuning tune;
     tune.nr = 1;
-    tune.nt = kReproNT;
+    tune.nt = repro_nt(g.Vh);
     set_caps(tune, slot, KQ_MODE_REFERENCE, false);
     tune.chunk = 16;
     CgmRunner<T, T, LF, LL> run(g, parity, fat, lng, 1, ns, c.stream, tune);
@@ -189,7 +189,7 @@ template <typename T, class LF, class LL> struct FullOps {
             a.src = Vec<T>{const_cast<V2 *>(src) + (size_t)(1 - q) * n3, g.Vh, n3};
             a.dst = Vec<T>{dst + (size_t)q * n3, g.Vh, n3};
             a.nrhs = 1;
-            launch_dslash(a, EPI_STORE, 1, kReproNT, st, 0);
+            launch_dslash(a, EPI_STORE, 1, repro_nt(g.Vh), st, 0);
         }
     }
     T dot(const V2 *u, const V2 *v)
@@ -287,9 +287,9 @@ static std::vector<double> true_res2_t(int slot, LinkD fat, LL lng, int parity, 
     // FP64 blocking and occupancy cap from the autotuner (one group of at most two
     // right-hand sides per workgroup); the fixed block size keeps the residuals reproducible
     const auto pick = tuned_launch(slot, KQ_MODE_FP64, nl);
-    const int nr = std::min(pick.first, 2), nt = kReproNT;
+    const int nr = std::min(pick.first, 2), nt = repro_nt(g.Vh);
     const int cap = tuned_cap(slot, KQ_MODE_FP64, nr, nt);
-    const uint32_t nblk_d = dslash_nblk(g.Vh, nt);
+    const uint32_t nblk_d = dslash_nblk(g.Vh, kMinDslashNT);
     DevBuf part(sizeof(double) * nk * std::max(nblk_d, blas_nblk(g.Vh)));
     std::vector<int> hl(which);
     hl.push_back(nl);
@@ -348,10 +348,12 @@ static bool debug_on()
 // autotuned right-hand-side blocking for 0..min(max_sys, 16) live systems
 static std::vector<int> nr_table(int slot, int mode, int max_sys)
 {
+    // each count up to 4 and then the largest of a step of counts, which serves the counts below it
+    static const int kUpTo[17] = {0, 1, 2, 3, 4, 6, 6, 8, 8, 12, 12, 12, 12, 16, 16, 16, 16};
     const int n = std::min(max_sys, 16);
     std::vector<int> t(n + 1, 1);
     for (int k = 2; k <= n; ++k)
-        t[k] = tuned_launch(slot, mode, k).first;
+        t[k] = tuned_launch(slot, mode, kUpTo[k]).first;
     return t;
 }
 
@@ -594,7 +596,7 @@ static void run_fp64(Problem &P, DevBuf &x_out, KqSolveReport *rep, std::vector<
     Context &c = ctx();
     const size_t n3 = (size_t)3 * P.g.Vh;
     RunnerTuning tune;
-    tune.nt = P.o->nt > 0 ? P.o->nt : kReproNT;
+    tune.nt = P.o->nt > 0 ? P.o->nt : repro_nt(P.g.Vh);
     if (P.o->nr > 0)
         tune.nr = P.o->nr;
     else

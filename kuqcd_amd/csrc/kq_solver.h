@@ -277,11 +277,9 @@ public:
         for (int i = 0; i < max_sys; ++i)
             state_h_[i].stop = 1;  // unused slots never run
         nblk_ = blas_nblk(g.Vh);
-        nblk_dsl_ = dslash_nblk(g.Vh, tune.nt);
-        // partials of both hopping terms the runner launches: the iteration's (block size
-        // tune.nt, stride nblk_dsl_) and the FP64 one of the reliable updates (tune.nt64),
-        // whose block sizes are tuned independently; rows for the smallest block size
-        // launch_dslash accepts fit either
+        // partials of both hopping terms the runner launches: the iteration's (tune.nt) and the FP64
+        // one of the reliable updates (tune.nt64), whose block sizes are tuned independently;
+        // rows for the smallest block size launch_dslash accepts fit either
         part_a_.alloc(sizeof(double) * max_sys * dslash_nblk(g.Vh, kMinDslashNT));
         part_b_.alloc(sizeof(double) * max_sys * nblk_);
         ints_.alloc(sizeof(int) * (2 * max_sys + 4));
@@ -596,7 +594,6 @@ private:
         CgmLaunch L;
         L.Vh = g_.Vh;
         L.nblk = nblk_;
-        L.nblk_dsl = nblk_dsl_;
         L.nsys = max_sys_;
         L.nlaunch = std::min(std::max(nlaunch, 1), max_sys_);
         L.rlist = rlist();
@@ -778,7 +775,7 @@ private:
     // grid sized for nr * groups live systems.
     void iteration(int nr, int groups)
     {
-        const CgmLaunch L = launch(nr * groups);
+        CgmLaunch L = launch(nr * groups);
         CgmState<S> *st = state_.as<CgmState<S>>();
         cgm_begin<S>(st, L, st_);
         DslashArgs<LF, LL, VR> d{};
@@ -799,7 +796,7 @@ private:
         d.aux = vec_p0();
         d.sigma = sigma_.as<double>();
         d.partial = part_a_.as<double>();
-        launch_dslash(d, EPI_AXMY_DOT, nr, tune_.nt, st_, tune_.cap_for(nr));
+        L.nblk_dsl = launch_dslash(d, EPI_AXMY_DOT, nr, tune_.nt, st_, tune_.cap_for(nr));
         cgm_scalars1<S>(st, L, st_);
         cgm_axpy_norm<S, VR>(st, vec(r_), vec(s_), L, st_);
         cgm_scalars2<S>(st, L, st_);
@@ -834,7 +831,7 @@ private:
     hipStream_t st_;
     RunnerTuning tune_;
     size_t n3_ = 0;
-    uint32_t nblk_ = 0, nblk_dsl_ = 0;
+    uint32_t nblk_ = 0;
     DevBuf r_, s_, tmp_, p_, x_, state_, part_a_, part_b_, ints_, sigma_, off_;
     Pinned<CgmState<S>> state_h_;
     Pinned<int> list_stage_;  // kStages slots of max_sys_ system indices

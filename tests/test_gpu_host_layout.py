@@ -107,3 +107,22 @@ def test_block_of_vectors_on_device_arrays(gpu, lat, prec, nrs):
                     assert rel_err(out, want) <= TOL[prec]
         finally:
             both.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lat,nrhs", [((6, 5, 4, 3), 5), ((22, 18, 15, 13), 9), ((24, 24, 24, 16), 8), ((24, 24, 24, 24), 8)])
+@pytest.mark.parametrize("mode", [2, 3, 4])
+def test_blocks_of_the_mixed_terms(gpu, lat, nrhs, mode):
+    """Every blocking of the 32-bit terms on colour planes, split (small lattices, and blocks of 8 on
+    any) and one thread per site (24^4 in blocks up to 4), with padded last blocks. Bounds as for the
+    formats elsewhere: FP32 1e-5, 16-bit links 3e-3, 16-bit long links 5e-4."""
+    kq = gpu
+    fat, lng = _load(kq, lat, 8, u3=mode == 4)
+    src = np.stack([kq.gen_source(lat, 0, seed=60 + r % 3) for r in range(nrhs)])
+    want = [oracle.dslash(fat, lng, src[r], lat, 1) for r in range(3)]
+    for nr in (1, 2, 3, 4, 8):
+        print("case", lat, mode, nr, flush=True)
+        out = np.full_like(src, np.nan)
+        assert kq.dslash_batched(src, out, 1, mode, nr, 64) == 0, kq.last_error()
+        for r in range(nrhs):
+            assert rel_err(out[r], want[r % 3]) <= {2: 1e-5, 3: 3e-3, 4: 5e-4}[mode], r
