@@ -26,7 +26,13 @@ template <typename S> struct CgmState {
     double tolk[kMaxShift];   // absolute squared-residual target per shift (inverter_cgm.cpp:72-73)
     double r2max;             // |r|^2 at the last reliable update (mixed precision)
     double pause2;            // pause when |r|^2 < pause2 * r2max (0: never)
+    // |r|^2 and maxTerm at the start of the iteration's updates (written by k_cgm_update_r, read by
+    // k_cgm_update_p while its scalar workgroup moves rr and maxTerm on)
+    S rr_prev;
+    int maxTermPrev;
     int nshift, maxTerm, maxTermUpd, iter, maxIter, stop, run, maxTermFold, pause;
+    int live;     // neither stopped nor paused: what a runner of one system iterates by (run: its
+                  // copy for k_cgm_update_p)
     int discard;  // set by the host for one fold: drop x_lo instead of adding it (diverged iteration)
     // deferred solution updates (multishift systems of the mixed solver): history slot of the
     // system (-1: x and p of every shift are updated each iteration) and the number of
@@ -58,25 +64,24 @@ struct CgmLaunch {
     uint32_t nblk_dsl = 0;  // blocks of the hopping-term launch (= stride of part_a)
     int nsys;           // system slots (k_cgm_begin scans all of them)
     int nlaunch;        // slots of the live list the per-system kernels cover (>= live systems)
-    int *rlist;         // compact list of live systems (written by k_cgm_begin)
-    int *nact;          // its length
+    int *rlist;         // compact list of live systems (written by k_cgm_begin); null: one system, by
+    int *nact;          // its flags. nact: the list's length
     int *any;           // 1 while any system is live
     double *part_a;     // [nsys][nblk_dsl] partial sums of <p, A p>
-    double *part_b;     // [nsys][nblk] partial sums of |r|^2
+    double *part_f;     // [nsys][kFoldParts] part_a in slices (lattices with more than kFoldAbove blocks)
+    double *part_b;     // [nsys][cgm_update_nblk] partial sums of |r|^2
     const size_t *off;  // [nsys] element offset of each system's p/x block
     double *shist;      // recorded scalars (hist_scalar_index), null without deferred updates
     void *rhist;        // recorded residuals: vector (dslot * kHistMax + j), 3 * Vh complex each
 };
 
 template <typename S> void cgm_begin(CgmState<S> *st, const CgmLaunch &L, hipStream_t stream);
-template <typename S> void cgm_scalars1(CgmState<S> *st, const CgmLaunch &L, hipStream_t stream);
-template <typename S> void cgm_scalars2(CgmState<S> *st, const CgmLaunch &L, hipStream_t stream);
-// r += beta_0 s ; partial |r|^2                        (inverter_cgm.cpp:50, 58)
+// beta recurrences; r += beta_0 s ; partial |r|^2        (inverter_cgm.cpp:47-58)
 template <typename S, typename VR>
-void cgm_axpy_norm(CgmState<S> *st, Vec<VR> r, Vec<VR> s, const CgmLaunch &L, hipStream_t stream);
-// x_k -= beta_k p_k ; p_k = zeta_k r + alpha_k p_k      (inverter_cgm.cpp:61-69)
+void cgm_update_r(CgmState<S> *st, Vec<VR> r, Vec<VR> s, const CgmLaunch &L, hipStream_t stream);
+// alpha recurrences, x_k -= beta_k p_k ; p_k = zeta_k r + alpha_k p_k ; drops, stop and pause
 template <typename S, typename VR, typename XR>
-void cgm_xp_update(CgmState<S> *st, XR *x, VR *p, Vec<VR> r, const CgmLaunch &L, hipStream_t stream);
+void cgm_update_p(CgmState<S> *st, XR *x, VR *p, Vec<VR> r, const CgmLaunch &L, hipStream_t stream);
 
 // ---- deferred solution updates (segment fold) of the listed systems with a history slot:
 // coefficients of each shift k < maxTermFold from the recorded scalars (coef: per slot and
@@ -189,5 +194,16 @@ void reduce_partials(const double *part, uint32_t nblk, int nrhs, double *out, h
 
 constexpr int kBlasNT = 256;
 inline uint32_t blas_nblk(uint32_t Vh) { return (Vh + kBlasNT - 1) / kBlasNT; }
+// Workgroups of the r and x/p updates over the sites: each sums the partials of the kernel before it,
+// so at most kBlasMaxBlocks (4 per CU), evenly loaded
+constexpr uint32_t kBlasMaxBlocks = 1024;
+inline uint32_t cgm_update_nblk(uint32_t Vh)
+{
+    const uint32_t n = blas_nblk(Vh), per = (n + kBlasMaxBlocks - 1) / kBlasMaxBlocks;
+    return (n + per - 1) / per;
+}
+// Above kFoldAbove partials (32 KB) a system's partials are first summed in kFoldParts slices: at
+// 48^3x96 the 1024 workgroups would each read 166 KB
+constexpr uint32_t kFoldAbove = 4096, kFoldParts = 64;
 
 }  // namespace kq

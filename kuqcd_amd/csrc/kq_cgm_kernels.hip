@@ -2,10 +2,13 @@
 // with the recurrence scalars kept in device memory, plus the start-up and
 // reliable-update kernels of the mixed-precision solver.
 //
-// Per iteration:  begin -> D (p0 -> tmp) -> D + axmy + <p0,s> -> scalars1 ->
-//                 r += b0 s, |r|^2 -> scalars2 -> x/p update of every live shift
+// Per iteration:  begin (several systems) -> D (p0 -> tmp) -> D + axmy + <p0,s> ->
+//                 beta, r += b0 s, |r|^2 -> alpha, x/p update of every live shift
 // Reductions are two-stage and deterministic: each workgroup writes one FP64
-// partial sum, and one workgroup adds the partials in a fixed order.
+// partial sum, and every workgroup that needs the total adds the partials in the same fixed
+// order. The scalar recurrences run in a workgroup of their own beside the vector update that
+// needs the scalar, instead of in one-workgroup kernels between the vector kernels (3-5 us each,
+// plus 1.2 us from one kernel to the next: a third of an iteration at 8^4 and 16^4).
 #include "kq_cgm_kernels.h"
 
 namespace kq {
@@ -28,20 +31,38 @@ __device__ inline double block_reduce_fixed(const double *part, uint32_t n)
     return lds[0];
 }
 
-// ------------------------------------------------------------ begin
-template <typename S> __global__ void k_cgm_begin(CgmState<S> *st, int nsys, int *rlist, int *nact, int *any)
+// The same sum in every thread of a workgroup of 256: `lds` holds 4 doubles, used by this call alone
+__device__ inline double sum_partials(const double *part, uint32_t n, double *lds)
 {
-    if (threadIdx.x != 0)
-        return;
+    double acc = 0.0;
+    for (uint32_t i = threadIdx.x; i < n; i += 256)
+        acc += part[i];
+    acc = wave_sum(acc);
+    if ((threadIdx.x & (kWave - 1)) == 0)
+        lds[threadIdx.x / kWave] = acc;
+    __syncthreads();
+    return (lds[0] + lds[1]) + (lds[2] + lds[3]);
+}
+
+// ------------------------------------------------------------ begin
+// One wave: the compact list of the live systems, in system order
+template <typename S>
+__global__ void __launch_bounds__(64) k_cgm_begin(CgmState<S> *st, int nsys, int *rlist, int *nact, int *any)
+{
+    const int lane = threadIdx.x;
     int n = 0;
-    for (int r = 0; r < nsys; ++r) {
-        const int live = (st[r].stop == 0) && (st[r].pause == 0);
-        st[r].run = live;
+    for (int r0 = 0; r0 < nsys; r0 += 64) {
+        const int r = r0 + lane;
+        const bool live = r < nsys && st[r].stop == 0 && st[r].pause == 0;
+        const unsigned long long m = __ballot(live);
         if (live)
-            rlist[n++] = r;
+            rlist[n + __popcll(m & ((1ull << lane) - 1ull))] = r;
+        n += __popcll(m);
     }
-    *nact = n;
-    *any = n > 0;
+    if (lane == 0) {
+        *nact = n;
+        *any = n > 0;
+    }
 }
 
 template <typename S> void cgm_begin(CgmState<S> *st, const CgmLaunch &L, hipStream_t stream)
@@ -50,227 +71,253 @@ template <typename S> void cgm_begin(CgmState<S> *st, const CgmLaunch &L, hipStr
     KQ_HIP_CHECK(hipGetLastError());
 }
 
-// ------------------------------------------------------------ scalars 1
-// pAp = <p0, s>;  beta_0 = -|r|^2 / pAp;  zeta/beta recurrences of the shifted
-// systems (inverter_cgm.cpp:47-57). The FP contraction is switched off so the
-// recurrence rounds exactly as written; the double literal 1.0 of the
-// reference keeps its type (the denominator is formed in double for S=float).
+// System of list slot `slot`, or -1 when the slot is empty. Without a list (a runner of one
+// system) the flag says whether the system iterates: `live` for the hopping terms and the r update,
+// its copy `run` for the x/p update, whose scalar workgroup rewrites `live`.
+__device__ inline int system_of(int slot, const int *rlist, const int *nact, const int *flag)
+{
+    if (nact == nullptr)
+        return *flag != 0 ? 0 : -1;
+    return slot < *nact ? rlist[slot] : -1;
+}
+
+// ------------------------------------------------------------ partial sums of large lattices
+// out[r][b] = sum of slice b of the kFoldParts slices of part[r][0..n)
 template <typename S>
-__global__ void __launch_bounds__(256) k_cgm_scalars1(CgmState<S> *st, const int *rlist, const int *nact,
-                                                      const double *part, uint32_t nblk, double *shist)
+__global__ void __launch_bounds__(256) k_fold_partials(const CgmState<S> *st, const int *rlist, const int *nact,
+                                                       const double *part, uint32_t n, double *out)
 {
-#pragma clang fp contract(off)
-    const int slot = blockIdx.x;
-    if (*nact <= slot)
+    __shared__ double lds[4];
+    const int r = system_of(blockIdx.y, rlist, nact, &st[0].live);
+    if (r < 0)
         return;
-    const int r = rlist[slot];
-    const double pAp_d = block_reduce_fixed(part + (size_t)r * nblk, nblk);
-    CgmState<S> &c = st[r];
-    // every thread reads the values the shifted updates share before any thread writes
-    const S B0 = -c.rr / (S)pAp_d;
-    const S Bm1 = c.Bm1, a0 = c.a[0];
-    const int mt = c.maxTerm;
-    const bool rec = shist != nullptr && c.dslot >= 0 && c.hist < kHistMax;
-    double *h = rec ? shist + hist_scalar_index(c.dslot, c.hist, 0, 0) : nullptr;
-    __syncthreads();
-    // one shifted system per thread; each touches only its own entries
-    for (int j = 1 + (int)threadIdx.x; j < mt; j += blockDim.x) {
-        const S zm1 = c.Zm1[j], z = c.Z[j];
-        const S num = Bm1 * zm1;
-        const S t1 = B0 * a0 * (zm1 - z);
-        const S t2 = zm1 * Bm1;
-        const S t3 = c.shift[j] * B0;
-        const S rr1 = (S)((double)num / ((double)t1 + (double)t2 * (1.0 - (double)t3)));
-        const S znew = z * rr1, bnew = B0 * rr1;
-        c.Zm1[j] = z;
-        c.Z[j] = znew;
-        c.B[j] = bnew;
-        if (rec) {
-            h[j] = (double)bnew;
-            h[kMaxShift + j] = (double)znew;
-        }
-    }
-    if (threadIdx.x == 0) {
-        c.B[0] = B0;
-        c.Bm1 = B0;
-        if (rec) {
-            h[0] = (double)B0;
-            h[kMaxShift] = (double)c.Z[0];
-        }
-    }
+    const uint32_t per = (n + kFoldParts - 1) / kFoldParts, i0 = blockIdx.x * per;
+    const uint32_t m = i0 >= n ? 0u : min(per, n - i0);
+    const double v = sum_partials(part + (size_t)r * n + i0, m, lds);
+    if (threadIdx.x == 0)
+        out[(size_t)r * kFoldParts + blockIdx.x] = v;
 }
 
-template <typename S> void cgm_scalars1(CgmState<S> *st, const CgmLaunch &L, hipStream_t stream)
-{
-    hipLaunchKernelGGL(k_cgm_scalars1<S>, dim3(L.nlaunch), dim3(256), 0, stream, st, L.rlist, L.nact, L.part_a,
-                       L.nblk_dsl, L.shist);
-    KQ_HIP_CHECK(hipGetLastError());
-}
-
-// ------------------------------------------------------------ scalars 2
-// |r|^2 new, alpha recurrences, drop converged shifts from the end,
-// iteration count and stop flag (inverter_cgm.cpp:58-78); pause flag for the
-// reliable-update schedule.
-template <typename S>
-__global__ void __launch_bounds__(256) k_cgm_scalars2(CgmState<S> *st, const int *rlist, const int *nact,
-                                                      const double *part, uint32_t nblk, double *shist)
-{
-#pragma clang fp contract(off)
-    const int slot = blockIdx.x;
-    if (*nact <= slot)
-        return;
-    const int r = rlist[slot];
-    const double l2_d = block_reduce_fixed(part + (size_t)r * nblk, nblk);
-    CgmState<S> &c = st[r];
-    // every thread reads the values the shifted updates share before thread 0 writes them
-    const S lambda2 = (S)l2_d;
-    const S a0 = lambda2 / c.rr;
-    const S B0 = c.B[0];
-    const int mt = c.maxTerm;
-    const bool rec = shist != nullptr && c.dslot >= 0 && c.hist < kHistMax;
-    double *h = rec ? shist + hist_scalar_index(c.dslot, c.hist, 2, 0) : nullptr;
-    __syncthreads();
-    for (int j = 1 + (int)threadIdx.x; j < mt; j += blockDim.x) {
-        const S aj = a0 * c.Z[j] * c.B[j] / (c.Zm1[j] * B0);
-        c.a[j] = aj;
-        if (rec)
-            h[j] = (double)aj;
-    }
-    if (threadIdx.x != 0)
-        return;
-    c.a[0] = a0;
-    c.rr = lambda2;
-    c.maxTermUpd = mt;
-    if (rec) {
-        h[0] = (double)a0;
-        h[kMaxShift] = (double)mt;
-        c.hist += 1;
-    }
-    // drop converged shifts from the end of the list (inverter_cgm.cpp:71-76)
-    while (c.maxTerm > 0) {
-        const S lambda = c.Z[c.maxTerm - 1] * c.Z[c.maxTerm - 1] * lambda2;
-        if (!((double)lambda < c.tolk[c.maxTerm - 1]))
-            break;
-        c.maxTerm--;
-    }
-    c.iter += 1;
-    if (c.maxTerm <= 0 || c.iter >= c.maxIter)
-        c.stop = 1;
-    if (c.pause2 > 0.0 && l2_d < c.pause2 * c.r2max)
-        c.pause = 1;
-}
-
-template <typename S> void cgm_scalars2(CgmState<S> *st, const CgmLaunch &L, hipStream_t stream)
-{
-    hipLaunchKernelGGL(k_cgm_scalars2<S>, dim3(L.nlaunch), dim3(256), 0, stream, st, L.rlist, L.nact, L.part_b,
-                       L.nblk, L.shist);
-    KQ_HIP_CHECK(hipGetLastError());
-}
-
-// ------------------------------------------------------------ r += b0 s, |r|^2
+// ------------------------------------------------------------ beta, r += b0 s, |r|^2
+// beta_0 = -|r|^2 / <p0, s>, then r += beta_0 s with the partial sums of |r|^2
+// (inverter_cgm.cpp:47-58). The last workgroup of each system runs the zeta/beta recurrences of its
+// shifted systems instead, one shift per thread; no other workgroup reads what it writes. The FP
+// contraction is switched off so the recurrence rounds exactly as written; the double literal 1.0
+// of the reference keeps its type (the denominator is formed in double for S=float).
+// HBM-bound at 32^4 (r, s in, r and the history slot out, 5.8 TB/s); the sum of the partials
+// costs every workgroup about 1 us of L2 reads (16 KB at 32^4), hence at most kBlasMaxBlocks of
+// them, each with several site ranges.
 template <typename S, typename VR>
-__global__ void __launch_bounds__(kBlasNT) k_axpy_norm(const CgmState<S> *st, Vec<VR> r, Vec<VR> s,
-                                                       const int *rlist, const int *nact, double *part,
-                                                       uint32_t nblk, c2_t<VR> *rhist)
+__global__ void __launch_bounds__(kBlasNT) k_cgm_update_r(CgmState<S> *st, Vec<VR> r, Vec<VR> s, const int *rlist,
+                                                          const int *nact, const double *part_a, uint32_t na,
+                                                          double *part_b, c2_t<VR> *rhist, double *shist)
 {
+#pragma clang fp contract(off)
     using V2 = c2_t<VR>;
-    __shared__ double lds[kBlasNT / kWave];
-    const int slot = blockIdx.y;
-    if (*nact <= slot)
+    static_assert(kBlasNT == 256, "sum_partials");
+    __shared__ double lsum[4], lds[kBlasNT / kWave];
+    const int rh = system_of(blockIdx.y, rlist, nact, &st[0].live);
+    const uint32_t nb = gridDim.x - 1;  // workgroups over the sites; the last one has the scalars
+    const bool scalars = blockIdx.x == nb;
+    if (rh < 0) {
+        if (nact == nullptr && scalars && threadIdx.x == 0)
+            st[0].run = 0;
         return;
-    const int rh = rlist[slot];
-    const VR b0 = (VR)st[rh].B[0];
-    const uint32_t i = blockIdx.x * kBlasNT + threadIdx.x;
+    }
+    const double pAp = sum_partials(part_a + (size_t)rh * na, na, lsum);
+    CgmState<S> &c = st[rh];
+    const S B0 = -c.rr / (S)pAp;
+    if (scalars) {
+        // every thread reads the values the shifted updates share before any thread writes
+        const S Bm1 = c.Bm1, a0 = c.a[0];
+        const int mt = c.maxTerm;
+        const bool rec = shist != nullptr && c.dslot >= 0 && c.hist < kHistMax;
+        double *h = rec ? shist + hist_scalar_index(c.dslot, c.hist, 0, 0) : nullptr;
+        __syncthreads();
+        // one shifted system per thread; each touches only its own entries
+        for (int j = 1 + (int)threadIdx.x; j < mt; j += blockDim.x) {
+            const S zm1 = c.Zm1[j], z = c.Z[j];
+            const S num = Bm1 * zm1;
+            const S t1 = B0 * a0 * (zm1 - z);
+            const S t2 = zm1 * Bm1;
+            const S t3 = c.shift[j] * B0;
+            const S rr1 = (S)((double)num / ((double)t1 + (double)t2 * (1.0 - (double)t3)));
+            const S znew = z * rr1, bnew = B0 * rr1;
+            c.Zm1[j] = z;
+            c.Z[j] = znew;
+            c.B[j] = bnew;
+            if (rec) {
+                h[j] = (double)bnew;
+                h[kMaxShift + j] = (double)znew;
+            }
+        }
+        if (threadIdx.x == 0) {
+            c.B[0] = B0;
+            c.Bm1 = B0;
+            c.rr_prev = c.rr;
+            c.maxTermPrev = mt;
+            c.run = 1;
+            if (rec) {
+                h[0] = (double)B0;
+                h[kMaxShift] = (double)c.Z[0];
+            }
+        }
+        return;
+    }
+    const VR b0 = (VR)B0;
+    const int ds = c.dslot, hj = c.hist;
+    V2 *hist = (rhist != nullptr && ds >= 0 && hj < kHistMax) ? rhist + ((size_t)ds * kHistMax + hj) * 3 * r.Vh : nullptr;
     double acc = 0.0;
-    if (i < r.Vh) {
+    for (uint32_t i = blockIdx.x * kBlasNT + threadIdx.x; i < r.Vh; i += nb * kBlasNT) {
         V2 rv[3], sv[3];
         r.load(rh, i, rv);
         s.load(rh, i, sv);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            rv[c].x += b0 * sv[c].x;
-            rv[c].y += b0 * sv[c].y;
-            acc += (double)rv[c].x * (double)rv[c].x + (double)rv[c].y * (double)rv[c].y;
+        for (int k = 0; k < 3; ++k) {
+            rv[k].x = fmadd(b0, sv[k].x, rv[k].x);
+            rv[k].y = fmadd(b0, sv[k].y, rv[k].y);
+            acc += (double)rv[k].x * (double)rv[k].x + (double)rv[k].y * (double)rv[k].y;
         }
         r.store(rh, i, rv);
-        const int ds = st[rh].dslot, hj = st[rh].hist;
-        if (rhist != nullptr && ds >= 0 && hj < kHistMax) {
-            V2 *h = rhist + ((size_t)ds * kHistMax + hj) * 3 * r.Vh + i;
+        if (hist != nullptr) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c)
-                st_nt(h + (size_t)c * r.Vh, rv[c]);
+            for (int k = 0; k < 3; ++k)
+                st_nt(hist + (size_t)k * r.Vh + i, rv[k]);
         }
     }
     const double tot = block_sum<kBlasNT>(acc, lds);
     if (threadIdx.x == 0)
-        part[(size_t)rh * nblk + blockIdx.x] = tot;
+        part_b[(size_t)rh * nb + blockIdx.x] = tot;
 }
 
 template <typename S, typename VR>
-void cgm_axpy_norm(CgmState<S> *st, Vec<VR> r, Vec<VR> s, const CgmLaunch &L, hipStream_t stream)
+void cgm_update_r(CgmState<S> *st, Vec<VR> r, Vec<VR> s, const CgmLaunch &L, hipStream_t stream)
 {
-    hipLaunchKernelGGL((k_axpy_norm<S, VR>), dim3(L.nblk, L.nlaunch), dim3(kBlasNT), 0, stream, st, r, s, L.rlist,
-                       L.nact, L.part_b, L.nblk, static_cast<c2_t<VR> *>(L.rhist));
+    const double *part = L.part_a;
+    uint32_t na = L.nblk_dsl;
+    if (na > kFoldAbove) {
+        hipLaunchKernelGGL(k_fold_partials<S>, dim3(kFoldParts, L.nlaunch), dim3(256), 0, stream, st, L.rlist, L.nact,
+                           L.part_a, na, L.part_f);
+        KQ_HIP_CHECK(hipGetLastError());
+        part = L.part_f;
+        na = kFoldParts;
+    }
+    hipLaunchKernelGGL((k_cgm_update_r<S, VR>), dim3(cgm_update_nblk(L.Vh) + 1, L.nlaunch), dim3(kBlasNT), 0, stream, st,
+                       r, s, L.rlist, L.nact, part, na, L.part_b, static_cast<c2_t<VR> *>(L.rhist), L.shist);
     KQ_HIP_CHECK(hipGetLastError());
 }
 
-// ------------------------------------------------------------ x/p update
+// ------------------------------------------------------------ alpha, x/p update
+// |r|^2, alpha_0 = |r_new|^2 / |r_old|^2, then x_k -= beta_k p_k and p_k = zeta_k r + alpha_k p_k
+// (inverter_cgm.cpp:58-69). The last workgroup of each system instead records the alphas, drops
+// converged shifts from the end, counts the iteration and sets the stop and pause flags
+// (inverter_cgm.cpp:70-78); the others read none of the fields it writes (rr_prev, maxTermPrev, run
+// and the betas and zetas were written by k_cgm_update_r).
 template <typename S, typename VR, typename XR>
-__global__ void __launch_bounds__(kBlasNT) k_xp_update(const CgmState<S> *st, XR *x, VR *p, Vec<VR> r,
-                                                       const size_t *off, const int *rlist, const int *nact)
+__global__ void __launch_bounds__(kBlasNT) k_cgm_update_p(CgmState<S> *st, XR *x, VR *p, Vec<VR> r, const size_t *off,
+                                                          const int *rlist, const int *nact, const double *part_b,
+                                                          double *shist)
 {
+#pragma clang fp contract(off)
     using V2 = c2_t<VR>;
     using X2 = c2_t<XR>;
-    const int slot = blockIdx.y;
-    if (*nact <= slot)
+    __shared__ double lsum[4];
+    const int rh = system_of(blockIdx.y, rlist, nact, &st[0].run);
+    if (rh < 0)
         return;
-    const int rh = rlist[slot];
-    const uint32_t i = blockIdx.x * kBlasNT + threadIdx.x;
-    const uint32_t Vh = r.Vh;
-    if (i >= Vh)
+    const uint32_t nb = gridDim.x - 1;
+    const double l2_d = sum_partials(part_b + (size_t)rh * nb, nb, lsum);
+    CgmState<S> &c = st[rh];
+    const S lambda2 = (S)l2_d;
+    const S a0 = lambda2 / c.rr_prev;
+    const S B0 = c.B[0];
+    const int mt = c.maxTermPrev;
+    const bool defer = c.dslot >= 0;
+    if (blockIdx.x == nb) {
+        const int hj = c.hist;
+        const bool rec = shist != nullptr && defer && hj < kHistMax;
+        double *h = rec ? shist + hist_scalar_index(c.dslot, hj, 2, 0) : nullptr;
+        __syncthreads();
+        for (int j = 1 + (int)threadIdx.x; j < mt; j += blockDim.x) {
+            const S aj = a0 * c.Z[j] * c.B[j] / (c.Zm1[j] * B0);
+            c.a[j] = aj;
+            if (rec)
+                h[j] = (double)aj;
+        }
+        if (threadIdx.x != 0)
+            return;
+        c.a[0] = a0;
+        c.rr = lambda2;
+        c.maxTermUpd = mt;
+        if (rec) {
+            h[0] = (double)a0;
+            h[kMaxShift] = (double)mt;
+            c.hist = hj + 1;
+        }
+        // drop converged shifts from the end of the list (inverter_cgm.cpp:71-76)
+        int left = mt;
+        while (left > 0) {
+            const S lambda = c.Z[left - 1] * c.Z[left - 1] * lambda2;
+            if (!((double)lambda < c.tolk[left - 1]))
+                break;
+            left--;
+        }
+        c.maxTerm = left;
+        const int iter = c.iter + 1;
+        c.iter = iter;
+        const bool stop = left <= 0 || iter >= c.maxIter;
+        const bool pause = c.pause2 > 0.0 && l2_d < c.pause2 * c.r2max;
+        if (stop)
+            c.stop = 1;
+        if (pause)
+            c.pause = 1;
+        c.live = !stop && !pause;
         return;
-    const CgmState<S> &c = st[rh];
+    }
     // a system with deferred solution updates keeps only p_0 current (its x_k and p_k, k >= 1,
     // are brought up to date by the next segment fold)
-    const bool defer = c.dslot >= 0;
-    const int m = defer ? 1 : c.maxTermUpd;
+    const int m = defer ? 1 : mt;
     const size_t o = off[rh];
-    V2 rv[3];
-    r.load(rh, i, rv);
-    for (int k = 0; k < m; ++k) {
-        const size_t base = o + (size_t)k * 3 * Vh + i;
-        const XR bk = (XR)c.B[k];
-        const VR zk = (VR)c.Z[k], ak = (VR)c.a[k];
-        V2 *pp = reinterpret_cast<V2 *>(p) + base;
-        X2 *xx = reinterpret_cast<X2 *>(x) + base;
-        // streaming accesses except the store of the unshifted direction p_0,
-        // which the next hopping term gathers: the solutions and the shifted
-        // directions are not touched again before the next update
+    const uint32_t Vh = r.Vh;
+    for (uint32_t i = blockIdx.x * kBlasNT + threadIdx.x; i < Vh; i += nb * kBlasNT) {
+        V2 rv[3];
+        r.load(rh, i, rv);
+        for (int k = 0; k < m; ++k) {
+            const size_t base = o + (size_t)k * 3 * Vh + i;
+            const S bk = c.B[k], zk = c.Z[k];
+            const VR z = (VR)zk, a = (VR)(k == 0 ? a0 : a0 * zk * bk / (c.Zm1[k] * B0));
+            const XR b = (XR)bk;
+            V2 *pp = reinterpret_cast<V2 *>(p) + base;
+            X2 *xx = reinterpret_cast<X2 *>(x) + base;
+            // streaming accesses except the store of the unshifted direction p_0,
+            // which the next hopping term gathers: the solutions and the shifted
+            // directions are not touched again before the next update
 #pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-            const V2 pv = ld_nt(pp + (size_t)cc * Vh);
-            if (!defer) {
-                X2 xv = ld_nt(xx + (size_t)cc * Vh);
-                xv.x -= bk * (XR)pv.x;
-                xv.y -= bk * (XR)pv.y;
-                st_nt(xx + (size_t)cc * Vh, xv);
+            for (int cc = 0; cc < 3; ++cc) {
+                const V2 pv = ld_nt(pp + (size_t)cc * Vh);
+                if (!defer) {
+                    X2 xv = ld_nt(xx + (size_t)cc * Vh);
+                    xv.x = fmadd(-b, (XR)pv.x, xv.x);
+                    xv.y = fmadd(-b, (XR)pv.y, xv.y);
+                    st_nt(xx + (size_t)cc * Vh, xv);
+                }
+                V2 np;
+                np.x = fmadd(z, rv[cc].x, a * pv.x);
+                np.y = fmadd(z, rv[cc].y, a * pv.y);
+                if (k == 0)
+                    pp[(size_t)cc * Vh] = np;
+                else
+                    st_nt(pp + (size_t)cc * Vh, np);
             }
-            V2 np;
-            np.x = zk * rv[cc].x + ak * pv.x;
-            np.y = zk * rv[cc].y + ak * pv.y;
-            if (k == 0)
-                pp[(size_t)cc * Vh] = np;
-            else
-                st_nt(pp + (size_t)cc * Vh, np);
         }
     }
 }
 
 template <typename S, typename VR, typename XR>
-void cgm_xp_update(CgmState<S> *st, XR *x, VR *p, Vec<VR> r, const CgmLaunch &L, hipStream_t stream)
+void cgm_update_p(CgmState<S> *st, XR *x, VR *p, Vec<VR> r, const CgmLaunch &L, hipStream_t stream)
 {
-    hipLaunchKernelGGL((k_xp_update<S, VR, XR>), dim3(L.nblk, L.nlaunch), dim3(kBlasNT), 0, stream, st, x, p, r, L.off,
-                       L.rlist, L.nact);
+    hipLaunchKernelGGL((k_cgm_update_p<S, VR, XR>), dim3(cgm_update_nblk(L.Vh) + 1, L.nlaunch), dim3(kBlasNT), 0, stream,
+                       st, x, p, r, L.off, L.rlist, L.nact, L.part_b, L.shist);
     KQ_HIP_CHECK(hipGetLastError());
 }
 
@@ -306,6 +353,7 @@ __global__ void __launch_bounds__(256) k_cgm_init_list(CgmState<S> *st, const in
     // the reference's do-while runs at least one iteration even for max_iter <= 0
     c.stop = (c.nshift <= 0) ? 1 : 0;
     c.run = 0;
+    c.live = !c.stop;
 }
 
 template <typename S>
@@ -430,6 +478,7 @@ template <typename S> __global__ void k_cgm_restart_list(CgmState<S> *st, const 
     }
     c.r2max = (double)c.rr;
     c.pause = 0;
+    c.live = !c.stop;
     c.hist = 0;
 }
 
@@ -718,8 +767,6 @@ void reduce_partials(const double *part, uint32_t nblk, int nrhs, double *out, h
 // ------------------------------------------------------------ instantiations
 #define KQ_INST_S(S)                                                                                          \
     template void cgm_begin<S>(CgmState<S> *, const CgmLaunch &, hipStream_t);                                \
-    template void cgm_scalars1<S>(CgmState<S> *, const CgmLaunch &, hipStream_t);                             \
-    template void cgm_scalars2<S>(CgmState<S> *, const CgmLaunch &, hipStream_t);                             \
     template void cgm_init_list<S>(CgmState<S> *, const int *, const int *, int, const double *, uint32_t,    \
                                    hipStream_t);                                                              \
     template void rel_set_rr<S>(CgmState<S> *, const int *, const int *, int, const double *, uint32_t,       \
@@ -731,8 +778,8 @@ KQ_INST_S(double)
 KQ_INST_S(float)
 
 #define KQ_INST_SV(S, VR)                                                                                      \
-    template void cgm_axpy_norm<S, VR>(CgmState<S> *, Vec<VR>, Vec<VR>, const CgmLaunch &, hipStream_t);       \
-    template void cgm_xp_update<S, VR, VR>(CgmState<S> *, VR *, VR *, Vec<VR>, const CgmLaunch &, hipStream_t); \
+    template void cgm_update_r<S, VR>(CgmState<S> *, Vec<VR>, Vec<VR>, const CgmLaunch &, hipStream_t);        \
+    template void cgm_update_p<S, VR, VR>(CgmState<S> *, VR *, VR *, Vec<VR>, const CgmLaunch &, hipStream_t); \
     template void rel_fold<S, VR>(CgmState<S> *, double *, VR *, const size_t *, uint32_t, const int *,        \
                                   const int *, int, hipStream_t);                                             \
     template void copy_r_to_p<S, VR>(const CgmState<S> *, Vec<VR>, VR *, const size_t *, const int *,          \
