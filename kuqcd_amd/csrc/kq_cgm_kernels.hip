@@ -124,6 +124,13 @@ __global__ void __launch_bounds__(kBlasNT) k_cgm_update_r(CgmState<S> *st, Vec<V
             st[0].run = 0;
         return;
     }
+    // the first site range is requested before the partials are summed
+    V2 rv[3], sv[3];
+    uint32_t i = blockIdx.x * kBlasNT + threadIdx.x;
+    if (!scalars && i < r.Vh) {
+        r.load(rh, i, rv);
+        s.load(rh, i, sv);
+    }
     const double pAp = sum_partials(part_a + (size_t)rh * na, na, lsum);
     CgmState<S> &c = st[rh];
     const S B0 = -c.rr / (S)pAp;
@@ -168,10 +175,7 @@ __global__ void __launch_bounds__(kBlasNT) k_cgm_update_r(CgmState<S> *st, Vec<V
     const int ds = c.dslot, hj = c.hist;
     V2 *hist = (rhist != nullptr && ds >= 0 && hj < kHistMax) ? rhist + ((size_t)ds * kHistMax + hj) * 3 * r.Vh : nullptr;
     double acc = 0.0;
-    for (uint32_t i = blockIdx.x * kBlasNT + threadIdx.x; i < r.Vh; i += nb * kBlasNT) {
-        V2 rv[3], sv[3];
-        r.load(rh, i, rv);
-        s.load(rh, i, sv);
+    while (i < r.Vh) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             rv[k].x = fmadd(b0, sv[k].x, rv[k].x);
@@ -183,6 +187,11 @@ __global__ void __launch_bounds__(kBlasNT) k_cgm_update_r(CgmState<S> *st, Vec<V
 #pragma unroll
             for (int k = 0; k < 3; ++k)
                 st_nt(hist + (size_t)k * r.Vh + i, rv[k]);
+        }
+        i += nb * kBlasNT;
+        if (i < r.Vh) {
+            r.load(rh, i, rv);
+            s.load(rh, i, sv);
         }
     }
     const double tot = block_sum<kBlasNT>(acc, lds);
@@ -225,7 +234,19 @@ __global__ void __launch_bounds__(kBlasNT) k_cgm_update_p(CgmState<S> *st, XR *x
     const int rh = system_of(blockIdx.y, rlist, nact, &st[0].run);
     if (rh < 0)
         return;
-    const uint32_t nb = gridDim.x - 1;
+    const uint32_t nb = gridDim.x - 1, Vh = r.Vh;
+    // the first site range of r and p_0 is requested before the partials are summed
+    V2 *p0 = reinterpret_cast<V2 *>(p) + off[rh];
+    V2 rv[3], pv[3];
+    uint32_t i = blockIdx.x * kBlasNT + threadIdx.x;
+    const auto fetch = [&] {
+        r.load(rh, i, rv);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            pv[k] = ld_nt(p0 + (size_t)k * Vh + i);
+    };
+    if (blockIdx.x < nb && i < Vh)
+        fetch();
     const double l2_d = sum_partials(part_b + (size_t)rh * nb, nb, lsum);
     CgmState<S> &c = st[rh];
     const S lambda2 = (S)l2_d;
@@ -277,39 +298,43 @@ __global__ void __launch_bounds__(kBlasNT) k_cgm_update_p(CgmState<S> *st, XR *x
     // a system with deferred solution updates keeps only p_0 current (its x_k and p_k, k >= 1,
     // are brought up to date by the next segment fold)
     const int m = defer ? 1 : mt;
-    const size_t o = off[rh];
-    const uint32_t Vh = r.Vh;
-    for (uint32_t i = blockIdx.x * kBlasNT + threadIdx.x; i < Vh; i += nb * kBlasNT) {
-        V2 rv[3];
-        r.load(rh, i, rv);
+    X2 *x0 = reinterpret_cast<X2 *>(x) + off[rh];
+    while (i < Vh) {
         for (int k = 0; k < m; ++k) {
-            const size_t base = o + (size_t)k * 3 * Vh + i;
+            const size_t base = (size_t)k * 3 * Vh + i;
             const S bk = c.B[k], zk = c.Z[k];
             const VR z = (VR)zk, a = (VR)(k == 0 ? a0 : a0 * zk * bk / (c.Zm1[k] * B0));
             const XR b = (XR)bk;
-            V2 *pp = reinterpret_cast<V2 *>(p) + base;
-            X2 *xx = reinterpret_cast<X2 *>(x) + base;
+            V2 *pp = p0 + base;
+            X2 *xx = x0 + base;
+            if (k > 0) {
+#pragma unroll
+                for (int cc = 0; cc < 3; ++cc)
+                    pv[cc] = ld_nt(pp + (size_t)cc * Vh);
+            }
             // streaming accesses except the store of the unshifted direction p_0,
             // which the next hopping term gathers: the solutions and the shifted
             // directions are not touched again before the next update
 #pragma unroll
             for (int cc = 0; cc < 3; ++cc) {
-                const V2 pv = ld_nt(pp + (size_t)cc * Vh);
                 if (!defer) {
                     X2 xv = ld_nt(xx + (size_t)cc * Vh);
-                    xv.x = fmadd(-b, (XR)pv.x, xv.x);
-                    xv.y = fmadd(-b, (XR)pv.y, xv.y);
+                    xv.x = fmadd(-b, (XR)pv[cc].x, xv.x);
+                    xv.y = fmadd(-b, (XR)pv[cc].y, xv.y);
                     st_nt(xx + (size_t)cc * Vh, xv);
                 }
                 V2 np;
-                np.x = fmadd(z, rv[cc].x, a * pv.x);
-                np.y = fmadd(z, rv[cc].y, a * pv.y);
+                np.x = fmadd(z, rv[cc].x, a * pv[cc].x);
+                np.y = fmadd(z, rv[cc].y, a * pv[cc].y);
                 if (k == 0)
                     pp[(size_t)cc * Vh] = np;
                 else
                     st_nt(pp + (size_t)cc * Vh, np);
             }
         }
+        i += nb * kBlasNT;
+        if (i < Vh)
+            fetch();
     }
 }
 

@@ -372,9 +372,13 @@ __global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL
     using V2 = c2_t<SR>;
     constexpr bool SA = (LAY & LAY_HOST_SRC) != 0, DA = (LAY & LAY_HOST_DST) != 0;
     constexpr int NT = 64 * S;
-    __shared__ R red[S][NR][6][64];
+    // results of half the waves: the other half adds its own to them, so that the workgroup's LDS is
+    // half of one slot per wave (blocks of 8 FP32 right-hand sides: 24.6 instead of 49 KB, 4
+    // instead of 3 workgroups per CU; LinkF + LinkF12 16^3x32 35.6 -> 30.3 us, 32^4 213 -> 203)
+    constexpr int H = S / 2, DOTS = EPI == EPI_AXMY_DOT ? NR : 1;
+    __shared__ R red[H][NR][6][64];
     __shared__ uint32_t site[64];
-    __shared__ double lds[S];
+    __shared__ double lds[S][DOTS];
     if (a.run != nullptr && *a.run == 0)
         return;  // uniform over the grid
     const int nact = a.nact ? *a.nact : a.nrhs;
@@ -402,15 +406,24 @@ __global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL
     }
     if (w == 0)
         site[lane] = valid ? s : 0xffffffffu;
+    if (w >= H) {
 #pragma unroll
-    for (int j = 0; j < NR; ++j)
+        for (int j = 0; j < NR; ++j)
 #pragma unroll
-        for (int k = 0; k < 6; ++k)
-            red[w][j][k][lane] = acc[j][k];
+            for (int k = 0; k < 6; ++k)
+                red[w - H][j][k][lane] = acc[j][k];
+    }
     __syncthreads();
-    // 192 complex results per right-hand side, summed over the waves in their order; consecutive
+    if (w < H) {
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+                red[w][j][k][lane] += acc[j][k];
+    }
+    __syncthreads();
+    // 192 complex results per right-hand side, summed over the slots in their order; consecutive
     // threads take consecutive entries of the destination's layout
-    constexpr int DOTS = EPI == EPI_AXMY_DOT ? NR : 1;
     double d[DOTS];
 #pragma unroll
     for (int j = 0; j < DOTS; ++j)
@@ -426,7 +439,7 @@ __global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL
                 continue;
             R x = red[0][j][2 * c][l], y = red[0][j][2 * c + 1][l];
 #pragma unroll
-            for (int k = 1; k < S; ++k) {
+            for (int k = 1; k < H; ++k) {
                 x += red[k][j][2 * c][l];
                 y += red[k][j][2 * c + 1][l];
             }
@@ -448,11 +461,20 @@ __global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL
     if constexpr (EPI == EPI_AXMY_DOT) {
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
-            const double tot = block_sum<NT>(d[j], lds);
-            if (threadIdx.x == 0 && j0 + j < nact)
-                a.partial[(size_t)rr[j] * a.nblk + blockIdx.x] = tot;
-            __syncthreads();
+            const double v = wave_sum(d[j]);
+            if (lane == 0)
+                lds[w][j] = v;
         }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+            if (threadIdx.x == j && j0 + j < nact) {
+                double tot = 0.0;
+#pragma unroll
+                for (int k = 0; k < S; ++k)
+                    tot += lds[k][j];
+                a.partial[(size_t)rr[j] * a.nblk + blockIdx.x] = tot;
+            }
     }
 }
 
@@ -639,6 +661,16 @@ static uint32_t launch_epi(DslashArgs<LF, LL, SR> a, int epi, int nt, int cap, h
         constexpr int S = NR <= 2 ? 8 : 4;
         if (dslash_split_waves(kDouble, a.g, (a.nrhs + NR - 1) / NR, NR) == S) {
             a.nblk = dslash_grid(a.g.Vh, 64);
+            // 16-bit long links in blocks of 8 on more than 48 K sites: 2 waves of 8 hops, whose
+            // 24.8 KB of LDS let all workgroups of a middle-sized lattice run at once (16^3x32
+            // 35 us with 4 waves, 30 with 2; 24^4 74 and 73.5, 48^4 1093 and 1040; but 16^4 17.6
+            // and 24)
+            if constexpr (NR == 8 && LL::kBytes < 40) {
+                if (a.g.Vh > 49152u) {
+                    launch_split<LF, LL, SR, NR, 2>(a, epi, st);
+                    return a.nblk;
+                }
+            }
             launch_split<LF, LL, SR, NR, S>(a, epi, st);
             return a.nblk;
         }
