@@ -33,128 +33,87 @@ __device__ __forceinline__ uint32_t pack_bf16(float2 v)
     return (a >> 16) | (b & 0xffff0000u);
 }
 
-// acc = L(s) x  or  acc = L(n)^+ x, for the tap's link format
-template <class LK, bool NEG, typename R>
-__device__ __forceinline__ void tap_mul(const LK &lk, int qo, int mu, uint32_t s, uint32_t n, const float2 x[3],
-                                        R acc[6])
+// Neighbours of (s, coordinates) along the direction mu of a wave, a value uniform over the wave: hops
+// +1, +3, -1, -3 (the taps t = 4 mu + 0..3). The direction stays a run-time value, with its
+// coordinate, extent and weights selected: specialised code for each wave's direction behind
+// branches on the wave index was compiled wrongly (one wave took other taps' weights, and with
+// 16-bit links an address that was never set).
+struct DirNb {
+    uint32_t n[4];
+};
+__device__ __forceinline__ DirNb dir_neighbours(const Geom &g, uint32_t s, const SiteCoord &sc, int mu)
 {
-    float2 U[9];
+    const int c = mu == 0 ? sc.c[0] : mu == 1 ? sc.c[1] : mu == 2 ? sc.c[2] : sc.c[3];
+    const int L = g.L[mu];
+    const uint32_t stride = g.stride[mu];
+    const int h[4] = {1, 3, -1, -3};
+    DirNb d;
 #pragma unroll
-    for (int k = 0; k < 6; ++k)
-        acc[k] = 0;
-    if (!NEG) {
-        lk.load(qo, mu, s, U);
+    for (int t = 0; t < 4; ++t) {
+        const int v = wrap_add(c, h[t], L);
+        d.n[t] = s + (mu == 0 ? (uint32_t)((v >> 1) - (c >> 1)) : (uint32_t)(v - c) * stride);
+    }
+    return d;
+}
+
+// The kernel's first argument in the argument segment: values indexed by the direction come from there
+// by scalar loads (indexing the by-value argument itself would copy it to scratch memory)
+template <class T> __device__ __forceinline__ const T &first_arg()
+{
+    return *(const T *)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// The links of the four taps: every load is issued before any is used
+template <class LF, class LL>
+__device__ __forceinline__ void dir_links(const LF &fat, const LL &lng, int qo, int mu, uint32_t s, const DirNb &d,
+                                          float2 U[4][9])
+{
+    fat.load(qo, mu, s, U[0]);
+    lng.load(qo, mu, s, U[1]);
+    fat.load(1 - qo, mu, d.n[2], U[2]);
+    lng.load(1 - qo, mu, d.n[3], U[3]);
+}
+
+// v = U x for a forward tap (t < 2), U^+ x for a backward one
+__device__ __forceinline__ void tap_mul(int t, const float2 U[9], const float2 x[3], float2 v[3])
+{
+    float acc[6] = {0, 0, 0, 0, 0, 0};
+    if (t < 2) {
         umv_add(U, x, acc);
     } else {
-        lk.load(1 - qo, mu, n, U);
         udmv_sub(U, x, acc);
 #pragma unroll
         for (int k = 0; k < 6; ++k)
             acc[k] = -acc[k];
     }
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        v[k] = mk<float2>(acc[2 * k], acc[2 * k + 1]);
 }
 
-// (T_t in)(s) for a one-channel field `in` on parity 1-qo
-template <class LK, int MU, int H, bool NEG>
-__device__ __forceinline__ void tap1(const Geom &g, int qo, const LK &lk, uint32_t s, const SiteCoord &sc,
-                                     const float2 *in, float2 v[3])
+// (T_t in)(s) for a one-channel field `in` on parity 1-qo, the four taps of direction mu
+template <class LF, class LL>
+__device__ __forceinline__ void taps1_dir(const Geom &g, int qo, const LF &fat, const LL &lng, uint32_t s, int mu,
+                                          const float2 *in, float2 v[4][3])
 {
-    const uint32_t n = nb_index<MU>(g, s, sc, NEG ? -H : H);
-    float2 x[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-        x[c] = in[(size_t)c * g.Vh + n];
-    float acc[6];
-    tap_mul<LK, NEG>(lk, qo, MU, s, n, x, acc);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-        v[c] = mk<float2>(acc[2 * c], acc[2 * c + 1]);
-}
-
-// (T_t sum_ch wt[ch] in_ch)(s) for a kPtHidden-channel field
-template <class LK, int MU, int H, bool NEG>
-__device__ __forceinline__ void tap_comb(const Geom &g, int qo, const LK &lk, uint32_t s, const SiteCoord &sc,
-                                         const float2 *in, const float2 wt[kPtHidden], float2 v[3])
-{
-    const uint32_t n = nb_index<MU>(g, s, sc, NEG ? -H : H);
-    float2 x[3] = {mk<float2>(0.f, 0.f), mk<float2>(0.f, 0.f), mk<float2>(0.f, 0.f)};
-#pragma unroll
-    for (int ch = 0; ch < kPtHidden; ++ch) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const float2 p = cmulf(wt[ch], in[((size_t)ch * 3 + c) * g.Vh + n]);
-            x[c].x += p.x;
-            x[c].y += p.y;
-        }
-    }
-    float acc[6];
-    tap_mul<LK, NEG>(lk, qo, MU, s, n, x, acc);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-        v[c] = mk<float2>(acc[2 * c], acc[2 * c + 1]);
-}
-
-// Layer 2 with bfloat16 channels, the four taps of direction MU (t = 4 MU + 0..3: hops +1,
-// +3, -1, -3, as KQ_PT_FOR_TAPS orders them) added to acc in tap order. Every gather and link
-// load of the four is issued before any of them is used: written tap by tap, the compiler
-// waited for each 16-byte gather before issuing the next (81 of 102 loads followed by a full
-// wait) and the kernel ran at a third of the HBM rate.
-template <class LF, class LL, int MU>
-__device__ __forceinline__ void taps16_dir(const Geom &g, int qo, const LF &fat, const LL &lng, uint32_t s,
-                                           const SiteCoord &sc, const kq_v4u *in, const PtWeightsBF &w,
-                                           float2 acc[3])
-{
-    const uint32_t n[4] = {nb_index<MU>(g, s, sc, 1), nb_index<MU>(g, s, sc, 3), nb_index<MU>(g, s, sc, -1),
-                           nb_index<MU>(g, s, sc, -3)};
-    kq_v4u u[4][3];
+    const DirNb d = dir_neighbours(g, s, site_coords(g, s, qo), mu);
+    float2 x[4][3], U[4][9];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
-            u[t][c] = in[(size_t)c * g.Vh + n[t]];
-    float2 U[4][9];
-    fat.load(qo, MU, s, U[0]);
-    lng.load(qo, MU, s, U[1]);
-    fat.load(1 - qo, MU, n[2], U[2]);
-    lng.load(1 - qo, MU, n[3], U[3]);
+            x[t][c] = in[(size_t)c * g.Vh + d.n[t]];
+    dir_links(fat, lng, qo, mu, s, d, U);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        float2 wt[kPtHidden];
-#pragma unroll
-        for (int c = 0; c < kPtHidden; ++c)
-            wt[c] = unpack_w(w.w2[c][4 * MU + t]);
-        float2 x[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const float2 p0 = cmulf(wt[0], unpack_w(u[t][c].x)), p1 = cmulf(wt[1], unpack_w(u[t][c].y));
-            const float2 p2 = cmulf(wt[2], unpack_w(u[t][c].z)), p3 = cmulf(wt[3], unpack_w(u[t][c].w));
-            x[c] = mk<float2>((p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y));
-        }
-        float v[6];
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-            v[k] = 0;
-        if (t < 2) {
-            umv_add(U[t], x, v);
-        } else {
-            udmv_sub(U[t], x, v);
-#pragma unroll
-            for (int k = 0; k < 6; ++k)
-                v[k] = -v[k];
-        }
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            acc[k].x += v[2 * k];
-            acc[k].y += v[2 * k + 1];
-        }
-    }
+    for (int t = 0; t < 4; ++t)
+        tap_mul(t, U[t], x[t], v[t]);
 }
 
-// the 16 taps as (t, mu, hop, negative)
-#define KQ_PT_FOR_TAPS(X)                                                                                       \
-    X(0, 0, 1, false) X(1, 0, 3, false) X(2, 0, 1, true) X(3, 0, 3, true) X(4, 1, 1, false) X(5, 1, 3, false)   \
-        X(6, 1, 1, true) X(7, 1, 3, true) X(8, 2, 1, false) X(9, 2, 3, false) X(10, 2, 1, true)                \
-            X(11, 2, 3, true) X(12, 3, 1, false) X(13, 3, 3, false) X(14, 3, 1, true) X(15, 3, 3, true)
+// The layers and the weight gradient give the 64 sites of a workgroup to 4 waves, one per direction
+// (4 of the 16 taps each), as k_dslash_split does with its hops: 4 times the waves in flight and a
+// quarter of the chain of dependent loads of one thread per site, and workgroups of 64 sites end a
+// grid evenly. One thread per site in workgroups of 256 -> 4 waves per 64 sites: see the kernels.
+constexpr int kSites = 64;
 
 struct PtLayerArgs {
     Geom g;
@@ -170,60 +129,146 @@ struct PtLayerArgs {
     PtWeightsBF w;       // layer-1 form uses w1; layer-2 form uses w2 and w0
 };
 
+// acc[c][k] += sum over direction mu's taps of w1[c][t] (T_t in)_k
+template <class LF, class LL>
+__device__ __forceinline__ void layer1_dir(const PtLayerArgs &a, const LF &fat, const LL &lng, uint32_t s, int mu,
+                                           float2 acc[kPtHidden][3])
+{
+    float2 v[4][3];
+    taps1_dir(a.g, a.qo, fat, lng, s, mu, a.in, v);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < kPtHidden; ++c) {
+            const float2 w = unpack_w(a.w.w1[c][4 * mu + t]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float2 p = cmulf(w, v[t][k]);
+                acc[c][k].x += p.x;
+                acc[c][k].y += p.y;
+            }
+        }
+}
+
 // layer-1 form: out_c(x) = sum_t w1[c][t] (T_t in)(x), one input channel, kPtHidden outputs
 template <class LF, class LL>
 __global__ void __launch_bounds__(kNT) k_pt_layer1(const PtLayerArgs a, LF fat, LL lng)
 {
+    static_assert(kNT == 4 * kSites, "one wave per direction");
+    constexpr int NV = 2 * 3 * kPtHidden;
+    __shared__ float red[2][NV][kSites];
+    __shared__ uint32_t site[kSites];
     if (a.stop && *a.stop)
         return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     bool valid;
-    const uint32_t s = tile_site<kNT>(a.g, blockIdx.x, gridDim.x, threadIdx.x, valid);
-    if (!valid)
-        return;
-    const SiteCoord sc = site_coords(a.g, s, a.qo);
+    const uint32_t s = tile_site<kSites>(a.g, blockIdx.x, gridDim.x, lane, valid);
     float2 acc[kPtHidden][3];
 #pragma unroll
     for (int c = 0; c < kPtHidden; ++c)
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             acc[c][k] = mk<float2>(0.f, 0.f);
-#define KQ_TAP1(T, MU, H, NEG)                                                    \
-    {                                                                             \
-        float2 v[3];                                                              \
-        if (H == 1)                                                               \
-            tap1<LF, MU, H, NEG>(a.g, a.qo, fat, s, sc, a.in, v);                 \
-        else                                                                      \
-            tap1<LL, MU, H, NEG>(a.g, a.qo, lng, s, sc, a.in, v);                 \
-        _Pragma("unroll") for (int c = 0; c < kPtHidden; ++c)                     \
-        {                                                                         \
-            const float2 w = unpack_w(a.w.w1[c][T]);                              \
-            _Pragma("unroll") for (int k = 0; k < 3; ++k)                         \
-            {                                                                     \
-                const float2 p = cmulf(w, v[k]);                                  \
-                acc[c][k].x += p.x;                                               \
-                acc[c][k].y += p.y;                                               \
-            }                                                                     \
-        }                                                                         \
-    }
-    KQ_PT_FOR_TAPS(KQ_TAP1)
-#undef KQ_TAP1
-    if (a.out) {
+    if (valid)
+        layer1_dir(first_arg<PtLayerArgs>(), fat, lng, s, w, acc);
+    if (w == 0)
+        site[lane] = valid ? s : 0xffffffffu;
+    if (w >= 2) {
 #pragma unroll
         for (int c = 0; c < kPtHidden; ++c)
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-                a.out[((size_t)c * 3 + k) * a.g.Vh + s] = acc[c][k];
+            for (int k = 0; k < 3; ++k) {
+                red[w - 2][6 * c + 2 * k][lane] = acc[c][k].x;
+                red[w - 2][6 * c + 2 * k + 1][lane] = acc[c][k].y;
+            }
     }
-    if (a.out16) {
+    __syncthreads();
+    if (w < 2) {
+#pragma unroll
+        for (int c = 0; c < kPtHidden; ++c)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                red[w][6 * c + 2 * k][lane] += acc[c][k].x;
+                red[w][6 * c + 2 * k + 1][lane] += acc[c][k].y;
+            }
+    }
+    __syncthreads();
+    const uint32_t sl = site[lane];
+    if (sl == 0xffffffffu)
+        return;
+    const auto entry = [&](int c, int k) {
+        return mk<float2>(red[0][6 * c + 2 * k][lane] + red[1][6 * c + 2 * k][lane],
+                          red[0][6 * c + 2 * k + 1][lane] + red[1][6 * c + 2 * k + 1][lane]);
+    };
+    if (a.out) {  // wave w writes channel w
+        static_assert(kPtHidden == 4, "one wave per channel");
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            a.out[((size_t)w * 3 + k) * a.g.Vh + sl] = entry(w, k);
+    }
+    if (a.out16 && w < 3) {  // wave w writes colour w
         static_assert(kPtHidden == 4, "the bfloat16 hidden layout holds 4 channels");
+        kq_v4u u;
+        u.x = pack_bf16(entry(0, w));
+        u.y = pack_bf16(entry(1, w));
+        u.z = pack_bf16(entry(2, w));
+        u.w = pack_bf16(entry(3, w));
+        a.out16[(size_t)w * a.g.Vh + sl] = u;
+    }
+}
+
+// acc += sum over direction mu's taps of T_t( sum_c w2[c][t] in_c ). With bfloat16 channels one
+// 16-byte load brings the four channels of one colour, and the 12 gathers and the link loads are all
+// issued before any is used (written tap by tap the compiler waited for each 16-byte gather).
+template <class LF, class LL, bool H16>
+__device__ __forceinline__ void layer2_dir(const PtLayerArgs &a, const LF &fat, const LL &lng, uint32_t s, int mu,
+                                           float2 acc[3])
+{
+    const uint32_t Vh = a.g.Vh;
+    const DirNb d = dir_neighbours(a.g, s, site_coords(a.g, s, a.qo), mu);
+    float2 x[4][3], U[4][9];
+    kq_v4u u[4][3];
+    if constexpr (H16) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                u[t][c] = a.in16[(size_t)c * Vh + d.n[t]];
+        dir_links(fat, lng, a.qo, mu, s, d, U);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        float2 wt[kPtHidden];
+#pragma unroll
+        for (int ch = 0; ch < kPtHidden; ++ch)
+            wt[ch] = unpack_w(a.w.w2[ch][4 * mu + t]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if constexpr (H16) {
+                const float2 p0 = cmulf(wt[0], unpack_w(u[t][c].x)), p1 = cmulf(wt[1], unpack_w(u[t][c].y));
+                const float2 p2 = cmulf(wt[2], unpack_w(u[t][c].z)), p3 = cmulf(wt[3], unpack_w(u[t][c].w));
+                x[t][c] = mk<float2>((p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y));
+            } else {
+                x[t][c] = mk<float2>(0.f, 0.f);
+#pragma unroll
+                for (int ch = 0; ch < kPtHidden; ++ch) {
+                    const float2 p = cmulf(wt[ch], a.in[((size_t)ch * 3 + c) * Vh + d.n[t]]);
+                    x[t][c].x += p.x;
+                    x[t][c].y += p.y;
+                }
+            }
+        }
+    }
+    if constexpr (!H16)
+        dir_links(fat, lng, a.qo, mu, s, d, U);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        float2 v[3];
+        tap_mul(t, U[t], x[t], v);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            kq_v4u u;
-            u.x = pack_bf16(acc[0][k]);
-            u.y = pack_bf16(acc[1][k]);
-            u.z = pack_bf16(acc[2][k]);
-            u.w = pack_bf16(acc[3][k]);
-            a.out16[(size_t)k * a.g.Vh + s] = u;
+            acc[k].x += v[k].x;
+            acc[k].y += v[k].y;
         }
     }
 }
@@ -233,132 +278,133 @@ template <class LF, class LL, bool H16>
 __global__ void __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(1, 4)))
 k_pt_layer2(const PtLayerArgs a, LF fat, LL lng)
 {
+    __shared__ float red[4][6][kSites];
+    __shared__ double lre[kNT / kWave], lim[kNT / kWave];
     if (a.stop && *a.stop)
         return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     bool valid;
-    const uint32_t s = tile_site<kNT>(a.g, blockIdx.x, gridDim.x, threadIdx.x, valid);
-    const SiteCoord sc = site_coords(a.g, s, a.qo);
-    float2 acc[3];
-    const float2 w0 = unpack_w(a.w.w0);
+    const uint32_t s = tile_site<kSites>(a.g, blockIdx.x, gridDim.x, lane, valid);
+    float2 acc[3] = {mk<float2>(0.f, 0.f), mk<float2>(0.f, 0.f), mk<float2>(0.f, 0.f)};
+    if (valid)
+        layer2_dir<LF, LL, H16>(first_arg<PtLayerArgs>(), fat, lng, s, w, acc);
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-        acc[k] = a.skip ? cmulf(w0, a.skip[(size_t)k * a.g.Vh + s]) : mk<float2>(0.f, 0.f);
-    if constexpr (H16) {
-        taps16_dir<LF, LL, 0>(a.g, a.qo, fat, lng, s, sc, a.in16, a.w, acc);
-        taps16_dir<LF, LL, 1>(a.g, a.qo, fat, lng, s, sc, a.in16, a.w, acc);
-        taps16_dir<LF, LL, 2>(a.g, a.qo, fat, lng, s, sc, a.in16, a.w, acc);
-        taps16_dir<LF, LL, 3>(a.g, a.qo, fat, lng, s, sc, a.in16, a.w, acc);
-    } else {
-#define KQ_TAP2(T, MU, H, NEG)                                                     \
-    {                                                                              \
-        float2 wt[kPtHidden], v[3];                                                \
-        _Pragma("unroll") for (int c = 0; c < kPtHidden; ++c) wt[c] = unpack_w(a.w.w2[c][T]); \
-        if (H == 1)                                                                \
-            tap_comb<LF, MU, H, NEG>(a.g, a.qo, fat, s, sc, a.in, wt, v);          \
-        else                                                                       \
-            tap_comb<LL, MU, H, NEG>(a.g, a.qo, lng, s, sc, a.in, wt, v);          \
-        _Pragma("unroll") for (int k = 0; k < 3; ++k)                              \
-        {                                                                          \
-            acc[k].x += v[k].x;                                                    \
-            acc[k].y += v[k].y;                                                    \
-        }                                                                          \
+    for (int k = 0; k < 3; ++k) {
+        red[w][2 * k][lane] = acc[k].x;
+        red[w][2 * k + 1][lane] = acc[k].y;
     }
-        KQ_PT_FOR_TAPS(KQ_TAP2)
-#undef KQ_TAP2
-    }
-    if (valid) {
+    __syncthreads();
+    // wave k < 3 finishes colour k
+    double re = 0.0, im = 0.0;
+    if (w < 3 && valid) {
+        const size_t e = (size_t)w * a.g.Vh + s;
+        float2 z = a.skip ? cmulf(unpack_w(a.w.w0), a.skip[e]) : mk<float2>(0.f, 0.f);
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            a.out[(size_t)k * a.g.Vh + s] = acc[k];
+        for (int d = 0; d < 4; ++d) {
+            z.x += red[d][2 * w][lane];
+            z.y += red[d][2 * w + 1][lane];
+        }
+        a.out[e] = z;
+        if (a.dotq) {
+            const float2 d = a.dotq[e];
+            re = (double)d.x * z.x + (double)d.y * z.y;
+            im = (double)d.x * z.y - (double)d.y * z.x;
+        }
     }
     if (a.dotq) {
-        __shared__ double lre[kNT / kWave], lim[kNT / kWave];
-        double re = 0.0, im = 0.0;
-        if (valid) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const float2 d = a.dotq[(size_t)k * a.g.Vh + s];
-                re += (double)d.x * acc[k].x + (double)d.y * acc[k].y;
-                im += (double)d.x * acc[k].y - (double)d.y * acc[k].x;
-            }
-        }
         re = wave_sum(re);
         im = wave_sum(im);
-        if ((threadIdx.x & (kWave - 1)) == 0) {
-            lre[threadIdx.x / kWave] = re;
-            lim[threadIdx.x / kWave] = im;
+        if (lane == 0) {
+            lre[w] = re;
+            lim[w] = im;
         }
         __syncthreads();
         if (threadIdx.x == 0) {
-            double sr = 0.0, si = 0.0;
-            for (int w = 0; w < kNT / kWave; ++w) {
-                sr += lre[w];
-                si += lim[w];
-            }
-            a.part[2 * blockIdx.x] = sr;
-            a.part[2 * blockIdx.x + 1] = si;
+            a.part[2 * blockIdx.x] = (lre[0] + lre[1]) + lre[2];
+            a.part[2 * blockIdx.x + 1] = (lim[0] + lim[1]) + lim[2];
         }
     }
 }
 
-// P[c][t] = sum over sites y of parity qo of <(T_t in)(y), b_c(y)>;
-// part[blk][c*16 + t] (complex, FP64)
+// P[c][t] = sum over sites y of parity qo of <(T_t in)(y), b_c(y)> for the two (in, b) pairs of a
+// gradient (blockIdx.y); part[pair][blk][c*16 + t] (complex, FP64).
+// Each wave forms the four tap vectors of its direction for the workgroup's 64 sites in LDS; then
+// every thread owns one (c, t) and a quarter of the sites and adds the FP64 products over them.
+// (Before, each thread kept its site and every one of the 64 complex sums was reduced over the
+// wave by 12 shuffles, 1536 in all: 41 us a pair at 16^4.) The strides of 98 and 26 floats put the
+// 64 threads of a wave on distinct banks in both phases.
+struct PtGradArgs {
+    const float2 *in[2], *b[2];
+};
+
+constexpr int kTapStride = 6 * kPtTaps + 2, kChanStride = 6 * kPtHidden + 2;
+
 template <class LF, class LL>
-__global__ void __launch_bounds__(kNT) k_pt_wgrad(Geom g, int qo, LF fat, LL lng, const float2 *in,
-                                                  const float2 *b, double2 *part)
+__global__ void __launch_bounds__(kNT) k_pt_wgrad(Geom g, int qo, LF fat, LL lng, const PtGradArgs p, double2 *part)
 {
-    __shared__ double lds[kNT / kWave][kPtHidden * kPtTaps * 2];
+    constexpr int J = kPtHidden * kPtTaps;
+    static_assert(J == kWave && kPtHidden == kNT / kWave, "one (c, t) per lane, one channel per wave");
+    __shared__ __align__(8) float tv[kSites * kTapStride];
+    __shared__ __align__(8) float bv[kSites * kChanStride];
+    __shared__ double2 sum[kNT / kWave][J];
+    const float2 *in = p.in[blockIdx.y], *b = p.b[blockIdx.y];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     bool valid;
-    const uint32_t s = tile_site<kNT>(g, blockIdx.x, gridDim.x, threadIdx.x, valid);
-    const SiteCoord sc = site_coords(g, s, qo);
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    float2 bb[kPtHidden][3];
+    const uint32_t s = tile_site<kSites>(g, blockIdx.x, gridDim.x, lane, valid);
+    float2 *row = reinterpret_cast<float2 *>(tv + lane * kTapStride);
+    if (valid) {
+        float2 v[4][3];
+        taps1_dir(first_arg<Geom>(), qo, fat, lng, s, w, in, v);
 #pragma unroll
-    for (int c = 0; c < kPtHidden; ++c)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            bb[c][k] = valid ? b[((size_t)c * 3 + k) * g.Vh + s] : mk<float2>(0.f, 0.f);
-#define KQ_TAPG(T, MU, H, NEG)                                                    \
-    {                                                                             \
-        float2 v[3];                                                              \
-        if (H == 1)                                                               \
-            tap1<LF, MU, H, NEG>(g, qo, fat, s, sc, in, v);                       \
-        else                                                                      \
-            tap1<LL, MU, H, NEG>(g, qo, lng, s, sc, in, v);                       \
-        _Pragma("unroll") for (int c = 0; c < kPtHidden; ++c)                     \
-        {                                                                         \
-            double re = 0.0, im = 0.0;                                            \
-            _Pragma("unroll") for (int k = 0; k < 3; ++k)                         \
-            {                                                                     \
-                re += (double)v[k].x * bb[c][k].x + (double)v[k].y * bb[c][k].y;  \
-                im += (double)v[k].x * bb[c][k].y - (double)v[k].y * bb[c][k].x;  \
-            }                                                                     \
-            re = wave_sum(re);                                                    \
-            im = wave_sum(im);                                                    \
-            if (lane == 0) {                                                      \
-                lds[wid][2 * (c * kPtTaps + T)] = re;                             \
-                lds[wid][2 * (c * kPtTaps + T) + 1] = im;                         \
-            }                                                                     \
-        }                                                                         \
+            for (int k = 0; k < 3; ++k)
+                row[12 * w + 3 * t + k] = v[t][k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            row[12 * w + k] = mk<float2>(0.f, 0.f);
     }
-    KQ_PT_FOR_TAPS(KQ_TAPG)
-#undef KQ_TAPG
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        reinterpret_cast<float2 *>(bv + lane * kChanStride)[3 * w + k] =
+            valid ? b[((size_t)w * 3 + k) * g.Vh + s] : mk<float2>(0.f, 0.f);
     __syncthreads();
-    if (threadIdx.x < kPtHidden * kPtTaps) {
-        double re = 0.0, im = 0.0;
-        for (int w = 0; w < kNT / kWave; ++w) {
-            re += lds[w][2 * threadIdx.x];
-            im += lds[w][2 * threadIdx.x + 1];
+    const int t = lane & (kPtTaps - 1), c = lane / kPtTaps;
+    double re = 0.0, im = 0.0;
+    for (int i = w * (kSites / 4); i < (w + 1) * (kSites / 4); ++i) {
+        const float2 *v = reinterpret_cast<const float2 *>(tv + i * kTapStride) + 3 * t;
+        const float2 *bb = reinterpret_cast<const float2 *>(bv + i * kChanStride) + 3 * c;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double vx = v[k].x, vy = v[k].y, bx = bb[k].x, by = bb[k].y;
+            re = fmadd(vx, bx, re);
+            re = fmadd(vy, by, re);
+            im = fmadd(vx, by, im);
+            im = fmadd(-vy, bx, im);
         }
-        part[(size_t)blockIdx.x * kPtHidden * kPtTaps + threadIdx.x] = mk<double2>(re, im);
+    }
+    sum[w][lane] = mk<double2>(re, im);
+    __syncthreads();
+    if (w == 0) {
+        double2 o = sum[0][lane];
+#pragma unroll
+        for (int k = 1; k < kNT / kWave; ++k) {
+            o.x += sum[k][lane].x;
+            o.y += sum[k][lane].y;
+        }
+        part[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * J + lane] = o;
     }
 }
 
-// out[j] = sum over blocks b of part[b*stride + j], j = blockIdx.x; fixed summation order
+// out[y*gridDim.x + j] = sum over blocks b of part[(y*nblk + b)*stride + j], j = blockIdx.x,
+// y = blockIdx.y; fixed summation order
 __global__ void __launch_bounds__(kNT) k_reduce_cols(const double2 *part, uint32_t nblk, uint32_t stride,
                                                      double2 *out)
 {
     const int j = blockIdx.x;
+    part += (size_t)blockIdx.y * nblk * stride;
+    out += (size_t)blockIdx.y * gridDim.x;
     __shared__ double lre[kNT], lim[kNT];
     double re = 0.0, im = 0.0;
     for (uint32_t b = threadIdx.x; b < nblk; b += kNT) {
@@ -477,7 +523,7 @@ void pt_unpack_hidden(const kq_v4u *h16, float2 *h, uint32_t Vh, hipStream_t st)
     KQ_HIP_CHECK(hipGetLastError());
 }
 
-uint32_t pt_layer_nblk(uint32_t Vh) { return (Vh + kNT - 1) / kNT; }
+uint32_t pt_layer_nblk(uint32_t Vh) { return dslash_grid(Vh, kSites); }
 
 template <class LF, class LL>
 void pt_forward(const Geom &g, int q, LF fat, LL lng, const PtWeightsBF &w, const float2 *r, float2 *h, float2 *z,
@@ -528,37 +574,29 @@ void pt_backward_hidden(const Geom &g, int q, LF fat, LL lng, const PtWeightsBF 
 }
 
 template <class LF, class LL>
-static void wgrad_pass(const Geom &g, int qo, LF fat, LL lng, const float2 *in, const float2 *b, double2 *res,
-                       hipStream_t st)
-{
-    const unsigned nb = pt_layer_nblk(g.Vh);
-    constexpr int J = kPtHidden * kPtTaps;
-    DevBuf part(sizeof(double2) * nb * J), out(sizeof(double2) * J);
-    hipLaunchKernelGGL((k_pt_wgrad<LF, LL>), dim3(nb), dim3(kNT), 0, st, g, qo, fat, lng, in, b, part.as<double2>());
-    KQ_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_reduce_cols, dim3(J), dim3(kNT), 0, st, part.as<double2>(), nb, (uint32_t)J,
-                       out.as<double2>());
-    KQ_HIP_CHECK(hipGetLastError());
-    KQ_HIP_CHECK(hipMemcpyAsync(res, out.as<void>(), sizeof(double2) * J, hipMemcpyDeviceToHost, st));
-    KQ_HIP_CHECK(hipStreamSynchronize(st));
-}
-
-template <class LF, class LL>
 void pt_weight_grads(const Geom &g, int q, LF fat, LL lng, const float2 *r, const float2 *h, const float2 *gz,
                      const float2 *gh, double *out, hipStream_t st)
 {
     constexpr int J = kPtHidden * kPtTaps;
-    double2 p1[J], p2[J];
     // gW1[c][t] = sum_y <T_t r, gh_c>, y on parity 1-q
-    wgrad_pass<LF, LL>(g, 1 - q, fat, lng, r, gh, p1, st);
     // gW2[c][t] = sum_y <h_c, T_{flip t} g> = conj(sum_y <T_{flip t} g, h_c>)
-    wgrad_pass<LF, LL>(g, 1 - q, fat, lng, gz, h, p2, st);
+    const unsigned nb = pt_layer_nblk(g.Vh);
+    DevBuf part(sizeof(double2) * nb * 2 * J), res(sizeof(double2) * 2 * J);
+    const PtGradArgs p{{r, gz}, {gh, h}};
+    hipLaunchKernelGGL((k_pt_wgrad<LF, LL>), dim3(nb, 2), dim3(kNT), 0, st, g, 1 - q, fat, lng, p, part.as<double2>());
+    KQ_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(k_reduce_cols, dim3(J, 2), dim3(kNT), 0, st, part.as<double2>(), nb, (uint32_t)J,
+                       res.as<double2>());
+    KQ_HIP_CHECK(hipGetLastError());
+    double2 h12[2 * J];
+    KQ_HIP_CHECK(hipMemcpyAsync(h12, res.as<void>(), sizeof(double2) * 2 * J, hipMemcpyDeviceToHost, st));
+    KQ_HIP_CHECK(hipStreamSynchronize(st));
     for (int c = 0; c < kPtHidden; ++c)
         for (int t = 0; t < kPtTaps; ++t) {
             const int j1 = c * kPtTaps + t, j2 = J + c * kPtTaps + t;
-            out[2 * j1] = p1[j1].x;
-            out[2 * j1 + 1] = p1[j1].y;
-            const double2 b = p2[c * kPtTaps + pt_flip_tap(t)];
+            out[2 * j1] = h12[j1].x;
+            out[2 * j1 + 1] = h12[j1].y;
+            const double2 b = h12[J + c * kPtTaps + pt_flip_tap(t)];
             out[2 * j2] = b.x;
             out[2 * j2 + 1] = -b.y;
         }

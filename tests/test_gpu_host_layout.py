@@ -126,3 +126,40 @@ def test_blocks_of_the_mixed_terms(gpu, lat, nrhs, mode):
         assert kq.dslash_batched(src, out, 1, mode, nr, 64) == 0, kq.last_error()
         for r in range(nrhs):
             assert rel_err(out[r], want[r % 3]) <= {2: 1e-5, 3: 3e-3, 4: 5e-4}[mode], r
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("links", ["su3", "u3", "general"])
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
+def test_split_terms_in_solves(gpu, links, mode):
+    """The split terms with the fused epilogue, as the solvers run them, in every link format (SU(3)
+    products, U(3) products and general long links) and blocking: solves on a lattice with a partial
+    last workgroup, every shift to an FP64 residual that the oracle confirms. A wrong term would not
+    converge, or only after many more iterations than the FP64 solve."""
+    kq = gpu
+    lat = (10, 6, 6, 6)
+    fat, lng = _load(kq, lat, 8, u3=links == "u3")
+    if links == "general":
+        rng = np.random.default_rng(8)
+        lng = lng * (1.0 + 0.05 * rng.normal(size=lng.shape))
+        kq.kuqcd_gauge_free()
+        kq.load_gauge_pair(fat, lng, lat)
+    shifts = np.array([0.05, 0.1, 0.3, 0.6, 1.0, 2.0, 3.0, 4.0])
+    given = np.concatenate([shifts[:1], shifts[1:] - shifts[0]])
+    nrhs = 2
+    b = [kq.gen_source(lat, 0, seed=70 + r) for r in range(nrhs)]
+    iters = {}
+    for m, nr in [(1, 1)] + [(mode, n) for n in ([2] if mode == 1 else [1, 2, 3, 4, 8])]:
+        print("case", links, m, nr, flush=True)
+        x = [np.zeros_like(b[0]) for _ in range(nrhs * len(shifts))]
+        p = kq.InvertParam(shifts=np.array([given] * nrhs), tol=1.0, max_iter=400, num_shift=len(shifts))
+        st, rep = kq.solve_batched(x, b, p, kq.default_options(mode=m, rel_tol=1e-10, nr=nr, verbose=0))
+        assert st == 0, kq.last_error()
+        iters[m, nr] = rep[0].iter
+        for r in range(nrhs):
+            for k in range(len(shifts)):
+                v = x[r * len(shifts) + k]
+                res = b[r] - (shifts[k] * v - oracle.mdaggm(fat, lng, v, lat, 0))
+                assert np.linalg.norm(res) <= 1.01e-10 * np.linalg.norm(b[r]), (m, nr, r, k)
+        # the 16-bit fat links leave the base system some more iterations (its refinement does the rest)
+        assert rep[0].iter <= (2 if m == 3 else 1.2) * iters[1, 1] + 5
