@@ -20,13 +20,8 @@
 namespace kq {
 
 struct FcgState {
-    double qz[2];     // <q_prev, z>
-    double pq;        // Re <p, q>
     double pq_prev;   // Re <p, q> of the previous iteration
-    double pr[2];     // <p, r>
     double rr;        // |r|^2
-    double alpha[2];  //
-    double beta[2];   //
     double rr_pause;  // stop (for a reliable update) when rr <= rr_pause
     double rr_stop;   // stop when rr <= rr_stop
     double sigma;     // shift of A
@@ -40,20 +35,22 @@ struct FcgState {
 
 constexpr int kFcgStopPause = 1, kFcgStopConverged = 2, kFcgStopMaxIter = 3;
 
-uint32_t fcg_nblk(size_t n);  // blocks of the vector kernels for n complex entries
+// blocks of the vector kernels for n complex entries: at most 2 per CU, since the updates sum all
+// partials of the kernel before them in every block
+constexpr uint32_t kFcgMaxBlocks = 512;
+uint32_t fcg_nblk(size_t n);
+// doubles of the `fold` scratch below
+constexpr size_t kFcgFold = 128;
 
 // partials of <q, z> (complex) -> part[2*blk], part[2*blk+1]
-void fcg_dot(FcgState *st, const float2 *q, const float2 *z, size_t n, double *part, hipStream_t s);
-// qz = sum(part); beta = first ? 0 : qz / pq_prev
-void fcg_beta(FcgState *st, const double *part, uint32_t nblk, hipStream_t s);
-// p = z - beta p (first: p = z); partials of <p, r>
-void fcg_p_update(FcgState *st, const float2 *z, float2 *p, const float2 *r, size_t n, double *part, hipStream_t s);
-// pq = sum(part_pq) (real, [nblk_pq]); pr = sum(part_pr) (complex); alpha = pr / pq; first = 0
-void fcg_alpha(FcgState *st, const double *part_pq, uint32_t nblk_pq, const double *part_pr, uint32_t nblk,
-               hipStream_t s);
-// x += alpha p; r -= alpha q; partials of |r|^2
-void fcg_xr_update(FcgState *st, float2 *x, float2 *r, const float2 *p, const float2 *q, size_t n, double *part,
-                   hipStream_t s);
+void fcg_dot(const FcgState *st, const float2 *q, const float2 *z, size_t n, double *part, hipStream_t s);
+// beta = first ? 0 : sum(part_qz) (complex, nblk) / pq_prev; p = z - beta p (first: p = z); partials of <p, r>
+void fcg_p_update(const FcgState *st, const double *part_qz, uint32_t nblk, double *fold, const float2 *z, float2 *p,
+                  const float2 *r, size_t n, double *part, hipStream_t s);
+// pq = sum(part_pq) (real, nblk_pq); alpha = sum(part_pr) / pq (part_pr of fcg_p_update); x += alpha p;
+// r -= alpha q; partials of |r|^2; pq_prev = pq, first = 0
+void fcg_xr_update(FcgState *st, const double *part_pq, uint32_t nblk_pq, double *fold, const double *part_pr, float2 *x,
+                   float2 *r, const float2 *p, const float2 *q, size_t n, double *part, hipStream_t s);
 // rr = sum(part); iter += 1; stop on rr_stop, rr_pause or max_iter
 void fcg_check(FcgState *st, const double *part, uint32_t nblk, hipStream_t s);
 

@@ -1,7 +1,10 @@
-// Kernels of the flexible CG: fused vector updates with block partial sums,
-// and single-block scalar kernels that finish the reductions in a fixed order
-// and update the device-resident FcgState.
+// Kernels of the flexible CG: fused vector updates with block partial sums. A vector update that
+// needs a scalar adds the partials of the kernel before it itself, in every workgroup and in the same
+// fixed order (one-workgroup kernels for beta and alpha took 4.3 and 7.6 us of an iteration at
+// 24^4); the check of the residual is a workgroup of its own, since it stops the kernels after it.
 #include "kq_fcg.h"
+
+#include <algorithm>
 
 namespace kq {
 
@@ -41,130 +44,156 @@ __device__ __forceinline__ void block_partial(double a, double b, double *part)
     }
 }
 
-// sum of part[k*stride + off], k < nblk, by one block in a fixed order; valid in thread 0
-__device__ double block_total(const double *part, uint32_t nblk, int stride, int off)
+// sums over k < nblk of the W values part[W*k .. W*k + W), the same in every thread of the workgroup;
+// lds: 4*W doubles used by this call alone
+template <int W> __device__ __forceinline__ void sum_partials(const double *part, uint32_t nblk, double *lds, double *out)
 {
-    __shared__ double l[kNT];
-    double s = 0.0;
+    double s[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+        s[w] = 0.0;
+#pragma unroll 4
     for (uint32_t k = threadIdx.x; k < nblk; k += kNT)
-        s += part[(size_t)k * stride + off];
-    l[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = kNT / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            l[threadIdx.x] += l[threadIdx.x + w];
-        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+            s[w] += part[(size_t)W * k + w];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        s[w] = wave_sum(s[w]);
+        if ((threadIdx.x & (kWave - 1)) == 0)
+            lds[W * (threadIdx.x / kWave) + w] = s[w];
     }
-    const double r = l[0];
     __syncthreads();
-    return r;
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+        out[w] = (lds[w] + lds[W + w]) + (lds[2 * W + w] + lds[3 * W + w]);
 }
 
-__global__ void __launch_bounds__(kNT) k_fcg_dot(FcgState *st, const float2 *q, const float2 *z, size_t n,
+// out[W*b + w] = sum of slice b of the kFoldParts slices of part (large lattices)
+constexpr uint32_t kFoldParts = 64;
+template <int W>
+__global__ void __launch_bounds__(kNT) k_fcg_fold_partials(const FcgState *st, const double *part, uint32_t n,
+                                                           double *out)
+{
+    __shared__ double lds[4 * W];
+    if (halted(st))
+        return;
+    const uint32_t per = (n + kFoldParts - 1) / kFoldParts, i0 = blockIdx.x * per;
+    double t[W];
+    sum_partials<W>(part + (size_t)W * i0, i0 >= n ? 0u : min(per, n - i0), lds, t);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+            out[W * blockIdx.x + w] = t[w];
+}
+
+__global__ void __launch_bounds__(kNT) k_fcg_dot(const FcgState *st, const float2 *q, const float2 *z, size_t n,
                                                  double *part)
 {
     if (halted(st))
         return;
-    const size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
     double re = 0.0, im = 0.0;
-    if (i < n) {
+    for (size_t i = (size_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (size_t)gridDim.x * kNT) {
         const float2 a = q[i], b = z[i];
-        re = (double)a.x * b.x + (double)a.y * b.y;
-        im = (double)a.x * b.y - (double)a.y * b.x;
+        re += (double)a.x * b.x + (double)a.y * b.y;
+        im += (double)a.x * b.y - (double)a.y * b.x;
     }
     block_partial<true>(re, im, part);
 }
 
-__global__ void __launch_bounds__(kNT) k_fcg_beta(FcgState *st, const double *part, uint32_t nblk)
+// beta = <q, z> / <p, q> of the previous iteration (0 on a first one), p = z - beta p, partials of <p, r>
+__global__ void __launch_bounds__(kNT) k_fcg_p_update(const FcgState *st, const double *part_qz, uint32_t nblk,
+                                                      const float2 *z, float2 *p, const float2 *r, size_t n,
+                                                      double *part)
 {
+    __shared__ double lds[8];
     if (halted(st))
         return;
-    const double re = block_total(part, nblk, 2, 0);
-    const double im = block_total(part, nblk, 2, 1);
-    if (threadIdx.x == 0) {
-        st->qz[0] = re;
-        st->qz[1] = im;
-        if (st->first || st->pq_prev == 0.0) {
-            st->beta[0] = 0.0;
-            st->beta[1] = 0.0;
-        } else {
-            st->beta[0] = re / st->pq_prev;
-            st->beta[1] = im / st->pq_prev;
+    size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
+    float2 zi = {}, ri = {}, po = {};
+    // the vectors' loads run while the partials are summed (p is read on a first iteration as well)
+    auto fetch = [&] {
+        if (i < n) {
+            zi = z[i];
+            ri = r[i];
+            po = p[i];
         }
-    }
-}
-
-__global__ void __launch_bounds__(kNT) k_fcg_p_update(FcgState *st, const float2 *z, float2 *p, const float2 *r,
-                                                      size_t n, double *part)
-{
-    if (halted(st))
-        return;
-    const size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
+    };
+    fetch();
+    double qz[2];
+    sum_partials<2>(part_qz, nblk, lds, qz);
+    const bool first = st->first != 0;
+    const double pq = st->pq_prev;
+    const bool none = first || pq == 0.0;
+    const float br = none ? 0.f : (float)(qz[0] / pq), bi = none ? 0.f : (float)(qz[1] / pq);
     double re = 0.0, im = 0.0;
-    if (i < n) {
-        const float br = (float)st->beta[0], bi = (float)st->beta[1];
-        const float2 zi = z[i];
-        float2 pi = mk<float2>(zi.x, zi.y);
-        if (!st->first) {
-            const float2 po = p[i];
+    for (; i < n; i += (size_t)gridDim.x * kNT, fetch()) {
+        float2 pi = zi;
+        if (!first) {
             pi.x -= br * po.x - bi * po.y;
             pi.y -= br * po.y + bi * po.x;
         }
         p[i] = pi;
-        const float2 ri = r[i];
-        re = (double)pi.x * ri.x + (double)pi.y * ri.y;
-        im = (double)pi.x * ri.y - (double)pi.y * ri.x;
+        re += (double)pi.x * ri.x + (double)pi.y * ri.y;
+        im += (double)pi.x * ri.y - (double)pi.y * ri.x;
     }
     block_partial<true>(re, im, part);
 }
 
-__global__ void __launch_bounds__(kNT) k_fcg_alpha(FcgState *st, const double *part_pq, uint32_t nblk_pq,
-                                                   const double *part_pr, uint32_t nblk)
+// alpha = <p, r> / <p, q>, x += alpha p, r -= alpha q, partials of |r|^2. The last workgroup keeps
+// <p, q> for the next beta instead (no other workgroup reads what it writes).
+__global__ void __launch_bounds__(kNT) k_fcg_xr_update(FcgState *st, const double *part_pq, uint32_t nblk_pq,
+                                                       const double *part_pr, uint32_t nblk_pr, float2 *x, float2 *r,
+                                                       const float2 *p, const float2 *q, size_t n, double *part)
 {
+    __shared__ double lpq[4], lpr[8];
     if (halted(st))
         return;
-    const double pq = block_total(part_pq, nblk_pq, 1, 0);
-    const double prr = block_total(part_pr, nblk, 2, 0);
-    const double pri = block_total(part_pr, nblk, 2, 1);
-    if (threadIdx.x == 0) {
-        st->pq = pq;
-        st->pr[0] = prr;
-        st->pr[1] = pri;
-        const bool ok = pq > 0.0;
-        st->alpha[0] = ok ? prr / pq : 0.0;
-        st->alpha[1] = ok ? pri / pq : 0.0;
-        st->pq_prev = pq;
-        st->first = 0;
+    const uint32_t nb = gridDim.x - 1;
+    size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
+    float2 pi = {}, qi = {}, xi = {}, ri = {};
+    auto fetch = [&] {
+        if (i < n) {
+            pi = p[i];
+            qi = q[i];
+            xi = x[i];
+            ri = r[i];
+        }
+    };
+    if (blockIdx.x < nb)
+        fetch();
+    double pq, pr[2];
+    sum_partials<1>(part_pq, nblk_pq, lpq, &pq);
+    if (blockIdx.x == nb) {
+        if (threadIdx.x == 0) {
+            st->pq_prev = pq;
+            st->first = 0;
+        }
+        return;
     }
-}
-
-__global__ void __launch_bounds__(kNT) k_fcg_xr_update(FcgState *st, float2 *x, float2 *r, const float2 *p,
-                                                       const float2 *q, size_t n, double *part)
-{
-    if (halted(st))
-        return;
-    const size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
+    sum_partials<2>(part_pr, nblk_pr, lpr, pr);
+    const bool ok = pq > 0.0;
+    const float ar = ok ? (float)(pr[0] / pq) : 0.f, ai = ok ? (float)(pr[1] / pq) : 0.f;
     double rr = 0.0;
-    if (i < n) {
-        const float ar = (float)st->alpha[0], ai = (float)st->alpha[1];
-        const float2 pi = p[i], qi = q[i];
-        float2 xi = x[i], ri = r[i];
+    for (; i < n; i += (size_t)nb * kNT, fetch()) {
         xi.x += ar * pi.x - ai * pi.y;
         xi.y += ar * pi.y + ai * pi.x;
         ri.x -= ar * qi.x - ai * qi.y;
         ri.y -= ar * qi.y + ai * qi.x;
         x[i] = xi;
         r[i] = ri;
-        rr = (double)ri.x * ri.x + (double)ri.y * ri.y;
+        rr += (double)ri.x * ri.x + (double)ri.y * ri.y;
     }
     block_partial<false>(rr, 0.0, part);
 }
 
 __global__ void __launch_bounds__(kNT) k_fcg_check(FcgState *st, const double *part, uint32_t nblk)
 {
+    __shared__ double lds[4];
     if (halted(st))
         return;
-    const double rr = block_total(part, nblk, 1, 0);
+    double rr;
+    sum_partials<1>(part, nblk, lds, &rr);
     if (threadIdx.x == 0) {
         st->rr = rr;
         st->iter += 1;
@@ -199,15 +228,14 @@ __global__ void k_fcg_fold(double2 *x64, float2 *x32, size_t n)
 __global__ void __launch_bounds__(kNT) k_fcg_residual(const double2 *b, const double2 *ax, double2 *r64,
                                                       float2 *r32, size_t n, double *part)
 {
-    const size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
     double rr = 0.0;
-    if (i < n) {
+    for (size_t i = (size_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (size_t)gridDim.x * kNT) {
         const double2 bi = b[i], ai = ax[i];
         const double2 ri = mk<double2>(bi.x - ai.x, bi.y - ai.y);
         if (r64)
             r64[i] = ri;
         r32[i] = mk<float2>((float)ri.x, (float)ri.y);
-        rr = ri.x * ri.x + ri.y * ri.y;
+        rr += ri.x * ri.x + ri.y * ri.y;
     }
     block_partial<false>(rr, 0.0, part);
 }
@@ -228,7 +256,8 @@ __global__ void k_fcg_to_f32(const double2 *a, const double2 *b, double scale, f
 
 }  // namespace
 
-uint32_t fcg_nblk(size_t n) { return (uint32_t)((n + kNT - 1) / kNT); }
+static uint32_t full_grid(size_t n) { return (uint32_t)((n + kNT - 1) / kNT); }
+uint32_t fcg_nblk(size_t n) { return std::min(full_grid(n), kFcgMaxBlocks); }
 
 #define KQ_FCG_LAUNCH(kernel, grid, ...)                                           \
     do {                                                                           \
@@ -236,27 +265,34 @@ uint32_t fcg_nblk(size_t n) { return (uint32_t)((n + kNT - 1) / kNT); }
         KQ_HIP_CHECK(hipGetLastError());                                           \
     } while (0)
 
-void fcg_dot(FcgState *st, const float2 *q, const float2 *z, size_t n, double *part, hipStream_t s)
+// Above this many partials (64 KB) they are first summed in slices: every workgroup of an update
+// reads all that are left
+constexpr uint32_t kFoldAbove = 8192;
+template <int W>
+static const double *folded(const FcgState *st, const double *part, uint32_t &n, double *fold, hipStream_t s)
+{
+    if ((size_t)W * n <= kFoldAbove)
+        return part;
+    KQ_FCG_LAUNCH(k_fcg_fold_partials<W>, kFoldParts, st, part, n, fold);
+    n = kFoldParts;
+    return fold;
+}
+
+void fcg_dot(const FcgState *st, const float2 *q, const float2 *z, size_t n, double *part, hipStream_t s)
 {
     KQ_FCG_LAUNCH(k_fcg_dot, fcg_nblk(n), st, q, z, n, part);
 }
-void fcg_beta(FcgState *st, const double *part, uint32_t nblk, hipStream_t s)
+void fcg_p_update(const FcgState *st, const double *part_qz, uint32_t nblk, double *fold, const float2 *z, float2 *p,
+                  const float2 *r, size_t n, double *part, hipStream_t s)
 {
-    KQ_FCG_LAUNCH(k_fcg_beta, 1, st, part, nblk);
+    part_qz = folded<2>(st, part_qz, nblk, fold, s);
+    KQ_FCG_LAUNCH(k_fcg_p_update, fcg_nblk(n), st, part_qz, nblk, z, p, r, n, part);
 }
-void fcg_p_update(FcgState *st, const float2 *z, float2 *p, const float2 *r, size_t n, double *part, hipStream_t s)
+void fcg_xr_update(FcgState *st, const double *part_pq, uint32_t nblk_pq, double *fold, const double *part_pr, float2 *x,
+                   float2 *r, const float2 *p, const float2 *q, size_t n, double *part, hipStream_t s)
 {
-    KQ_FCG_LAUNCH(k_fcg_p_update, fcg_nblk(n), st, z, p, r, n, part);
-}
-void fcg_alpha(FcgState *st, const double *part_pq, uint32_t nblk_pq, const double *part_pr, uint32_t nblk,
-               hipStream_t s)
-{
-    KQ_FCG_LAUNCH(k_fcg_alpha, 1, st, part_pq, nblk_pq, part_pr, nblk);
-}
-void fcg_xr_update(FcgState *st, float2 *x, float2 *r, const float2 *p, const float2 *q, size_t n, double *part,
-                   hipStream_t s)
-{
-    KQ_FCG_LAUNCH(k_fcg_xr_update, fcg_nblk(n), st, x, r, p, q, n, part);
+    part_pq = folded<1>(st, part_pq, nblk_pq, fold, s);
+    KQ_FCG_LAUNCH(k_fcg_xr_update, fcg_nblk(n) + 1, st, part_pq, nblk_pq, part_pr, fcg_nblk(n), x, r, p, q, n, part);
 }
 void fcg_check(FcgState *st, const double *part, uint32_t nblk, hipStream_t s)
 {
@@ -265,7 +301,7 @@ void fcg_check(FcgState *st, const double *part, uint32_t nblk, hipStream_t s)
 void fcg_fold(double2 *x64, float2 *x32, size_t n, hipStream_t s)
 {
     if (n)
-        KQ_FCG_LAUNCH(k_fcg_fold, fcg_nblk(n), x64, x32, n);
+        KQ_FCG_LAUNCH(k_fcg_fold, full_grid(n), x64, x32, n);
 }
 void fcg_residual(const double2 *b, const double2 *ax, double2 *r64, float2 *r32, size_t n, double *part,
                   hipStream_t s)
@@ -277,7 +313,7 @@ void fcg_residual(const double2 *b, const double2 *ax, double2 *r64, float2 *r32
 void fcg_to_f32(const double2 *a, const double2 *b, double scale, float2 *out, size_t n, hipStream_t s)
 {
     if (n)
-        KQ_FCG_LAUNCH(k_fcg_to_f32, fcg_nblk(n), a, b, scale, out, n);
+        KQ_FCG_LAUNCH(k_fcg_to_f32, full_grid(n), a, b, scale, out, n);
 }
 
 }  // namespace kq

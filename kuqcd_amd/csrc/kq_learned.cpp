@@ -195,7 +195,8 @@ FcgOut fcg_solve(const Geom &g, int q, AF af, AL al, PF pf, PL pl, LinkD df, Lin
     DevBuf vh16(cfg.learned ? sizeof(kq_v4u) * n3 : 0);
     DevBuf ax64(db), t64(db), r64(hook ? db : 0), xbest(cfg.learned ? db : 0);
     DevBuf part_qz(sizeof(double) * 2 * std::max(nbv, nbl)), part_pr(sizeof(double) * 2 * nbv),
-        part_pq(sizeof(double) * A.max_nblk()), part_rr(sizeof(double) * nbv);
+        part_pq(sizeof(double) * A.max_nblk()), part_rr(sizeof(double) * nbv),
+        fold(sizeof(double) * kFcgFold);
     DevBuf sdev(sizeof(FcgState));
     Pinned<FcgState> sh(1);
     FcgState &H = *sh.get();
@@ -227,18 +228,17 @@ FcgOut fcg_solve(const Geom &g, int q, AF af, AL al, PF pf, PL pl, LinkD df, Lin
         if (net) {
             pt_forward<PF, PL>(g, q, pf, pl, cfg.wf, vr.as<float2>(), nullptr, vz.as<float2>(), st,
                                vq.as<float2>(), part_qz.as<double>(), &S->stop, vh16.as<kq_v4u>());
-            fcg_beta(S, part_qz.as<double>(), nbl, st);
-            fcg_p_update(S, vz.as<float2>(), vp.as<float2>(), vr.as<float2>(), n3, part_pr.as<double>(), st);
+            fcg_p_update(S, part_qz.as<double>(), nbl, fold.as<double>(), vz.as<float2>(), vp.as<float2>(),
+                         vr.as<float2>(), n3, part_pr.as<double>(), st);
         } else {
             fcg_dot(S, vq.as<float2>(), vr.as<float2>(), n3, part_qz.as<double>(), st);
-            fcg_beta(S, part_qz.as<double>(), nbv, st);
-            fcg_p_update(S, vr.as<float2>(), vp.as<float2>(), vr.as<float2>(), n3, part_pr.as<double>(), st);
+            fcg_p_update(S, part_qz.as<double>(), nbv, fold.as<double>(), vr.as<float2>(), vp.as<float2>(),
+                         vr.as<float2>(), n3, part_pr.as<double>(), st);
         }
         const uint32_t nbp = A.apply(vp.as<float2>(), vt.as<float2>(), vq.as<float2>(), &S->sigma, part_pq.as<double>(),
                                      &S->run, st);
-        fcg_alpha(S, part_pq.as<double>(), nbp, part_pr.as<double>(), nbv, st);
-        fcg_xr_update(S, vx.as<float2>(), vr.as<float2>(), vp.as<float2>(), vq.as<float2>(), n3,
-                      part_rr.as<double>(), st);
+        fcg_xr_update(S, part_pq.as<double>(), nbp, fold.as<double>(), part_pr.as<double>(), vx.as<float2>(),
+                      vr.as<float2>(), vp.as<float2>(), vq.as<float2>(), n3, part_rr.as<double>(), st);
         fcg_check(S, part_rr.as<double>(), nbv, st);
     };
     hipGraphExec_t graphs[2] = {nullptr, nullptr};
