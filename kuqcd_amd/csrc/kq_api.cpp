@@ -46,6 +46,16 @@ void ensure_device()
     c.device_ready = true;
 }
 
+Pinned<double> &host_scratch()
+{
+    Context &c = ctx();
+    if (!c.scratch_event)
+        KQ_HIP_CHECK(hipEventCreateWithFlags(&c.scratch_event, hipEventDisableTiming));
+    if (!c.scratch)
+        c.scratch = new Pinned<double>(kScratchDoubles);
+    return *c.scratch;
+}
+
 void log_info(const char *fmt, ...)
 {
     if (ctx().verbosity <= 0)
@@ -527,6 +537,11 @@ void kq_end(void)
         }
         learned_release();
         DevPool::get().trim();
+        delete c.scratch;
+        c.scratch = nullptr;
+        if (c.scratch_event)
+            (void)hipEventDestroy(c.scratch_event);
+        c.scratch_event = nullptr;
     } catch (...) {
     }
 }

@@ -57,6 +57,10 @@ struct Context {
     hipStream_t stream = nullptr;
     // second stream (default priority) for device-to-host copies that overlap the solver's kernels
     hipStream_t copy_stream = nullptr;
+    // kScratchDoubles of pinned host memory for scalars read back from the device, and an event for
+    // those that other work is queued after; made by host_scratch(), given back by kq_end
+    Pinned<double> *scratch = nullptr;
+    hipEvent_t scratch_event = nullptr;
     int grid[4] = {1, 1, 1, 1};
     // slot order = reference dispatch order (kuqcd.cpp:415-435):
     // 0 float/BATCH, 1 double/BATCH, 2 float/NORMAL, 3 double/NORMAL
@@ -76,6 +80,8 @@ struct Context {
 
 Context &ctx();
 void ensure_device();
+constexpr size_t kScratchDoubles = 2048;
+Pinned<double> &host_scratch();
 inline int slot_index(int order, int prec) { return (order == KUQCD_BATCH_ORDER ? 0 : 2) + (prec == KUQCD_DOUBLE ? 1 : 0); }
 // first slot with both fat and long loaded, in dispatch order; -1 if none
 int active_slot();

@@ -93,18 +93,47 @@ int slot_or_throw(bool need_double = true)
     return slot;
 }
 
+// Link norms of a slot in two halves: begin() queues the sums, finish() waits for them alone, so that
+// what does not need the norms can be queued in between.
+constexpr size_t kNormParts = 2 * (size_t)kSumsqParts;
+struct NormJob {
+    size_t n[2] = {0, 0};
+    Geom g;
+    void begin(int slot, double *part)  // part: kNormParts doubles of device memory
+    {
+        Context &c = ctx();
+        g = slot_geom(slot);
+        const GaugeSlot *s[2] = {&c.fat[slot], &c.lng[slot]};
+        const double *x[2];
+        for (int h = 0; h < 2; ++h) {
+            x[h] = s[h]->soa.as<double>();
+            n[h] = s[h]->soa.bytes() / sizeof(double);
+        }
+        static_assert(kNormParts <= kScratchDoubles && 2 * kPtSums <= kScratchDoubles, "host scratch too small");
+        vd_sumsq_partials(x, n, 2, part, c.stream);
+        copy_words(part, host_scratch().dev(), sizeof(double) * kNormParts, c.stream);
+        KQ_HIP_CHECK(hipEventRecord(c.scratch_event, c.stream));
+    }
+    PtNorms finish() const
+    {
+        Context &c = ctx();
+        KQ_HIP_CHECK(hipEventSynchronize(c.scratch_event));
+        PtNorms nu;
+        for (int h = 0; h < 2; ++h) {
+            const double ss = vd_sumsq_total(host_scratch().get() + (size_t)h * kSumsqParts, n[h]);
+            const double rows = 24.0 * g.Vh;  // 8 Vh links of 3 rows
+            nu.nu[h] = ss > 0.0 ? std::sqrt(ss / rows) : 1.0;
+        }
+        return nu;
+    }
+};
+
 PtNorms slot_norms(int slot)
 {
-    Context &c = ctx();
-    const Geom g = slot_geom(slot);
-    PtNorms nu;
-    const GaugeSlot *s[2] = {&c.fat[slot], &c.lng[slot]};
-    for (int h = 0; h < 2; ++h) {
-        const double ss = vd_sumsq(s[h]->soa.as<double>(), s[h]->soa.bytes() / sizeof(double), c.stream);
-        const double rows = 24.0 * g.Vh;  // 8 Vh links of 3 rows
-        nu.nu[h] = ss > 0.0 ? std::sqrt(ss / rows) : 1.0;
-    }
-    return nu;
+    DevBuf part(sizeof(double) * kNormParts);
+    NormJob j;
+    j.begin(slot, part.as<double>());
+    return j.finish();
 }
 
 template <class Fn> void with_format(int slot, int mode, Fn &&fn) { (void)with_mixed_links(slot, mode, fn); }
@@ -341,27 +370,41 @@ FcgOut fcg_solve(const Geom &g, int q, AF af, AL al, PF pf, PL pl, LinkD df, Lin
 // ---------------------------------------------------------------- loss and gradient
 constexpr int kTrainNT = 128;  // hopping-term block size of the training kernels
 
+// Device scratch of a loss and gradient, one allocation: taking a buffer from the pool while work is
+// queued waits for that work.
 struct Work {
-    DevBuf h, z, az, t, d, gz, gh, sig, part;
+    DevBuf buf;
+    float2 *h = nullptr, *z, *az, *t, *d, *gz, *gh, *r, *e, *ae;
+    double *sigma, *part, *norms;
+    double2 *gpart, *lpart, *sums;
     size_t n3 = 0;
-    int nt = 0;
-    void ensure(uint32_t Vh, int nt_)
+    void ensure(uint32_t Vh)
     {
         const size_t n = (size_t)3 * Vh;
-        if (n <= n3 && nt_ == nt)
+        if (n <= n3)
             return;
         n3 = n;
-        nt = nt_;
+        size_t total = 0;
+        auto add = [&](size_t bytes) {
+            const size_t o = total;
+            total += (bytes + 255) / 256 * 256;
+            return o;
+        };
         const size_t fb = sizeof(float2) * n;
-        h.alloc(4 * fb);
-        z.alloc(fb);
-        az.alloc(fb);
-        t.alloc(fb);
-        d.alloc(fb);
-        gz.alloc(fb);
-        gh.alloc(4 * fb);
-        sig.alloc(sizeof(double));
-        part.alloc(sizeof(double) * dslash_nblk(Vh, kMinDslashNT));
+        const size_t oh = add(4 * fb), oz = add(fb), oaz = add(fb), ot = add(fb), od = add(fb), ogz = add(fb),
+                     ogh = add(4 * fb), orr = add(fb), oe = add(fb), oae = add(fb), os = add(sizeof(double)),
+                     op = add(sizeof(double) * dslash_nblk(Vh, kMinDslashNT)),
+                     on = add(sizeof(double) * kNormParts), og = add(sizeof(double2) * pt_grad_parts(Vh)),
+                     ol = add(sizeof(double2) * 2 * loss_nblk(n)), osum = add(sizeof(double2) * kPtSums);
+        buf.alloc(total);
+        char *p = buf.as<char>();
+        auto f2 = [&](size_t o) { return reinterpret_cast<float2 *>(p + o); };
+        auto d1 = [&](size_t o) { return reinterpret_cast<double *>(p + o); };
+        auto d2 = [&](size_t o) { return reinterpret_cast<double2 *>(p + o); };
+        h = f2(oh), z = f2(oz), az = f2(oaz), t = f2(ot), d = f2(od), gz = f2(ogz), gh = f2(ogh);
+        r = f2(orr), e = f2(oe), ae = f2(oae);
+        sigma = d1(os), part = d1(op), norms = d1(on);
+        gpart = d2(og), lpart = d2(ol), sums = d2(osum);
     }
 };
 
@@ -369,23 +412,33 @@ struct Work {
 // the error of the correction z in the A^2 norm (for a solver pair, r = A e and L is
 // the residual one application of M leaves). grad (optional, 2*kPtParams doubles):
 // dL/dconj(w) of the master weights, from dL/dconj(z) = A (A z - A e) / |A e|^2.
+// W has the lattice's size and the shift of A in W.sigma. Everything is queued without a wait and the
+// sums come back in one transfer (two reductions to the host in between left the GPU idle for 60
+// of 334 us at 16^4).
 template <class LF, class LL>
-double sample_loss(const Geom &g, int q, LF fat, LL lng, const PtNorms &nu, const PtWeights &w, double sigma,
-                   const float2 *r, const float2 *ae, Work &W, int nt, double *grad, hipStream_t st)
+double sample_loss(const Geom &g, int q, LF fat, LL lng, const PtNorms &nu, const PtWeights &w, const float2 *r,
+                   const float2 *ae, Work &W, int nt, double *grad, hipStream_t st)
 {
-    W.ensure(g.Vh, nt);
     const size_t n3 = (size_t)3 * g.Vh;
-    pt_forward<LF, LL>(g, q, fat, lng, pt_pack(w, nu), r, W.h.as<float2>(), W.z.as<float2>(), st);
-    KQ_HIP_CHECK(hipMemcpyAsync(W.sig.as<void>(), &sigma, sizeof(double), hipMemcpyHostToDevice, st));
+    const uint32_t nl = loss_nblk(n3);
+    double2 *part_rg = W.lpart, *part_loss = W.lpart + nl;
+    pt_forward<LF, LL>(g, q, fat, lng, pt_pack(w, nu), r, W.h, W.z, st);
     const OpA<LF, LL, float> A{g, q, fat, lng, nt};
-    A.apply(W.z.as<float2>(), W.t.as<float2>(), W.az.as<float2>(), W.sig.as<double>(), W.part.as<double>(), nullptr,
-            st);
-    vf_lincomb(W.d.as<float2>(), W.az.as<float2>(), mk<float2>(1.f, 0.f), ae, mk<float2>(-1.f, 0.f), n3, st);
-    const float2 *xs[2] = {W.d.as<float2>(), ae};
-    const float2 *ys[2] = {W.d.as<float2>(), ae};
-    double2 dd[2];
-    vf_dots(xs, ys, 2, n3, dd, st);
-    const double num = dd[0].x, den = dd[1].x;
+    A.apply(W.z, W.t, W.az, W.sigma, W.part, nullptr, st);
+    loss_residual(W.az, ae, W.d, n3, part_loss, st);
+    if (grad) {
+        A.apply(W.d, W.t, W.gz, W.sigma, W.part, nullptr, st);
+        loss_scale(part_loss, W.gz, r, n3, part_rg, st);
+        pt_backward_hidden<LF, LL>(g, q, fat, lng, pt_pack_backward(w, nu), W.gz, W.gh, st);
+        pt_weight_grads<LF, LL>(g, q, fat, lng, r, W.h, W.gz, W.gh, W.gpart, st);
+        pt_reduce(W.gpart, W.lpart, g.Vh, n3, W.sums, st);
+    } else {
+        pt_reduce(nullptr, W.lpart, 0, n3, W.sums, st);
+    }
+    copy_words(W.sums, host_scratch().dev(), sizeof(double2) * kPtSums, st);
+    KQ_HIP_CHECK(hipStreamSynchronize(st));
+    const double2 *sums = reinterpret_cast<const double2 *>(host_scratch().get());
+    const double num = sums[kPtSumLoss].x, den = sums[kPtSumLoss].y;
     if (grad)
         std::fill(grad, grad + 2 * kPtParams, 0.0);
     if (!(den > 0.0))
@@ -393,13 +446,7 @@ double sample_loss(const Geom &g, int q, LF fat, LL lng, const PtNorms &nu, cons
     const double loss = num / den;
     if (!grad)
         return loss;
-    A.apply(W.d.as<float2>(), W.t.as<float2>(), W.gz.as<float2>(), W.sig.as<double>(), W.part.as<double>(), nullptr,
-            st);
-    const float inv = (float)(1.0 / den);
-    vf_lincomb(W.gz.as<float2>(), W.gz.as<float2>(), mk<float2>(inv, 0.f), W.gz.as<float2>(), mk<float2>(0.f, 0.f),
-               n3, st);
-    pt_backward_hidden<LF, LL>(g, q, fat, lng, pt_pack_backward(w, nu), W.gz.as<float2>(), W.gh.as<float2>(), st);
-    pt_weight_grads<LF, LL>(g, q, fat, lng, r, W.h.as<float2>(), W.gz.as<float2>(), W.gh.as<float2>(), grad, st);
+    pt_unpack_grads(sums, grad);
     // w_eff = w / nu_hop for the tap weights
     for (int l = 0; l < 2; ++l)
         for (int c = 0; c < kPtHidden; ++c)
@@ -416,8 +463,10 @@ double train_sample_loss(const TrainSample &s, const PtWeights &w, Work &W, doub
 {
     const TrainGauge &G = *learned().gauges[s.gauge];
     const LinkF fat = as_linkF(G.fat, G.g.Vh), lng = as_linkF(G.lng, G.g.Vh);
-    return sample_loss<LinkF, LinkF>(G.g, s.parity, fat, lng, G.nu, w, s.sigma, s.r.as<float2>(), s.ae.as<float2>(),
-                                     W, kTrainNT, grad, st);
+    W.ensure(G.g.Vh);
+    vd_set(W.sigma, s.sigma, st);
+    return sample_loss<LinkF, LinkF>(G.g, s.parity, fat, lng, G.nu, w, s.r.as<float2>(), s.ae.as<float2>(), W,
+                                     kTrainNT, grad, st);
 }
 
 double mean_loss(const PtWeights &w, Work &W, hipStream_t st)
@@ -644,7 +693,7 @@ static KuQCDStatus ptnet_forward(const KqPtWeights *w, int parity, int link_form
         const PtWeightsBF wf = pt_pack(from_abi(*w), slot_norms(slot));
         DevBuf vr(sizeof(float2) * n3), vz(sizeof(float2) * n3), vh(sizeof(float2) * 4 * n3), stage;
         DevBuf vh16(hidden16 ? sizeof(kq_v4u) * n3 : 0);
-        upload_vec<double, float>(r, Vec<float>{vr.as<float2>(), g.Vh, n3}, 0, stage, c.stream);
+        upload_vec<double, float>(r, Vec<float>{vr.as<float2>(), g.Vh, n3}, 0, stage, c.stream, false);
         with_format(slot, link_format, [&](auto fat, auto lng) {
             pt_forward(g, parity, fat, lng, wf, vr.as<float2>(), hidden16 ? nullptr : vh.as<float2>(),
                        vz.as<float2>(), c.stream, nullptr, nullptr, nullptr, hidden16 ? vh16.as<kq_v4u>() : nullptr);
@@ -686,15 +735,20 @@ KuQCDStatus kq_ptnet_loss_grad(const KqPtWeights *w, int parity, double sigma, c
         const int slot = slot_or_throw();
         const Geom g = slot_geom(slot);
         const size_t n3 = (size_t)3 * g.Vh;
-        DevBuf vr(sizeof(float2) * n3), ve(sizeof(float2) * n3), vae(sizeof(float2) * n3), stage;
-        upload_vec<double, float>(r, Vec<float>{vr.as<float2>(), g.Vh, n3}, 0, stage, c.stream);
-        upload_vec<double, float>(e, Vec<float>{ve.as<float2>(), g.Vh, n3}, 0, stage, c.stream);
+        Work W;
+        W.ensure(g.Vh);
+        DevBuf stage;
         DerivedFormats &d = derived(slot, true, false);
         const LinkF fat = as_linkF(d.fat_f, g.Vh), lng = as_linkF(d.lng_f, g.Vh);
-        apply_a_f32(g, parity, fat, lng, sigma, ve.as<float2>(), vae.as<float2>(), kTrainNT, c.stream);
-        Work W;
-        *loss = sample_loss<LinkF, LinkF>(g, parity, fat, lng, slot_norms(slot), from_abi(*w), sigma, vr.as<float2>(),
-                                          vae.as<float2>(), W, kTrainNT, grad, c.stream);
+        NormJob norms;
+        norms.begin(slot, W.norms);
+        vd_set(W.sigma, sigma, c.stream);
+        upload_vec<double, float>(e, Vec<float>{W.e, g.Vh, n3}, 0, stage, c.stream, false);
+        upload_vec<double, float>(r, Vec<float>{W.r, g.Vh, n3}, 0, stage, c.stream, false);
+        const OpA<LinkF, LinkF, float> A{g, parity, fat, lng, kTrainNT};
+        A.apply(W.e, W.t, W.ae, W.sigma, W.part, nullptr, c.stream);
+        *loss = sample_loss<LinkF, LinkF>(g, parity, fat, lng, norms.finish(), from_abi(*w), W.r, W.ae, W, kTrainNT,
+                                          grad, c.stream);
         return KUQCD_SUCCESS;
     });
 }

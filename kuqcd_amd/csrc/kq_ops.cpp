@@ -28,7 +28,7 @@ static void apply_host(LF fat, LL lng, const Geom &g, int nrhs, const void *src,
 {
     Context &c = ctx();
     const size_t n3 = (size_t)3 * g.Vh, bytes = sizeof(c2_t<R>) * n3 * (size_t)nrhs;
-    const auto usable = [](const void *p) { return (uintptr_t)p % sizeof(R) == 0 && on_this_device(p); };
+    const auto usable = [&](const void *p) { return in_place(p, bytes, sizeof(R)); };
     const bool put_back = !usable(dst);
     DevBuf s, d, t;
     if (overlap(src, dst, bytes) || !usable(src)) {

@@ -80,10 +80,24 @@ void pt_backward_hidden(const Geom &g, int q, LF fat, LL lng, const PtWeightsBF 
                         hipStream_t st);
 // Gradients with respect to the conjugate effective weights for one sample, in FP64:
 //   gW1[c][t] = sum_y <T_t r, gh_c>,  gW2[c][t] = sum_y <h_c, T_t^+ g>,  gW0 = sum_x <r, g>
-// out[2*j], out[2*j+1] = re, im of parameter j (order w1, w2, w0)
+// as block partials of gW1 and gW2 (pt_grad_parts entries) and, from loss_scale, of gW0
 template <class LF, class LL>
 void pt_weight_grads(const Geom &g, int q, LF fat, LL lng, const float2 *r, const float2 *h, const float2 *gz,
-                     const float2 *gh, double *out, hipStream_t st);
+                     const float2 *gh, double2 *part, hipStream_t st);
+size_t pt_grad_parts(uint32_t Vh);
+constexpr int kJ = kPtHidden * kPtTaps;
+// sums of a loss and gradient: kJ of gW1, kJ of gW2, then <r, g> and (|A z - A e|^2, |A e|^2)
+constexpr int kPtSumRG = 2 * kJ, kPtSumLoss = 2 * kJ + 1, kPtSums = 2 * kJ + 2;
+// out (device, kPtSums; the first 2*kJ zero if grad_part is null) from the partials of pt_weight_grads and the loss_nblk(n) partials each of
+// loss_scale and loss_residual, which stand one after the other in loss_part
+void pt_reduce(const double2 *grad_part, const double2 *loss_part, uint32_t Vh, size_t n, double2 *out,
+               hipStream_t st);
+// out[2*j], out[2*j+1] = re, im of parameter j (order w1, w2, w0) from the kPtSums sums (host)
+void pt_unpack_grads(const double2 *sums, double *out);
+// d = az - ae, partials (|d|^2, |ae|^2); g /= sum |ae|^2, partials of <r, g>
+uint32_t loss_nblk(size_t n);
+void loss_residual(const float2 *az, const float2 *ae, float2 *d, size_t n, double2 *part, hipStream_t st);
+void loss_scale(const double2 *part_loss, float2 *g, const float2 *r, size_t n, double2 *part, hipStream_t st);
 uint32_t pt_layer_nblk(uint32_t Vh);
 
 // ---- FP32 vector helpers (n complex entries)
@@ -94,5 +108,11 @@ void vf_lincomb(float2 *y, const float2 *x1, float2 a1, const float2 *x2, float2
 void vf_dots(const float2 *const *xs, const float2 *const *ys, int ndot, size_t n, double2 *out, hipStream_t st);
 // sum of squares of n doubles (host result)
 double vd_sumsq(const double *x, size_t n, hipStream_t st);
+// the same of up to two arrays in one launch, as partials: part[y*kSumsqParts ..], to be added in order
+// by vd_sumsq_total once they are on the host
+constexpr uint32_t kSumsqParts = 1024;
+void vd_sumsq_partials(const double *const *x, const size_t *n, int count, double *part, hipStream_t st);
+double vd_sumsq_total(const double *part, size_t n);
+void vd_set(double *p, double v, hipStream_t st);  // *p = v (device)
 
 }  // namespace kq

@@ -342,7 +342,7 @@ constexpr int kTapStride = 6 * kPtTaps + 2, kChanStride = 6 * kPtHidden + 2;
 template <class LF, class LL>
 __global__ void __launch_bounds__(kNT) k_pt_wgrad(Geom g, int qo, LF fat, LL lng, const PtGradArgs p, double2 *part)
 {
-    constexpr int J = kPtHidden * kPtTaps;
+    constexpr int J = kJ;
     static_assert(J == kWave && kPtHidden == kNT / kWave, "one (c, t) per lane, one channel per wave");
     __shared__ __align__(8) float tv[kSites * kTapStride];
     __shared__ __align__(8) float bv[kSites * kChanStride];
@@ -398,13 +398,23 @@ __global__ void __launch_bounds__(kNT) k_pt_wgrad(Geom g, int qo, LF fat, LL lng
 }
 
 // out[y*gridDim.x + j] = sum over blocks b of part[(y*nblk + b)*stride + j], j = blockIdx.x,
-// y = blockIdx.y; fixed summation order
+// y = blockIdx.y < 2; fixed summation order. For y = 2, j < 2: the sums over the nblk2 entries of
+// part2 + j*nblk2.
 __global__ void __launch_bounds__(kNT) k_reduce_cols(const double2 *part, uint32_t nblk, uint32_t stride,
-                                                     double2 *out)
+                                                     double2 *out, const double2 *part2, uint32_t nblk2)
 {
-    const int j = blockIdx.x;
-    part += (size_t)blockIdx.y * nblk * stride;
-    out += (size_t)blockIdx.y * gridDim.x;
+    int j = blockIdx.x;
+    out += (size_t)blockIdx.y * gridDim.x + j;
+    if (blockIdx.y == 2) {
+        if (j > 1)
+            return;
+        part = part2 + (size_t)j * nblk2;
+        nblk = nblk2;
+        stride = 1;
+        j = 0;
+    } else {
+        part += (size_t)blockIdx.y * nblk * stride;
+    }
     __shared__ double lre[kNT], lim[kNT];
     double re = 0.0, im = 0.0;
     for (uint32_t b = threadIdx.x; b < nblk; b += kNT) {
@@ -423,7 +433,7 @@ __global__ void __launch_bounds__(kNT) k_reduce_cols(const double2 *part, uint32
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        out[j] = mk<double2>(lre[0], lim[0]);
+        *out = mk<double2>(lre[0], lim[0]);
 }
 
 __global__ void k_vf_axpy(float2 *y, const float2 *x, float2 a, size_t n)
@@ -480,11 +490,23 @@ __global__ void __launch_bounds__(kNT) k_vf_dots(DotSet d, int nd, size_t n, dou
     }
 }
 
-__global__ void __launch_bounds__(kNT) k_vd_sumsq(const double *x, size_t n, double *part)
+struct SumsqSet {
+    const double *x[2];
+    size_t n[2];
+    uint32_t nb[2];
+};
+
+// part[y*kSumsqParts + blk] = block partial of |x_y|^2, y = blockIdx.y
+__global__ void __launch_bounds__(kNT) k_vd_sumsq(SumsqSet a, double *part)
 {
     __shared__ double l[kNT / kWave];
+    const int y = blockIdx.y;
+    const double *x = a.x[y];
+    const uint32_t nb = a.nb[y];
+    if (blockIdx.x >= nb)
+        return;
     double acc = 0.0;
-    for (size_t i = (size_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (size_t)gridDim.x * kNT)
+    for (size_t i = (size_t)blockIdx.x * kNT + threadIdx.x; i < a.n[y]; i += (size_t)nb * kNT)
         acc += x[i] * x[i];
     acc = wave_sum(acc);
     if ((threadIdx.x & (kWave - 1)) == 0)
@@ -494,8 +516,73 @@ __global__ void __launch_bounds__(kNT) k_vd_sumsq(const double *x, size_t n, dou
         double s = 0.0;
         for (int w = 0; w < kNT / kWave; ++w)
             s += l[w];
-        part[blockIdx.x] = s;
+        part[(size_t)y * kSumsqParts + blockIdx.x] = s;
     }
+}
+
+__global__ void k_vd_set(double *p, double v) { *p = v; }
+
+// block sum of (a, b), valid in thread 0
+__device__ __forceinline__ double2 block_sum2(double a, double b)
+{
+    __shared__ double la[kNT / kWave], lb[kNT / kWave];
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        la[threadIdx.x / kWave] = a;
+        lb[threadIdx.x / kWave] = b;
+    }
+    __syncthreads();
+    double2 o = mk<double2>(0.0, 0.0);
+    for (int w = 0; w < kNT / kWave; ++w) {
+        o.x += la[w];
+        o.y += lb[w];
+    }
+    return o;
+}
+
+// d = az - ae; part[blk] = (|d|^2, |ae|^2)
+__global__ void __launch_bounds__(kNT) k_loss_residual(const float2 *az, const float2 *ae, float2 *d, size_t n,
+                                                       double2 *part)
+{
+    double dd = 0.0, aa = 0.0;
+    for (size_t i = (size_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (size_t)gridDim.x * kNT) {
+        const float2 p = az[i], q = ae[i], o = mk<float2>(p.x - q.x, p.y - q.y);
+        d[i] = o;
+        dd += (double)o.x * o.x + (double)o.y * o.y;
+        aa += (double)q.x * q.x + (double)q.y * q.y;
+    }
+    const double2 t = block_sum2(dd, aa);
+    if (threadIdx.x == 0)
+        part[blockIdx.x] = t;
+}
+
+// g = g / |ae|^2 with |ae|^2 the sum over the nblk partials of k_loss_residual, added here by every
+// block in the same order; part[blk] = <r, g>. The host sees |ae|^2 after the gradient and drops
+// the gradient if it is not positive.
+__global__ void __launch_bounds__(kNT) k_loss_scale(const double2 *part_loss, uint32_t nblk, float2 *g,
+                                                    const float2 *r, size_t n, double2 *part)
+{
+    __shared__ double l[kNT / kWave];
+    double den = 0.0;
+    for (uint32_t k = threadIdx.x; k < nblk; k += kNT)
+        den += part_loss[k].y;
+    den = wave_sum(den);
+    if ((threadIdx.x & (kWave - 1)) == 0)
+        l[threadIdx.x / kWave] = den;
+    __syncthreads();
+    den = (l[0] + l[1]) + (l[2] + l[3]);
+    const float inv = den > 0.0 ? (float)(1.0 / den) : 0.f;
+    double re = 0.0, im = 0.0;
+    for (size_t i = (size_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (size_t)gridDim.x * kNT) {
+        const float2 o = mk<float2>(inv * g[i].x, inv * g[i].y), a = r[i];
+        g[i] = o;
+        re += (double)a.x * o.x + (double)a.y * o.y;
+        im += (double)a.x * o.y - (double)a.y * o.x;
+    }
+    const double2 t = block_sum2(re, im);
+    if (threadIdx.x == 0)
+        part[blockIdx.x] = t;
 }
 
 __global__ void __launch_bounds__(kNT) k_unpack_hidden(const kq_v4u *h16, float2 *h, uint32_t Vh)
@@ -575,38 +662,56 @@ void pt_backward_hidden(const Geom &g, int q, LF fat, LL lng, const PtWeightsBF 
 
 template <class LF, class LL>
 void pt_weight_grads(const Geom &g, int q, LF fat, LL lng, const float2 *r, const float2 *h, const float2 *gz,
-                     const float2 *gh, double *out, hipStream_t st)
+                     const float2 *gh, double2 *part, hipStream_t st)
 {
-    constexpr int J = kPtHidden * kPtTaps;
+    if (g.Vh == 0)
+        return;
     // gW1[c][t] = sum_y <T_t r, gh_c>, y on parity 1-q
     // gW2[c][t] = sum_y <h_c, T_{flip t} g> = conj(sum_y <T_{flip t} g, h_c>)
-    const unsigned nb = pt_layer_nblk(g.Vh);
-    DevBuf part(sizeof(double2) * nb * 2 * J), res(sizeof(double2) * 2 * J);
     const PtGradArgs p{{r, gz}, {gh, h}};
-    hipLaunchKernelGGL((k_pt_wgrad<LF, LL>), dim3(nb, 2), dim3(kNT), 0, st, g, 1 - q, fat, lng, p, part.as<double2>());
+    hipLaunchKernelGGL((k_pt_wgrad<LF, LL>), dim3(pt_layer_nblk(g.Vh), 2), dim3(kNT), 0, st, g, 1 - q, fat, lng, p,
+                       part);
     KQ_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_reduce_cols, dim3(J, 2), dim3(kNT), 0, st, part.as<double2>(), nb, (uint32_t)J,
-                       res.as<double2>());
+}
+
+size_t pt_grad_parts(uint32_t Vh) { return (size_t)pt_layer_nblk(Vh) * 2 * kJ; }
+
+void pt_reduce(const double2 *grad_part, const double2 *loss_part, uint32_t Vh, size_t n, double2 *out,
+               hipStream_t st)
+{
+    hipLaunchKernelGGL(k_reduce_cols, dim3(kJ, 3), dim3(kNT), 0, st, grad_part, grad_part ? pt_layer_nblk(Vh) : 0u,
+                       (uint32_t)kJ, out, loss_part, loss_nblk(n));
     KQ_HIP_CHECK(hipGetLastError());
-    double2 h12[2 * J];
-    KQ_HIP_CHECK(hipMemcpyAsync(h12, res.as<void>(), sizeof(double2) * 2 * J, hipMemcpyDeviceToHost, st));
-    KQ_HIP_CHECK(hipStreamSynchronize(st));
+}
+
+void pt_unpack_grads(const double2 *sums, double *out)
+{
     for (int c = 0; c < kPtHidden; ++c)
         for (int t = 0; t < kPtTaps; ++t) {
-            const int j1 = c * kPtTaps + t, j2 = J + c * kPtTaps + t;
-            out[2 * j1] = h12[j1].x;
-            out[2 * j1 + 1] = h12[j1].y;
-            const double2 b = h12[J + c * kPtTaps + pt_flip_tap(t)];
+            const int j1 = c * kPtTaps + t, j2 = kJ + c * kPtTaps + t;
+            out[2 * j1] = sums[j1].x;
+            out[2 * j1 + 1] = sums[j1].y;
+            const double2 b = sums[kJ + c * kPtTaps + pt_flip_tap(t)];
             out[2 * j2] = b.x;
             out[2 * j2 + 1] = -b.y;
         }
     // gW0 = sum_x <r, g>
-    double2 d0;
-    const float2 *xs[1] = {r};
-    const float2 *ys[1] = {gz};
-    vf_dots(xs, ys, 1, (size_t)3 * g.Vh, &d0, st);
-    out[4 * J] = d0.x;
-    out[4 * J + 1] = d0.y;
+    out[4 * kJ] = sums[kPtSumRG].x;
+    out[4 * kJ + 1] = sums[kPtSumRG].y;
+}
+
+uint32_t loss_nblk(size_t n) { return (uint32_t)std::min<size_t>(512, grid_of(n)); }
+
+void loss_residual(const float2 *az, const float2 *ae, float2 *d, size_t n, double2 *part, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_loss_residual, dim3(loss_nblk(n)), dim3(kNT), 0, st, az, ae, d, n, part);
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
+void loss_scale(const double2 *part_loss, float2 *g, const float2 *r, size_t n, double2 *part, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_loss_scale, dim3(loss_nblk(n)), dim3(kNT), 0, st, part_loss, loss_nblk(n), g, r, n, part);
+    KQ_HIP_CHECK(hipGetLastError());
 }
 
 // ---------------------------------------------------------------- weights
@@ -718,28 +823,55 @@ void vf_dots(const float2 *const *xs, const float2 *const *ys, int ndot, size_t 
     KQ_HIP_CHECK(hipGetLastError());
     for (int k = 0; k < ndot; ++k) {
         hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(kNT), 0, st, part.as<double2>() + (size_t)k * nb, nb, 1u,
-                           res.as<double2>() + k);
+                           res.as<double2>() + k, nullptr, 0u);
         KQ_HIP_CHECK(hipGetLastError());
     }
     KQ_HIP_CHECK(hipMemcpyAsync(out, res.as<void>(), sizeof(double2) * ndot, hipMemcpyDeviceToHost, st));
     KQ_HIP_CHECK(hipStreamSynchronize(st));
 }
 
+static uint32_t sumsq_nblk(size_t n) { return (uint32_t)std::min<size_t>(kSumsqParts, grid_of(n)); }
+
+void vd_sumsq_partials(const double *const *x, const size_t *n, int count, double *part, hipStream_t st)
+{
+    SumsqSet a{};
+    uint32_t nb = 0;
+    for (int y = 0; y < count; ++y) {
+        a.x[y] = x[y];
+        a.n[y] = n[y];
+        a.nb[y] = sumsq_nblk(n[y]);
+        nb = std::max(nb, a.nb[y]);
+    }
+    if (nb == 0)
+        return;
+    hipLaunchKernelGGL(k_vd_sumsq, dim3(nb, count), dim3(kNT), 0, st, a, part);
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
+double vd_sumsq_total(const double *part, size_t n)
+{
+    double s = 0.0;
+    for (uint32_t k = 0; k < sumsq_nblk(n); ++k)
+        s += part[k];
+    return s;
+}
+
+void vd_set(double *p, double v, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_vd_set, dim3(1), dim3(1), 0, st, p, v);
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
 double vd_sumsq(const double *x, size_t n, hipStream_t st)
 {
     if (n == 0)
         return 0.0;
-    const unsigned nb = (unsigned)std::min<size_t>(1024, grid_of(n));
-    DevBuf part(sizeof(double) * nb);
-    hipLaunchKernelGGL(k_vd_sumsq, dim3(nb), dim3(kNT), 0, st, x, n, part.as<double>());
-    KQ_HIP_CHECK(hipGetLastError());
-    std::vector<double> h(nb);
-    KQ_HIP_CHECK(hipMemcpyAsync(h.data(), part.as<void>(), sizeof(double) * nb, hipMemcpyDeviceToHost, st));
+    DevBuf part(sizeof(double) * kSumsqParts);
+    vd_sumsq_partials(&x, &n, 1, part.as<double>(), st);
+    std::vector<double> h(sumsq_nblk(n));
+    KQ_HIP_CHECK(hipMemcpyAsync(h.data(), part.as<void>(), sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
     KQ_HIP_CHECK(hipStreamSynchronize(st));
-    double s = 0.0;
-    for (double v : h)
-        s += v;
-    return s;
+    return vd_sumsq_total(h.data(), n);
 }
 
 #define KQ_PT_INST(LF, LL)                                                                                          \
@@ -748,7 +880,7 @@ double vd_sumsq(const double *x, size_t n, hipStream_t st)
     template void pt_backward_hidden<LF, LL>(const Geom &, int, LF, LL, const PtWeightsBF &, const float2 *,         \
                                              float2 *, hipStream_t);                                                \
     template void pt_weight_grads<LF, LL>(const Geom &, int, LF, LL, const float2 *, const float2 *,                 \
-                                          const float2 *, const float2 *, double *, hipStream_t);
+                                          const float2 *, const float2 *, double2 *, hipStream_t);
 KQ_PT_INST(LinkF, LinkF)
 KQ_PT_INST(LinkF, LinkF12)
 KQ_PT_INST(LinkH, LinkH12)

@@ -101,7 +101,7 @@ static KuQCDStatus solve_ref_t(int slot, LF fat, LL lng, void **x, void *b, KuQC
     run.enable_deferred(deferred_slots<T>(1, g.Vh));
     DevBuf stage, bdev(sizeof(c2_t<T>) * 3 * (size_t)g.Vh);
     const size_t n3 = (size_t)3 * g.Vh;
-    upload_vec<T, T>(b, Vec<T>{bdev.as<c2_t<T>>(), g.Vh, n3}, 0, stage, c.stream);
+    upload_vec<T, T>(b, Vec<T>{bdev.as<c2_t<T>>(), g.Vh, n3}, 0, stage, c.stream, false);
     std::vector<T> sh(ns);
     for (int k = 0; k < ns; ++k)
         sh[k] = (T)p.shifts[k];  // kuqcd.cpp:270-272
@@ -145,8 +145,9 @@ static KuQCDStatus solve_ref_t(int slot, LF fat, LL lng, void **x, void *b, KuQC
         if (copied[k])
             continue;
         Vec<T> xv{reinterpret_cast<c2_t<T> *>(run.x_lo(0, k)), g.Vh, n3};
-        download_vec<T, T>(xv, 0, x[k], stage, c.stream);
+        download_vec<T, T>(xv, 0, x[k], stage, c.stream, false);
     }
+    KQ_HIP_CHECK(hipStreamSynchronize(c.stream));
     p.iter = iter;
     print_iters(iter, p.max_iter);
     return KUQCD_SUCCESS;
@@ -226,7 +227,7 @@ static KuQCDStatus solve_full_t(int slot, LF fat, LL lng, void **x, void *b, KuQ
                        base + (3 + (size_t)ns) * n, part.as<double>(), part.as<double>() + flat_dot_nblk(n)};
     const Vec<T> rv{ops.r, g.Vh, n3};
     for (int q = 0; q < 2; ++q)
-        upload_vec<T, T>(static_cast<const T *>(b) + (size_t)6 * g.Vh * q, rv, q, stage, c.stream);
+        upload_vec<T, T>(static_cast<const T *>(b) + (size_t)6 * g.Vh * q, rv, q, stage, c.stream, false);
     for (int k = 0; k < ns; ++k)
         KQ_HIP_CHECK(hipMemcpyAsync(ops.pk(k), ops.r, sizeof(V2) * n, hipMemcpyDeviceToDevice, c.stream));
     KQ_HIP_CHECK(hipMemsetAsync(ops.x, 0, sizeof(V2) * n * ns, c.stream));
@@ -237,7 +238,8 @@ static KuQCDStatus solve_full_t(int slot, LF fat, LL lng, void **x, void *b, KuQ
     for (int k = 0; k < ns; ++k)
         for (int q = 0; q < 2; ++q)
             download_vec<T, T>(Vec<T>{ops.xk(k), g.Vh, n3}, q, static_cast<T *>(x[k]) + (size_t)6 * g.Vh * q, stage,
-                               c.stream);
+                               c.stream, false);
+    KQ_HIP_CHECK(hipStreamSynchronize(c.stream));
     p.iter = iter;
     print_iters(iter, p.max_iter);
     return KUQCD_SUCCESS;
@@ -689,7 +691,7 @@ KuQCDStatus solve_extended(int slot, int nrhs, void **x, void **b, KuQCDInvertPa
     DevBuf bdev(sizeof(double2) * nrhs * n3), stage;
     for (int r = 0; r < nrhs; ++r) {
         Vec<double> bv{bdev.as<double2>(), P.g.Vh, n3};
-        upload_vec<double, double>(b[r], bv, r, stage, c.stream);
+        upload_vec<double, double>(b[r], bv, r, stage, c.stream, false);
     }
     P.b = &bdev;
     {
@@ -720,12 +722,13 @@ KuQCDStatus solve_extended(int slot, int nrhs, void **x, void **b, KuQCDInvertPa
         set_error("unknown mode");
         return KUQCD_ERR_INVALID_PARAM;
     }
-    // solutions to the host (double)
+    // solutions to the caller's arrays (double)
     for (int r = 0; r < nrhs; ++r)
         for (int k = 0; k < P.ns; ++k) {
             Vec<double> xv{xdev.as<double2>() + ((size_t)r * P.ns + k) * n3, P.g.Vh, n3};
-            download_vec<double, double>(xv, 0, x[(size_t)r * P.ns + k], stage, c.stream);
+            download_vec<double, double>(xv, 0, x[(size_t)r * P.ns + k], stage, c.stream, false);
         }
+    KQ_HIP_CHECK(hipStreamSynchronize(c.stream));
     const double total = secs(t0, clk::now());
     int maxit = 0;
     for (int r = 0; r < nrhs; ++r) {

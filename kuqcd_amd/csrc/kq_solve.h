@@ -26,6 +26,10 @@ void copy_from_host(void *d, const void *h, size_t bytes, hipStream_t st);
 
 // true for device memory of the current GPU (not host, managed or another GPU's memory)
 bool on_this_device(const void *p);
+// true where kernels can read or write a caller's array of `bytes` bytes with elements of `elem` bytes
+// themselves: aligned, in device memory of the current GPU and inside one allocation. Other arrays
+// go through a copy, which reports what it cannot reach.
+bool in_place(const void *p, size_t bytes, size_t elem);
 
 // dst = sigma src - D D src on parity `parity`, src and dst in the caller's host layout in device
 // memory (not overlapping), tmp a device vector of the other parity: two launches, not waited for
@@ -52,10 +56,19 @@ inline void mdaggm_host(LF fat, LL lng, const Geom &g, const R *src, R *dst, c2_
     launch_dslash_host(a, LAY_HOST_DST, EPI_AXMY, 1, st);
 }
 
-// caller vector (reference layout, HR; host or device memory) -> device SoA vector r of v
-template <typename HR, typename VR> inline void upload_vec(const void *h, Vec<VR> v, int r, DevBuf &stage, hipStream_t st)
+// caller vector (reference layout, HR; host or device memory) -> device SoA vector r of v. Device
+// arrays are converted where they lie (an upload through a staging copy took 16 us at 16^4, 5 of
+// them the copy and 8 the wait); wait = false leaves the wait for the conversion to the caller,
+// who waits for the stream before its own return.
+template <typename HR, typename VR> inline void upload_vec(const void *h, Vec<VR> v, int r, DevBuf &stage, hipStream_t st, bool wait = true)
 {
     const size_t n = (size_t)6 * v.Vh;
+    if (in_place(h, sizeof(HR) * n, sizeof(HR))) {
+        vec_host_to_soa<HR, VR>(static_cast<const HR *>(h), v, r, st);
+        if (wait)
+            KQ_HIP_CHECK(hipStreamSynchronize(st));
+        return;
+    }
     if (stage.bytes() < sizeof(HR) * n)
         stage.alloc(sizeof(HR) * n);
     copy_from_host(stage.as<void>(), h, sizeof(HR) * n, st);
@@ -63,9 +76,15 @@ template <typename HR, typename VR> inline void upload_vec(const void *h, Vec<VR
     KQ_HIP_CHECK(hipStreamSynchronize(st));
 }
 
-template <typename VR, typename HR> inline void download_vec(Vec<VR> v, int r, void *h, DevBuf &stage, hipStream_t st)
+template <typename VR, typename HR> inline void download_vec(Vec<VR> v, int r, void *h, DevBuf &stage, hipStream_t st, bool wait = true)
 {
     const size_t n = (size_t)6 * v.Vh;
+    if (in_place(h, sizeof(HR) * n, sizeof(HR))) {
+        vec_soa_to_host<VR, HR>(v, r, static_cast<HR *>(h), st);
+        if (wait)
+            KQ_HIP_CHECK(hipStreamSynchronize(st));
+        return;
+    }
     if (stage.bytes() < sizeof(HR) * n)
         stage.alloc(sizeof(HR) * n);
     vec_soa_to_host<VR, HR>(v, r, stage.as<HR>(), st);

@@ -140,6 +140,20 @@ bool pageable(const void *p)
 
 }  // namespace
 
+bool in_place(const void *p, size_t bytes, size_t elem)
+{
+    if ((uintptr_t)p % elem != 0 || !on_this_device(p))
+        return false;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, const_cast<void *>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t o = (size_t)(static_cast<const char *>(p) - static_cast<const char *>(base));
+    return o <= size && bytes <= size - o;
+}
+
 bool on_this_device(const void *p)
 {
     hipPointerAttribute_t a{};

@@ -163,3 +163,85 @@ def test_split_terms_in_solves(gpu, links, mode):
                 assert np.linalg.norm(res) <= 1.01e-10 * np.linalg.norm(b[r]), (m, nr, r, k)
         # the 16-bit fat links leave the base system some more iterations (its refinement does the rest)
         assert rep[0].iter <= (2 if m == 3 else 1.2) * iters[1, 1] + 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [8, 4])
+def test_solves_and_gradients_on_device_arrays(gpu, prec):
+    """Sources and solutions on the device, aligned and one real off, and in host arrays: the same numbers."""
+    kq, L = gpu, gpu.L.lib()
+    lat, ns = (10, 6, 6, 6), 4
+    dt = np.float64 if prec == 8 else np.float32
+    _load(kq, lat, prec)
+    b = kq.gen_source(lat, 0, seed=81).astype(dt)
+
+    def par():
+        return kq.InvertParam(shifts=[0.05, 0.1, 0.5, 1.0], tol=1e-8, max_iter=400, num_shift=ns, prec=prec)
+
+    want = [np.zeros_like(b) for _ in range(ns)]
+    assert kq.kuqcd_solve_multishift(want, b, par()) == 0, kq.last_error()
+    for shift in (0, prec):
+        bd, xd = _Dev(kq, b.nbytes, shift), [_Dev(kq, b.nbytes, shift) for _ in range(ns)]
+        try:
+            bd.put(b)
+            xp = (C.c_void_p * ns)(*[x.p for x in xd])
+            assert L.kq_solve_multishift(xp, C.c_void_p(bd.p), C.byref(par().struct())) == 0, kq.last_error()
+            for k in range(ns):
+                assert np.array_equal(xd[k].get(b), want[k])
+        finally:
+            for a in [bd] + xd:
+                a.free()
+    if prec == 4:
+        return
+    w = kq.ptnet_init_weights(3, 0.2)
+    e = kq.gen_source(lat, 0, seed=82)
+    res = []
+    for shift in (None, 0, 8):
+        dev = [] if shift is None else [_Dev(kq, b.nbytes, shift) for _ in range(2)]
+        try:
+            for a, v in zip(dev, (b, e)):
+                a.put(v)
+            at = [a.p for a in dev] or [b.ctypes.data, e.ctypes.data]
+            loss, only, g = C.c_double(), C.c_double(), np.empty(2 * kq.KQ_PT_PARAMS)
+            assert L.kq_ptnet_loss_grad(C.byref(w), 0, 0.05, C.c_void_p(at[0]), C.c_void_p(at[1]), C.byref(loss),
+                                        g.ctypes.data_as(C.POINTER(C.c_double))) == 0, kq.last_error()
+            assert L.kq_ptnet_loss_grad(C.byref(w), 0, 0.05, C.c_void_p(at[0]), C.c_void_p(at[1]), C.byref(only),
+                                        None) == 0, kq.last_error()
+            assert only.value == loss.value > 0.0
+            res.append(np.append(g, loss.value))
+        finally:
+            for a in dev:
+                a.free()
+    assert np.array_equal(res[0], res[1]) and np.array_equal(res[0], res[2])
+    # a zero pair: loss and gradient are 0
+    z = np.zeros_like(b)
+    assert L.kq_ptnet_loss_grad(C.byref(w), 0, 0.05, z.ctypes.data_as(C.c_void_p), z.ctypes.data_as(C.c_void_p),
+                                C.byref(loss), g.ctypes.data_as(C.POINTER(C.c_double))) == 0
+    assert loss.value == 0.0 and not g.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lat", [(6, 5, 4, 3), (32, 32, 32, 18), (32, 32, 32, 34)])
+def test_refinement_over_its_partial_sums(gpu, lat):
+    """The flexible CG with fewer sites than a workgroup, and where the network layer's partials
+    (above 262144 half-lattice sites) and the operator's (above 524288) are summed in slices first:
+    plain CG and the network's iteration reach the residual, which the operator confirms."""
+    kq, L = gpu, gpu.L.lib()
+    _load(kq, lat, 8)
+    b = kq.gen_source(lat, 0, seed=91)
+    # channel 0 is D r, the output 8/b r - c A r = (8/b - c sigma) r + c D D r: positive up to A = b
+    nu, sigma, bound = kq.ptnet_norms(), 0.5, 5.0
+    c = 0.9 * 8.0 / bound**2
+    hop = np.array([(-1.0 if t & 2 else 1.0) * nu[t & 1] for t in range(16)])
+    W1, W2 = np.zeros((4, 16), complex), np.zeros((4, 16), complex)
+    W1[0], W2[0] = hop, c * hop
+    assert kq.ptnet_set_weights(kq.weights_from_array(W1, W2, 8.0 / bound - c * sigma)) == 0
+    for learned in (0, 1):
+        print("case", lat, learned, flush=True)
+        x = np.zeros_like(b)
+        st, rep = kq.fcg_refine(b, x, sigma, 0, kq.refine_options(rel_tol=1e-9, learned=learned, max_iter=300))
+        assert st == 0, kq.last_error()
+        assert rep.converged and not rep.fallback and rep.iter < 100
+        ax = np.empty_like(b)
+        assert kq.mdaggm(x, ax, 0, sigma, 1) == 0
+        assert np.linalg.norm(b - ax) <= 1.01e-9 * np.linalg.norm(b)
