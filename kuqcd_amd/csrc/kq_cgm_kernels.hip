@@ -9,7 +9,7 @@
 // order. The scalar recurrences run in a workgroup of their own beside the vector update that
 // needs the scalar, instead of in one-workgroup kernels between the vector kernels (3-5 us each,
 // plus 1.2 us from one kernel to the next: a third of an iteration at 8^4 and 16^4).
-#include "kq_cgm_kernels.h"
+#include "kq_cgm_device.h"
 
 namespace kq {
 
@@ -255,44 +255,7 @@ __global__ void __launch_bounds__(kBlasNT) k_cgm_update_p(CgmState<S> *st, XR *x
     const int mt = c.maxTermPrev;
     const bool defer = c.dslot >= 0;
     if (blockIdx.x == nb) {
-        const int hj = c.hist;
-        const bool rec = shist != nullptr && defer && hj < kHistMax;
-        double *h = rec ? shist + hist_scalar_index(c.dslot, hj, 2, 0) : nullptr;
-        __syncthreads();
-        for (int j = 1 + (int)threadIdx.x; j < mt; j += blockDim.x) {
-            const S aj = a0 * c.Z[j] * c.B[j] / (c.Zm1[j] * B0);
-            c.a[j] = aj;
-            if (rec)
-                h[j] = (double)aj;
-        }
-        if (threadIdx.x != 0)
-            return;
-        c.a[0] = a0;
-        c.rr = lambda2;
-        c.maxTermUpd = mt;
-        if (rec) {
-            h[0] = (double)a0;
-            h[kMaxShift] = (double)mt;
-            c.hist = hj + 1;
-        }
-        // drop converged shifts from the end of the list (inverter_cgm.cpp:71-76)
-        int left = mt;
-        while (left > 0) {
-            const S lambda = c.Z[left - 1] * c.Z[left - 1] * lambda2;
-            if (!((double)lambda < c.tolk[left - 1]))
-                break;
-            left--;
-        }
-        c.maxTerm = left;
-        const int iter = c.iter + 1;
-        c.iter = iter;
-        const bool stop = left <= 0 || iter >= c.maxIter;
-        const bool pause = c.pause2 > 0.0 && l2_d < c.pause2 * c.r2max;
-        if (stop)
-            c.stop = 1;
-        if (pause)
-            c.pause = 1;
-        c.live = !stop && !pause;
+        cgm_finish_iteration(c, l2_d, shist);
         return;
     }
     // a system with deferred solution updates keeps only p_0 current (its x_k and p_k, k >= 1,

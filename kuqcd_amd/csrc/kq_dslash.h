@@ -55,7 +55,16 @@ inline int repro_nt(uint32_t Vh) { return Vh < 200000u ? 64 : 256; }
 template <class LF, class LL, typename SR>
 uint32_t launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStream_t st, int cap = 0);
 
-// The same on vectors of the loaded gauge's precision in the caller's host layout (device memory,
+// D p with p = z r + a p formed on the way, for one system that is deferred or has one live shift
+// (k_dslash_split_p): a.src holds p before the update, pnew takes it after the update, part the npart
+// partial sums of |r|^2; x, if not deferred, takes x - beta p. Does nothing unless st->run is set. Only where dslash_split_waves(.., 1, 1)
+// is 8.
+template <typename S> struct CgmState;
+template <class LF, class LL, typename SR>
+void launch_dslash_p(DslashArgs<LF, LL, SR> a, CgmState<SR> *st, const c2_t<SR> *r, Vec<SR> pnew, Vec<SR> x,
+                     const double *part, uint32_t npart, double *shist, hipStream_t stream);
+
+// launch_dslash on vectors of the loaded gauge's precision in the caller's host layout (device memory,
 // aligned to their reals): lay LAY_HOST with EPI_STORE (D src, nr right-hand sides per block), or
 // the two terms of sigma0 src - D D src on one right-hand side, LAY_HOST_SRC with EPI_STORE and
 // LAY_HOST_DST with EPI_AXMY, whose intermediate is in colour planes. The vectors of one launch

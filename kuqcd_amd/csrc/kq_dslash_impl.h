@@ -13,6 +13,7 @@
 // formats (one translation unit per family, so they compile in parallel).
 #pragma once
 
+#include "kq_cgm_device.h"
 #include "kq_dslash.h"
 
 #include <algorithm>
@@ -34,9 +35,29 @@ __device__ __forceinline__ void gather(const V2 *src, uint32_t n, uint32_t Vh, V
     }
 }
 
-template <class A, class LK, int NR, int MU, int H, bool AOS = false>
+// A search direction that is formed where it is gathered: z r + a p, rounded as k_cgm_update_p does
+template <class V2, typename R> struct PSource {
+    const V2 *p, *r;
+    R z, a;
+    __device__ __forceinline__ V2 at(size_t i) const
+    {
+#pragma clang fp contract(off)
+        const V2 pv = p[i], rv = r[i];
+        return mk<V2>(fmadd(z, rv.x, a * pv.x), fmadd(z, rv.y, a * pv.y));
+    }
+};
+template <bool AOS = false, class V2, typename R>
+__device__ __forceinline__ void gather(const PSource<V2, R> &src, uint32_t n, uint32_t Vh, V2 v[3])
+{
+    static_assert(!AOS, "colour planes");
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        v[c] = src.at((size_t)c * Vh + n);
+}
+
+template <class A, class LK, int NR, int MU, int H, bool AOS = false, class Src>
 __device__ __forceinline__ void hop_fwd(const A &a, const LK &lk, uint32_t s, const SiteCoord &sc,
-                                        const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+                                        const Src *src, typename A::R acc[NR][6])
 {
     using R = typename A::R;
     c2_t<R> U[9];
@@ -50,9 +71,9 @@ __device__ __forceinline__ void hop_fwd(const A &a, const LK &lk, uint32_t s, co
     }
 }
 
-template <class A, class LK, int NR, int MU, int H, bool AOS = false>
+template <class A, class LK, int NR, int MU, int H, bool AOS = false, class Src>
 __device__ __forceinline__ void hop_bwd(const A &a, const LK &lk, uint32_t s, const SiteCoord &sc,
-                                        const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+                                        const Src *src, typename A::R acc[NR][6])
 {
     using R = typename A::R;
     const uint32_t n = nb_index<MU>(a.g, s, sc, -H);
@@ -330,9 +351,9 @@ __global__ void __launch_bounds__(NT) k_dslash(const DslashArgs<LF, LL, SR> a)
 // (32^4 176 -> 195). S = 4 and 16 are up to 10 % slower than 8 at 8^4 to 16^4.
 
 // Hops of one wave: hop I = 4 mu + 2 (backward) + (3 hops)
-template <class A, class LF, class LL, int NR, bool SA, int I>
-__device__ __forceinline__ void split_hop(const A &a, uint32_t s, const SiteCoord &sc,
-                                          const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+template <class A, class LF, class LL, int NR, bool SA, int I, class Src>
+__device__ __forceinline__ void split_hop(const A &a, uint32_t s, const SiteCoord &sc, const Src *src,
+                                          typename A::R acc[NR][6])
 {
     constexpr int MU = I / 4;
     if constexpr ((I & 3) == 0)
@@ -345,18 +366,18 @@ __device__ __forceinline__ void split_hop(const A &a, uint32_t s, const SiteCoor
         hop_bwd<A, LL, NR, MU, 3, SA>(a, a.lng, s, sc, src, acc);
 }
 
-template <class A, class LF, class LL, int NR, bool SA, int I, int N>
-__device__ __forceinline__ void split_hops(const A &a, uint32_t s, const SiteCoord &sc,
-                                           const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+template <class A, class LF, class LL, int NR, bool SA, int I, int N, class Src>
+__device__ __forceinline__ void split_hops(const A &a, uint32_t s, const SiteCoord &sc, const Src *src,
+                                           typename A::R acc[NR][6])
 {
     split_hop<A, LF, LL, NR, SA, I>(a, s, sc, src, acc);
     if constexpr (N > 1)
         split_hops<A, LF, LL, NR, SA, I + 1, N - 1>(a, s, sc, src, acc);
 }
 
-template <class A, class LF, class LL, int NR, bool SA, int S, int W>
-__device__ __forceinline__ void split_wave(int w, const A &a, uint32_t s, const SiteCoord &sc,
-                                           const typename A::V2 *const src[NR], typename A::R acc[NR][6])
+template <class A, class LF, class LL, int NR, bool SA, int S, int W, class Src>
+__device__ __forceinline__ void split_wave(int w, const A &a, uint32_t s, const SiteCoord &sc, const Src *src,
+                                           typename A::R acc[NR][6])
 {
     if (w == W)
         split_hops<A, LF, LL, NR, SA, W * (16 / S), 16 / S>(a, s, sc, src, acc);
@@ -476,6 +497,97 @@ __global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL
                 a.partial[(size_t)rr[j] * a.nblk + blockIdx.x] = tot;
             }
     }
+}
+
+// The split hopping term of one system, deferred or down to one shift, with the previous iteration's
+// direction update on the way: src is p before the update, every gather forms z r + a p, and the
+// workgroup stores the updated direction of its own 64 entries in pnew (two buffers take turns: other
+// workgroups still gather the old one) and, if the system is not deferred, their solution. An iteration
+// then has 3 kernels instead of 4, which is what a small lattice's time consists of; the gathers
+// double, from L2. The last workgroup finishes the previous iteration's scalars instead, and every
+// workgroup adds the npart partials of |r|^2 wave by wave in the same order.
+// Per launch (LinkD, LinkD14, 8^4) 6.4 us against 5.1 for the plain term and 3.7 for the update; at
+// 16^4 in FP32 10.9 against 8.8 and 4.2. Bound by its chain of loads and by the launch itself.
+template <class LF, class LL, typename SR>
+__global__ void __launch_bounds__(512)
+k_dslash_split_p(const DslashArgs<LF, LL, SR> a, CgmState<SR> *st, const c2_t<SR> *r, Vec<SR> pnew, Vec<SR> x,
+                 const double *part, uint32_t npart, double *shist)
+{
+    using A = DslashArgs<LF, LL, SR>;
+    using V2 = c2_t<SR>;
+    constexpr int S = 8, H = S / 2, NT = 64 * S;
+    __shared__ SR red[H][1][6][64];
+    __shared__ uint32_t site[64];
+    if (st->run == 0)
+        return;  // uniform over the grid: no workgroup of this kernel writes it
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double l2 = 0.0;
+    for (uint32_t i = lane; i < npart; i += 64)
+        l2 += part[i];
+    l2 = wave_sum(l2);
+    if (blockIdx.x == a.nblk) {
+        cgm_finish_iteration(*st, l2, shist);
+        return;
+    }
+    const PSource<V2, SR> src{a.src.p + a.src.base(0), r, st->Z[0], (SR)l2 / st->rr_prev};
+    bool valid;
+    const uint32_t s = tile_site<64>(a.g, blockIdx.x, a.nblk, lane, valid);
+    SR acc[1][6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+        acc[0][k] = 0;
+    if (valid) {
+        const SiteCoord sc = site_coords(a.g, s, a.dst_parity);
+        split_wave<A, LF, LL, 1, false, S, 0>(w, a, s, sc, &src, acc);
+    }
+    if (w == 0)
+        site[lane] = valid ? s : 0xffffffffu;
+    if (w >= H) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            red[w - H][0][k][lane] = acc[0][k];
+    }
+    __syncthreads();
+    if (w < H) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            red[w][0][k][lane] += acc[0][k];
+    }
+    __syncthreads();
+    const int e = threadIdx.x - (NT - 192);  // the last three waves store one colour each
+    if (e < 0)
+        return;
+    const int l = e & 63, c = e >> 6;
+    const uint32_t sl = site[l];
+    if (sl == 0xffffffffu)
+        return;
+    SR re = red[0][0][2 * c][l], im = red[0][0][2 * c + 1][l];
+#pragma unroll
+    for (int k = 1; k < H; ++k) {
+        re += red[k][0][2 * c][l];
+        im += red[k][0][2 * c + 1][l];
+    }
+    const size_t o = (size_t)c * a.g.Vh + sl;
+    put<LF>(&a.dst.p[a.dst.base(0) + o], mk<V2>(re, im));
+    pnew.p[pnew.base(0) + o] = src.at(o);
+    if (st->dslot < 0) {
+        const SR b = st->B[0];
+        const V2 po = src.p[o];
+        V2 *xo = x.p + x.base(0) + o, xv = *xo;
+        xv.x = fmadd(-b, po.x, xv.x);
+        xv.y = fmadd(-b, po.y, xv.y);
+        *xo = xv;
+    }
+}
+
+template <class LF, class LL, typename SR>
+void launch_dslash_p(DslashArgs<LF, LL, SR> a, CgmState<SR> *st, const c2_t<SR> *r, Vec<SR> pnew, Vec<SR> x,
+                     const double *part, uint32_t npart, double *shist, hipStream_t stream)
+{
+    a.nblk = dslash_grid(a.g.Vh, 64);
+    hipLaunchKernelGGL((k_dslash_split_p<LF, LL, SR>), dim3(a.nblk + 1), dim3(512), 0, stream, a, st, r, pnew, x,
+                       part, npart, shist);
+    KQ_HIP_CHECK(hipGetLastError());
 }
 
 // The batched hopping term with the x and y neighbours read from LDS: the workgroup (256 sites,

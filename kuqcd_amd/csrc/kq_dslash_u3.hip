@@ -11,5 +11,7 @@ template uint32_t launch_dslash<LinkF, LinkH12C, float>(DslashArgs<LinkF, LinkH1
 template uint32_t launch_dslash<LinkH, LinkH12C, float>(DslashArgs<LinkH, LinkH12C, float>, int, int, int, hipStream_t,
                                                     int);
 template void launch_dslash_host<LinkF, LinkF12C, float>(const DslashArgs<LinkF, LinkF12C, float> &, int, int, int, hipStream_t);
+template void launch_dslash_p<LinkF, LinkF12C, float>(DslashArgs<LinkF, LinkF12C, float>, CgmState<float> *, const c2_t<float> *, Vec<float>, Vec<float>,
+                                              const double *, uint32_t, double *, hipStream_t);
 
 }  // namespace kq

@@ -342,11 +342,27 @@ public:
         ndslot_ = std::max(0, slots);
         if (ndslot_ == 0)
             return;
+        if constexpr (std::is_same<S, VR>::value)
+            if (max_sys_ == 1 && !reliable_ && g_.Vh <= kHopDirectionSites) {
+                // a runner of one system: it is deferred until one shift is left, so the direction
+                // updates can be part of the hopping terms (chunk()). The direction changes buffers
+                // in every iteration but the first of a chunk, and ends the chunk where it began.
+                tune_.chunk = (tune_.chunk - 1) | 1;
+                p1_.alloc(sizeof(V2) * n3_);
+            }
         shist_.alloc(sizeof(double) * hist_scalar_index(ndslot_, 0, 0, 0));
         rhist_.alloc(sizeof(V2) * (size_t)ndslot_ * kHistMax * n3_);
         p0snap_.alloc(sizeof(V2) * (size_t)ndslot_ * n3_);
         coef_.alloc(sizeof(double) * (size_t)ndslot_ * kMaxShift * kCoefStride);
     }
+
+    // Largest half lattice whose hopping terms update the direction of a single system: one workgroup of
+    // 64 sites per CU. Reference solves with 4 shifts, separate update -> in the hopping term: FP64
+    // 8^4 3.52 -> 3.24 ms, 12^3x8 4.05 -> 3.49, 12^4 4.32 -> 3.89, 16x12^3 4.57 -> 4.37, 16^2x12^2 (18432
+    // sites) 5.91 -> 5.90, 16^4 7.00 -> 7.16; FP32 8^4 2.22 -> 1.92, 12^4 2.36 -> 1.97, 16x12^3
+    // 2.45 -> 2.09, 16^2x12^2 2.57 -> 2.51, 16^4 2.82 -> 2.88. (Where the split term is used with 8
+    // waves in both precisions, which the launch relies on.)
+    static constexpr uint32_t kHopDirectionSites = 16384;
 
     // Register a system; it starts at the next run() step. shifts: reference
     // convention (absolute shifts[0], shifts[k>=1] relative to it); tolk: absolute
@@ -420,8 +436,7 @@ public:
                 nlive += (!state_h_[sys].stop && !state_h_[sys].pause) ? 1 : 0;
             if (direct_launches()) {
                 const int nr = tune_.pick_nr(nlive);
-                for (int c = 0; c < tune_.chunk; ++c)
-                    iteration(nr, std::max(1, (nlive + nr - 1) / nr));
+                chunk(nr, std::max(1, (nlive + nr - 1) / nr));
             } else {
                 hipGraphExec_t gx = graph_for(nlive);
                 KQ_HIP_CHECK(hipGraphLaunch(gx, st_));
@@ -773,10 +788,30 @@ private:
         download_states();  // keep the host copy current (rr, r2max set on the device)
     }
 
-    // One iteration on the runner's stream (what the graphs hold), with the
-    // hopping term blocked nr right-hand sides per thread and every per-system
-    // grid sized for nr * groups live systems.
-    void iteration(int nr, int groups)
+    // One chunk of iterations on the runner's stream (what the graphs hold), with the hopping term
+    // blocked nr right-hand sides per thread and every per-system grid sized for nr * groups live
+    // systems. A single system on a small lattice (p1_) has the direction updates of all
+    // but the chunk's last iteration done by the hopping terms after them, so that only whole
+    // iterations are seen between chunks.
+    void chunk(int nr, int groups)
+    {
+        const Vec<VR> p0 = vec_p0();
+        Vec<VR> p = p0;
+        for (int i = 0; i < tune_.chunk; ++i) {
+            if (!p1_) {
+                iteration(nr, groups, p, nullptr, true);
+            } else {
+                const Vec<VR> q = p.p == p0.p ? vec(p1_) : p0;
+                iteration(nr, groups, p, i > 0 ? &q : nullptr, i == tune_.chunk - 1);
+                if (i > 0)
+                    p = q;
+            }
+        }
+    }
+
+    // One iteration from the directions p, or from the pending update of p into pnew; update_p: update
+    // the directions at its end
+    void iteration(int nr, int groups, Vec<VR> p, const Vec<VR> *pnew, bool update_p)
     {
         CgmLaunch L = launch(nr * groups);
         CgmState<S> *st = state_.as<CgmState<S>>();
@@ -791,18 +826,27 @@ private:
         d.nact = L.nact;
         d.nrhs = L.nlaunch;
         d.dst_parity = 1 - parity_;
-        d.src = vec_p0();
+        d.src = p;
         d.dst = vec(tmp_);
-        launch_dslash(d, EPI_STORE, nr, tune_.nt, st_, tune_.cap_for(nr));
+        if constexpr (std::is_same<S, VR>::value) {
+            if (pnew)
+                launch_dslash_p(d, st, r_.as<V2>(), *pnew, Vec<VR>{x_.as<V2>(), g_.Vh, 0, off_.as<size_t>()},
+                                part_b_.as<double>(), cgm_update_nblk(g_.Vh), L.shist, st_);
+        }
+        if (!pnew)
+            launch_dslash(d, EPI_STORE, nr, tune_.nt, st_, tune_.cap_for(nr));
+        else
+            p = *pnew;
         d.dst_parity = parity_;
         d.src = vec(tmp_);
         d.dst = vec(s_);
-        d.aux = vec_p0();
+        d.aux = p;
         d.sigma = sigma_.as<double>();
         d.partial = part_a_.as<double>();
         L.nblk_dsl = launch_dslash(d, EPI_AXMY_DOT, nr, tune_.nt, st_, tune_.cap_for(nr));
         cgm_update_r<S, VR>(st, vec(r_), vec(s_), L, st_);
-        cgm_update_p<S, VR, VR>(st, x_.as<VR>(), p_.as<VR>(), vec(r_), L, st_);
+        if (update_p)
+            cgm_update_p<S, VR, VR>(st, x_.as<VR>(), p_.as<VR>(), vec(r_), L, st_);
     }
 
     // graph of one chunk of iterations for nlive live systems: right-hand-side blocking nr
@@ -817,8 +861,7 @@ private:
         if (!gx) {
             hipGraph_t graph;
             KQ_HIP_CHECK(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
-            for (int i = 0; i < tune_.chunk; ++i)
-                iteration(nr, groups);
+            chunk(nr, groups);
             KQ_HIP_CHECK(hipStreamEndCapture(st_, &graph));
             KQ_HIP_CHECK(hipGraphInstantiate(&gx, graph, nullptr, nullptr, 0));
             KQ_HIP_CHECK(hipGraphDestroy(graph));
@@ -836,7 +879,7 @@ private:
     RunnerTuning tune_;
     size_t n3_ = 0;
     uint32_t nblk_ = 0;
-    DevBuf r_, s_, tmp_, p_, x_, state_, part_a_, part_b_, part_f_, ints_, sigma_, off_;
+    DevBuf r_, s_, tmp_, p_, p1_, x_, state_, part_a_, part_b_, part_f_, ints_, sigma_, off_;
     Pinned<CgmState<S>> state_h_;
     Pinned<int> list_stage_;  // kStages slots of max_sys_ system indices
     int stage_slot_ = 0, stage_uses_ = 0, list_size_ = 1;

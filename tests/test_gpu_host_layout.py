@@ -245,3 +245,37 @@ def test_refinement_over_its_partial_sums(gpu, lat):
         ax = np.empty_like(b)
         assert kq.mdaggm(x, ax, 0, sigma, 1) == 0
         assert np.linalg.norm(b - ax) <= 1.01e-9 * np.linalg.norm(b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("links", ["su3", "u3", "general"])
+@pytest.mark.parametrize("prec", [8, 4])
+def test_direction_update_in_the_hopping_term(gpu, prec, links):
+    """The reference solve on small lattices, where the hopping term updates the direction (and on the smallest
+    one where it no longer does): stopped after
+    every kind of place in its chunks of 15 iterations (first, second, last, first of the next, within
+    the phase of one live shift) it has the oracle's iterate, with one shift and with several, on
+    ragged and odd extents. Bounds: rounding of at most 34 iterations of a system of condition
+    below 100, 1e-12 in FP64 and 1e-4 in FP32."""
+    kq = gpu
+    dt = np.float64 if prec == 8 else np.float32
+    for lat in ((6, 5, 4, 3), (10, 6, 6, 6), (16, 16, 16, 8), (18, 16, 16, 8)):
+        fat, lng = _load(kq, lat, prec, u3=links == "u3")
+        if links == "general":
+            lng = (lng * (1.0 + 0.05 * np.random.default_rng(8).normal(size=lng.shape))).astype(dt)
+            kq.kuqcd_gauge_free()
+            kq.load_gauge_pair(fat, lng, lat, prec=prec)
+        b = kq.gen_source(lat, 0, seed=95).astype(dt)
+        for given in ([0.5], [0.5, 0.2, 3.0]):
+            for max_iter in (1, 2, 15, 16, 17, 34):
+                print("case", prec, links, lat, given, max_iter, flush=True)
+                sh = np.array(given, dt)
+                x = [np.zeros_like(b) for _ in sh]
+                p = kq.InvertParam(shifts=np.array(given), tol=1e-6 if prec == 4 else 1e-18, max_iter=max_iter,
+                                   num_shift=len(given), prec=prec)
+                assert kq.kuqcd_solve_multishift(x, b, p) == 0, kq.last_error()
+                want, it = oracle.cgm(fat.astype(dt), lng.astype(dt), lat, 0, sh, b, p.tol, max_iter)
+                assert abs(p.iter - it) <= (0 if prec == 8 else 1)
+                if p.iter == it:
+                    for k in range(len(given)):
+                        assert rel_err(x[k], want[k]) <= (1e-12 if prec == 8 else 1e-4), k
