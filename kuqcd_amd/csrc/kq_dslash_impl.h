@@ -847,6 +847,13 @@ void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int n
             else
                 launch_host_split<LF, LL, SR, 1, 8>(a, lay, epi, st);
         } else {
+            // Blocks of 4 of more than 4 vectors would read the links twice: above 16384 sites they run
+            // as blocks of 8 (calls with 8 vectors in blocks of 4 -> 8, LinkF + LinkF12: 16^4
+            // 29.1 -> 26.3 us, 16^3x32 45.5 -> 42.7, 24^4 92.6 -> 76.1, 32^4 259 -> 198, 48^4
+            // 1364 -> 981; with 5 vectors 27.4 -> 25.6 to 1238 -> 853; LinkF12C likewise; but 12^4
+            // 20.7 -> 21.8, 8^4 16.8 -> 19.5)
+            if (nr == 4 && a.nrhs > 4 && a.g.Vh > 16384u)
+                nr = 8;
             switch (nr) {
             case 1:
                 launch_host_split<LF, LL, SR, 1, 8>(a, lay, epi, st);

@@ -86,7 +86,7 @@ def test_operator_on_device_arrays(gpu, lat, prec):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec,nrs", [(8, (1, 2, 4, 8)), (4, (1, 2, 3, 4, 8))])
-@pytest.mark.parametrize("lat", [(6, 5, 4, 3), (16, 12, 8, 8)])
+@pytest.mark.parametrize("lat", [(6, 5, 4, 3), (16, 12, 8, 8), (22, 18, 15, 13)])
 def test_block_of_vectors_on_device_arrays(gpu, lat, prec, nrs):
     kq, L = gpu, gpu.L.lib()
     dt = np.float64 if prec == 8 else np.float32
