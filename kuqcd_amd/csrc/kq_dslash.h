@@ -107,22 +107,27 @@ inline bool dslash_staged(const Geom &g, int nr, int nt)
     return nr >= 2 && nt == 256 && stage_enabled() && stage_lattice(g);
 }
 
-// Waves per 64 sites of the split hopping term (k_dslash_split) that launch_dslash uses for
-// `groups` groups of nr right-hand sides, or 0 where one thread per site serves better: when the
-// one-thread form's waves (Vh * groups / 64) already fill the chip. Measured per term, one
+// Waves per 64 sites of the split hopping term (k_dslash_split) that launch_dslash uses for nrhs
+// right-hand sides in blocks of nr, or 0 where one thread per site serves better: when the
+// one-thread form's waves (Vh / 64 per block) already fill the chip. Measured per term, one
 // thread per site -> split: FP64 (blocks of 1) 8^4 8.9 -> 4.5 us, 16^4 18.9 -> 12.7, 22x18x15x13
 // 20.6 -> 17.1, 16^3x32 23.9 -> 25.2; FP32 (LinkF, LinkF12) blocks of 1: 16^4 12.1 -> 7.1, 16^3x32
 // 14.5 -> 12.6, 20^4 19.0 -> 16.4, 24^4 29.8 -> 31.2; blocks of 4: 16^4 21.8 -> 12.4, 16^3x32
 // 23.8 -> 21.1, but two groups of 4 there 33 -> 37, 24^4 50 -> 47 (47.6 in workgroups of 64).
 // Blocks of 8 FP32 right-hand sides leave the one-thread form one wave per SIMD, waiting for its
-// gathers: split into 4 waves at every size, 16^4 41 -> 18, 24^4 82 -> 75, 48^4 1316 -> 1118,
-// except where the larger lattices stage rows in LDS (32^4: 174 staged, 217 split).
-inline int dslash_split_waves(bool fp64, const Geom &g, int groups, int nr)
+// gathers: split into 4 waves (or 2, launch_epi) at every size, 16^4 41 -> 18, 24^4 82 -> 75, 48^4
+// 1316 -> 1118, except where the larger lattices stage rows in LDS (32^4: 174 staged, 203 split).
+//
+// The two forms add the 16 hops in different orders. The FP64 rule therefore counts blocks of 2
+// whatever nr is: nr comes from timings in the FP64 solve of several systems and in the FP64
+// verification, whose results are the same in every process (repro_nt). Two or more FP64 vectors
+// run faster as pairs on either form (two vectors in single blocks -> a pair: 16^4 20.7 -> 13.1 us, 24^4
+// 115 -> 65, 32^4 354 -> 193, 48^4 1948 -> 1077; only at 8^4 4.4 -> 5.0), so the rule follows those.
+inline int dslash_split_waves(bool fp64, const Geom &g, int nrhs, int nr)
 {
-    const uint64_t work = (uint64_t)g.Vh * (uint64_t)groups;
     if (fp64)
-        return nr <= 2 && work <= 49152u ? 8 : 0;
-    if (work <= 98304u)
+        return nr <= 2 && (uint64_t)g.Vh * (uint64_t)((nrhs + 1) / 2) <= 49152u ? 8 : 0;
+    if ((uint64_t)g.Vh * (uint64_t)((nrhs + nr - 1) / nr) <= 98304u)
         return nr <= 2 ? 8 : 4;
     return nr == 8 && !stage_lattice(g) ? 4 : 0;
 }

@@ -771,7 +771,7 @@ static uint32_t launch_epi(DslashArgs<LF, LL, SR> a, int epi, int nt, int cap, h
     constexpr bool kDouble = std::is_same<SR, double>::value;
     if constexpr (!kDouble || NR <= 2) {
         constexpr int S = NR <= 2 ? 8 : 4;
-        if (dslash_split_waves(kDouble, a.g, (a.nrhs + NR - 1) / NR, NR) == S) {
+        if (dslash_split_waves(kDouble, a.g, a.nrhs, NR) == S) {
             a.nblk = dslash_grid(a.g.Vh, 64);
             // 16-bit long links in blocks of 8 on more than 48 K sites: 2 waves of 8 hops, whose
             // 24.8 KB of LDS let all workgroups of a middle-sized lattice run at once (16^3x32

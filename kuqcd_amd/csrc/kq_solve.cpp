@@ -287,7 +287,8 @@ static std::vector<double> true_res2_t(int slot, LinkD fat, LL lng, int parity, 
     DevBuf tmp(sizeof(double2) * nk * n3), ax(sizeof(double2) * nk * n3), sig(sizeof(double) * nk);
     DevBuf list(sizeof(int) * (nl + 1));
     // FP64 blocking and occupancy cap from the autotuner (one group of at most two
-    // right-hand sides per workgroup); the fixed block size keeps the residuals reproducible
+    // right-hand sides per workgroup); neither changes a bit of the residuals (dslash_split_waves),
+    // and the block size is fixed by the lattice
     const auto pick = tuned_launch(slot, KQ_MODE_FP64, nl);
     const int nr = std::min(pick.first, 2), nt = repro_nt(g.Vh);
     const int cap = tuned_cap(slot, KQ_MODE_FP64, nr, nt);
