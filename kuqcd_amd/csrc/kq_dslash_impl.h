@@ -375,6 +375,14 @@ __device__ __forceinline__ void split_hops(const A &a, uint32_t s, const SiteCoo
         split_hops<A, LF, LL, NR, SA, I + 1, N - 1>(a, s, sc, src, acc);
 }
 
+// Each wave branches on its index, a value uniform over the wave, to code of its own. The network's
+// layers in that form were compiled wrongly (dir_neighbours in kq_ptnet.hip): the 64 weights that
+// each path takes from the kernel's arguments filled the scalar registers, and a path was left with
+// another one's. What a path here has in scalar registers of its own are link strides. None of these
+// kernels may spill a scalar register (tests/test_kernel_resources.py); in the listing of each, walked
+// for every wave index, no register is read and no address formed before it is written; and since no
+// branch between the waves depends on data, the tests, which run every instantiation against
+// the oracle, run all of its paths.
 template <class A, class LF, class LL, int NR, bool SA, int S, int W, class Src>
 __device__ __forceinline__ void split_wave(int w, const A &a, uint32_t s, const SiteCoord &sc, const Src *src,
                                            typename A::R acc[NR][6])
@@ -443,6 +451,14 @@ __global__ void __launch_bounds__(64 * S) k_dslash_split(const DslashArgs<LF, LL
                 red[w][j][k][lane] += acc[j][k];
     }
     __syncthreads();
+    if constexpr (NR == 8 && EPI == EPI_AXMY_DOT) {
+        // The epilogue's pointers are resolved again: kept across the waves' hops, 24 of them spilled
+        // scalar registers there (split_wave). The empty asm makes the block's index unknown to the
+        // compiler, which would keep the first ones otherwise.
+        uint32_t y = blockIdx.y;
+        asm("" : "+s"(y));
+        dslash_rhs<NR>(a, (int)y * NR, nact, rr, dst, src, aux, true);
+    }
     // 192 complex results per right-hand side, summed over the slots in their order; consecutive
     // threads take consecutive entries of the destination's layout
     double d[DOTS];

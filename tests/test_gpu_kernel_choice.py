@@ -2,9 +2,12 @@
 import numpy as np
 import pytest
 
+import oracle
+from conftest import rel_err
 
-def _load(kq, lat, u3=False, general=False):
-    """A weak-field double pair; long links as multiples of SU(3), U(3), or (general) neither."""
+
+def _load(kq, lat, u3=False, general=False, prec=8):
+    """A weak-field pair; long links as multiples of SU(3), U(3), or (general) neither."""
     fat, lng = kq.gen_gauge(lat, kind=kq.KQ_GEN_WEAK, eps=0.3, seed_fat=21, seed_long=22)
     if u3:
         ph = np.exp(1j * np.random.default_rng(5).normal(size=lng.shape[:2]))[:, :, None]
@@ -12,7 +15,7 @@ def _load(kq, lat, u3=False, general=False):
     if general:
         lng = lng * (1.0 + 0.05 * np.random.default_rng(8).normal(size=lng.shape))
     kq.kuqcd_gauge_free()
-    kq.load_gauge_pair(fat, lng, lat)
+    kq.load_gauge_pair(fat, lng, lat, prec=prec)
     return fat, lng
 
 
@@ -47,3 +50,50 @@ def test_fp64_results_do_not_depend_on_the_blocking(gpu, lat, n):
             assert out[nr][1][r].iter == out[1][1][r].iter
             assert list(out[nr][1][r].true_rel_res) == list(out[1][1][r].true_rel_res)
         assert all(np.array_equal(u, v) for u, v in zip(out[nr][0], out[1][0])), nr
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("links", ["su3", "u3"])
+@pytest.mark.parametrize("mode", [3, 4])
+def test_split_term_with_two_waves_in_solves(gpu, mode, links):
+    """Blocks of 8 with 16-bit long links on more than 49152 sites of one parity run with 2 waves per
+    64 sites, in both terms of an iteration: solves whose every shift reaches an FP64 residual that
+    the oracle confirms, in about the iterations of the FP64 solve (a wrong term would not converge,
+    or only after many more; the 16-bit fat links of mode 3 leave the base system some)."""
+    kq = gpu
+    lat, shifts = (24, 16, 16, 18), (0.05, 0.1, 0.3, 1.0)
+    print("case", mode, links, flush=True)
+    fat, lng = _load(kq, lat, u3=links == "u3")
+    b = [kq.gen_source(lat, 0, seed=70 + r) for r in range(2)]
+    _, rep1 = _solve(kq, b, 1, 2, shifts)
+    x, rep = _solve(kq, b, mode, 8, shifts)
+    for r in range(2):
+        for k, s in enumerate(shifts):
+            v = x[r * len(shifts) + k]
+            res = b[r] - (s * v - oracle.mdaggm(fat, lng, v, lat, 0))
+            assert np.linalg.norm(res) <= 1.01e-10 * np.linalg.norm(b[r]), (r, k)
+        assert rep[r].iter <= (2 if mode == 3 else 1.2) * rep1[r].iter + 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,links", [(8, "general"), (4, "general"), (4, "u3")])
+@pytest.mark.parametrize("lat", [(6, 5, 4, 3), (10, 6, 6, 6)])
+def test_host_layout_in_every_link_format(gpu, lat, prec, links):
+    """The operator and every blocking of the hopping term on the caller's arrays, in the long-link
+    formats that the other tests of these kernels do not load: 18 reals, and FP32 in 12 reals with a
+    complex scale. Bounds of the path: 1e-13 (FP64), 1e-5 (FP32)."""
+    kq = gpu
+    dt, tol = (np.float64, 1e-13) if prec == 8 else (np.float32, 1e-5)
+    fat, lng = _load(kq, lat, u3=links == "u3", general=links == "general", prec=prec)
+    fat, lng = (a.astype(dt).astype(np.float64) for a in (fat, lng))
+    src = np.stack([kq.gen_source(lat, 0, seed=80 + r) for r in range(9)]).astype(dt)
+    want = np.stack([oracle.dslash(fat, lng, v.astype(np.float64), lat, 1) for v in src])
+    for nr in (1, 2, 3, 4, 8):
+        print("case", lat, prec, links, nr, flush=True)
+        out = np.full_like(src, np.nan)
+        assert kq.dslash_batched(src, out, 1, 0, nr, 256) == 0, kq.last_error()
+        for r in range(len(src)):
+            assert rel_err(out[r], want[r]) <= tol, r
+    v, out = np.ascontiguousarray(src[0]), np.empty_like(src[0])
+    assert kq.mdaggm(v, out, 0, 0.07, 0) == 0, kq.last_error()
+    assert rel_err(out, 0.07 * v.astype(np.float64) - oracle.mdaggm(fat, lng, v.astype(np.float64), lat, 0)) <= tol
