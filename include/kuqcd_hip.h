@@ -256,6 +256,10 @@ KQ_API int kq_device_count(void);
 /* host check of the fast division used by the kernels' index math: returns
  * the number of n in [0, n_max) with n / d != the fast quotient */
 KQ_API long kq_selftest_fastdiv(uint32_t d, uint32_t n_max);
+/* the kernel that a hopping term of the solvers and of the mixed modes runs on: 0 one thread per site,
+ * 1 rows staged in LDS, 8, 4 or 2 split over that many waves per 64 sites. fp64: FP64 vectors;
+ * small_long: 16-bit long links in 28 or 32 bytes; nrhs vectors in blocks of nr, nt threads per block */
+KQ_API int kq_selftest_hop_kernel(const int lat[4], int fp64, int small_long, int nrhs, int nr, int nt);
 /* host check of the reliable-update fold rule of the mixed solver: 1 if the fold adds the
  * low-precision update of shift k to its FP64 solution, for a system with max_term shifts still
  * iterating and the host's divergence flag `discard` */

@@ -196,6 +196,12 @@ def neighbour_index(lat, q: int, s: int, mu: int, h: int) -> int:
     return L.lib().kq_neighbour_index(la, q, s, mu, h)
 
 
+def hop_kernel(lat, nrhs: int, nr: int, nt: int, fp64: bool, small_long: bool = False) -> int:
+    """The kernel of a hopping term (kq_selftest_hop_kernel): 0 one thread per site, 1 staged, 8/4/2 split."""
+    la = (C.c_int * 4)(*[int(v) for v in lat])
+    return L.lib().kq_selftest_hop_kernel(la, fp64, small_long, nrhs, nr, nt)
+
+
 def load_gauge_pair(fat: np.ndarray, lng: np.ndarray, lat, prec=L.KUQCD_DOUBLE, order=L.KUQCD_NORMAL_ORDER) -> None:
     """Load fat then long links (the reference call order); raises on error."""
     dt = np.float64 if prec == L.KUQCD_DOUBLE else np.float32

@@ -132,4 +132,19 @@ inline int dslash_split_waves(bool fp64, const Geom &g, int nrhs, int nr)
     return nr == 8 && !stage_lattice(g) ? 4 : 0;
 }
 
+// The kernel of one hopping term on colour planes: waves per 64 sites of the split one (8, 4 or 2),
+// kHopStaged for the one with rows in LDS, kHopSingle for one thread per site. small_long: long links
+// of fewer than 40 bytes (LinkH12, LinkH12C). Their blocks of 8 on more than 48 K sites take 2 waves of
+// 8 hops, whose 12.7 KB of LDS let all workgroups of a middle-sized lattice run at once (16^3x32 35 us
+// with 4 waves, 30 with 2; 24^4 74 and 73.5, 48^4 1093 and 1040; but 16^4 17.6 and 24); the general
+// 16-bit links (LinkH, 40 bytes) keep 4, which is all that was measured for them.
+constexpr int kHopSingle = 0, kHopStaged = 1;
+inline int hop_kernel(bool fp64, bool small_long, const Geom &g, int nrhs, int nr, int nt)
+{
+    const int waves = dslash_split_waves(fp64, g, nrhs, nr);
+    if (waves > 0)
+        return waves == 4 && nr == 8 && small_long && g.Vh > 49152u ? 2 : waves;
+    return dslash_staged(g, nr, nt) ? kHopStaged : kHopSingle;
+}
+
 }  // namespace kq

@@ -737,7 +737,7 @@ static size_t cap_lds_bytes(int cap, int nt)
 }
 
 template <class LF, class LL, typename SR, int NR, int EPI>
-static void launch_nt(const DslashArgs<LF, LL, SR> &a, int nt, int cap, hipStream_t st)
+static void launch_nt(const DslashArgs<LF, LL, SR> &a, int kernel, int nt, int cap, hipStream_t st)
 {
     const int nact_max = a.nrhs;
     const dim3 grid(a.nblk, (nact_max + NR - 1) / NR);
@@ -747,7 +747,7 @@ static void launch_nt(const DslashArgs<LF, LL, SR> &a, int nt, int cap, hipStrea
         // nt + 6 Lx/2 sites of the workgroup's rows and their +-3 y-neighbour rows; an occupancy
         // cap adds dynamic LDS only beyond that
         const size_t sb = (size_t)NR * 3 * (256 + 6 * kStageLxh) * sizeof(c2_t<SR>);
-        if (dslash_staged(a.g, NR, nt) && sb + 1024 <= (size_t)lds_block_bytes()) {
+        if (kernel == kHopStaged && sb + 1024 <= (size_t)lds_block_bytes()) {
             hipLaunchKernelGGL((k_dslash_staged<LF, LL, SR, NR, EPI>), grid, dim3(256), lds > sb ? lds - sb : 0,
                                st, a);
             KQ_HIP_CHECK(hipGetLastError());
@@ -785,29 +785,28 @@ template <class LF, class LL, typename SR, int NR>
 static uint32_t launch_epi(DslashArgs<LF, LL, SR> a, int epi, int nt, int cap, hipStream_t st)
 {
     constexpr bool kDouble = std::is_same<SR, double>::value;
+    constexpr bool kSmallLong = LL::kBytes < 40;
+    const int kernel = hop_kernel(kDouble, kSmallLong, a.g, a.nrhs, NR, nt);
+    if (kernel > kHopStaged)
+        a.nblk = dslash_grid(a.g.Vh, 64);
     if constexpr (!kDouble || NR <= 2) {
         constexpr int S = NR <= 2 ? 8 : 4;
-        if (dslash_split_waves(kDouble, a.g, a.nrhs, NR) == S) {
-            a.nblk = dslash_grid(a.g.Vh, 64);
-            // 16-bit long links in blocks of 8 on more than 48 K sites: 2 waves of 8 hops, whose
-            // 24.8 KB of LDS let all workgroups of a middle-sized lattice run at once (16^3x32
-            // 35 us with 4 waves, 30 with 2; 24^4 74 and 73.5, 48^4 1093 and 1040; but 16^4 17.6
-            // and 24)
-            if constexpr (NR == 8 && LL::kBytes < 40) {
-                if (a.g.Vh > 49152u) {
-                    launch_split<LF, LL, SR, NR, 2>(a, epi, st);
-                    return a.nblk;
-                }
-            }
+        if (kernel == S) {
             launch_split<LF, LL, SR, NR, S>(a, epi, st);
+            return a.nblk;
+        }
+    }
+    if constexpr (NR == 8 && kSmallLong) {
+        if (kernel == 2) {
+            launch_split<LF, LL, SR, NR, 2>(a, epi, st);
             return a.nblk;
         }
     }
     a.nblk = dslash_grid(a.g.Vh, nt);
     if (epi == EPI_STORE)
-        launch_nt<LF, LL, SR, NR, EPI_STORE>(a, nt, cap, st);
+        launch_nt<LF, LL, SR, NR, EPI_STORE>(a, kernel, nt, cap, st);
     else
-        launch_nt<LF, LL, SR, NR, EPI_AXMY_DOT>(a, nt, cap, st);
+        launch_nt<LF, LL, SR, NR, EPI_AXMY_DOT>(a, kernel, nt, cap, st);
     return a.nblk;
 }
 

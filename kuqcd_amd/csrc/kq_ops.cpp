@@ -513,6 +513,11 @@ long kq_selftest_fastdiv(uint32_t d, uint32_t n_max)
     return bad;
 }
 
+int kq_selftest_hop_kernel(const int lat[4], int fp64, int small_long, int nrhs, int nr, int nt)
+{
+    return lat == nullptr ? -1 : hop_kernel(fp64 != 0, small_long != 0, make_geom(lat), nrhs, nr, nt);
+}
+
 int kq_selftest_fold_keeps(int discard, int k, int max_term)
 {
     return fold_keeps(discard, k, max_term) ? 1 : 0;

@@ -1,9 +1,13 @@
 """Which kernel a hopping term runs on, and that what may not depend on that choice does not."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 import oracle
-from conftest import rel_err
+from conftest import ROOT, rel_err
 
 
 def _load(kq, lat, u3=False, general=False, prec=8):
@@ -64,6 +68,7 @@ def test_split_term_with_two_waves_in_solves(gpu, mode, links):
     lat, shifts = (24, 16, 16, 18), (0.05, 0.1, 0.3, 1.0)
     print("case", mode, links, flush=True)
     fat, lng = _load(kq, lat, u3=links == "u3")
+    assert kq.hop_kernel(lat, 8, 8, 256, fp64=False, small_long=True) == 2
     b = [kq.gen_source(lat, 0, seed=70 + r) for r in range(2)]
     _, rep1 = _solve(kq, b, 1, 2, shifts)
     x, rep = _solve(kq, b, mode, 8, shifts)
@@ -97,3 +102,84 @@ def test_host_layout_in_every_link_format(gpu, lat, prec, links):
     v, out = np.ascontiguousarray(src[0]), np.empty_like(src[0])
     assert kq.mdaggm(v, out, 0, 0.07, 0) == 0, kq.last_error()
     assert rel_err(out, 0.07 * v.astype(np.float64) - oracle.mdaggm(fat, lng, v.astype(np.float64), lat, 0)) <= tol
+
+
+# Lx = 32 and more than 98304 sites of one parity: blocks of any size are staged. One workgroup per (x, y) plane
+# with more staged rows than the plane has (the y wrap repeats rows), and two per plane.
+STAGED = [(32, 16, 16, 32), (32, 32, 16, 16)]
+MIXED_NRS = (2, 3, 4, 8)
+
+
+def test_the_staged_kernel_is_the_one_tested(kq):
+    for lat in STAGED:
+        for nr in MIXED_NRS:
+            for small in (False, True):
+                assert kq.hop_kernel(lat, 5, nr, 256, fp64=False, small_long=small) == 1
+        assert kq.hop_kernel(lat, 5, 1, 256, fp64=False) == 0
+        assert kq.hop_kernel(lat, 2, 2, 256, fp64=True) == 1 and kq.hop_kernel(lat, 2, 1, 256, fp64=True) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lat", STAGED)
+@pytest.mark.parametrize("mode,tol", [(2, 1e-5), (3, 3e-3), (4, 5e-4)])
+def test_staged_rows_of_the_mixed_terms(gpu, lat, mode, tol):
+    """Blocks with their rows in LDS against single vectors (one thread per site, the same arithmetic to
+    rounding) and the oracle, with a padded last block."""
+    kq = gpu
+    fat, lng = _load(kq, lat)
+    src = np.stack([kq.gen_source(lat, 0, seed=200 + r) for r in range(5)])
+    single = np.empty_like(src)
+    for r in range(5):
+        assert kq.dslash(np.ascontiguousarray(src[r]), single[r], 1, mode) == 0
+    for r in (0, 4):
+        assert rel_err(single[r], oracle.dslash(fat, lng, src[r], lat, 1)) <= tol
+    for nr in MIXED_NRS:
+        print("case", lat, mode, nr, flush=True)
+        out = np.full_like(src, np.nan)
+        assert kq.dslash_batched(src, out, 1, mode, nr, 256) == 0, kq.last_error()
+        assert rel_err(out, single) <= 1e-6, nr
+
+
+_UNSTAGED = """
+import sys
+sys.path[:0] = [{root!r}, {tests!r}]
+import numpy as np
+import kuqcd_amd.api as kq
+import test_gpu_kernel_choice as T
+kq.set_verbosity(0)
+assert kq.kuqcd_init() == kq.KUQCD_SUCCESS
+np.save({path!r}, T.staged_results(kq, {lat!r}))
+kq.kuqcd_gauge_free()
+kq.kuqcd_end()
+"""
+
+
+def staged_results(kq, lat):
+    """Everything that the staged kernel computes on this lattice: the mixed terms in blocks, and an FP64
+    solve of two systems as pairs in workgroups of 256."""
+    _load(kq, lat)
+    src = np.stack([kq.gen_source(lat, 0, seed=300 + r) for r in range(5)])
+    res = []
+    for mode in (2, 3, 4):
+        for nr in MIXED_NRS:
+            print("case", lat, mode, nr, flush=True)
+            out = np.empty_like(src)
+            assert kq.dslash_batched(src, out, 1, mode, nr, 256) == 0, kq.last_error()
+            res.append(out)
+    x, rep = _solve(kq, [src[0], src[1]], 1, 2, nt=256)
+    res.append(np.stack(x))
+    return np.concatenate([v.reshape(-1) for v in res] + [np.array(rep[r].true_rel_res) for r in range(2)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lat", STAGED)
+def test_staged_rows_bitwise_equal_to_unstaged(gpu, tmp_path, lat):
+    """The staged kernel (with its link prefetch for 4 or more FP32 vectors) adds in the unstaged one's
+    order: the bits are those of a process with the staging switched off."""
+    out = staged_results(gpu, lat)
+    path = str(tmp_path / "unstaged.npy")
+    code = _UNSTAGED.format(root=str(ROOT), tests=str(ROOT / "tests"), path=path, lat=lat)
+    r = subprocess.run([sys.executable, "-c", code], env={**os.environ, "KQ_STAGE": "0"}, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert np.array_equal(out, np.load(path))
