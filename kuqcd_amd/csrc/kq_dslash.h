@@ -57,8 +57,8 @@ uint32_t launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStr
 
 // D p with p = z r + a p formed on the way, for one system that is deferred or has one live shift
 // (k_dslash_split_p): a.src holds p before the update, pnew takes it after the update, part the npart
-// partial sums of |r|^2; x, if not deferred, takes x - beta p. Does nothing unless st->run is set. Only where dslash_split_waves(.., 1, 1)
-// is 8.
+// partial sums of |r|^2; x, if not deferred, takes x - beta p. Does nothing unless st->run is set. Only
+// for one system on a lattice whose split term has 8 waves; refuses others.
 template <typename S> struct CgmState;
 template <class LF, class LL, typename SR>
 void launch_dslash_p(DslashArgs<LF, LL, SR> a, CgmState<SR> *st, const c2_t<SR> *r, Vec<SR> pnew, Vec<SR> x,
@@ -123,11 +123,12 @@ inline bool dslash_staged(const Geom &g, int nr, int nt)
 // verification, whose results are the same in every process (repro_nt). Two or more FP64 vectors
 // run faster as pairs on either form (two vectors in single blocks -> a pair: 16^4 20.7 -> 13.1 us, 24^4
 // 115 -> 65, 32^4 354 -> 193, 48^4 1948 -> 1077; only at 8^4 4.4 -> 5.0), so the rule follows those.
+constexpr uint32_t kSplitSites64 = 49152, kSplitSites32 = 98304;
 inline int dslash_split_waves(bool fp64, const Geom &g, int nrhs, int nr)
 {
     if (fp64)
-        return nr <= 2 && (uint64_t)g.Vh * (uint64_t)((nrhs + 1) / 2) <= 49152u ? 8 : 0;
-    if ((uint64_t)g.Vh * (uint64_t)((nrhs + nr - 1) / nr) <= 98304u)
+        return nr <= 2 && (uint64_t)g.Vh * (uint64_t)((nrhs + 1) / 2) <= kSplitSites64 ? 8 : 0;
+    if ((uint64_t)g.Vh * (uint64_t)((nrhs + nr - 1) / nr) <= kSplitSites32)
         return nr <= 2 ? 8 : 4;
     return nr == 8 && !stage_lattice(g) ? 4 : 0;
 }

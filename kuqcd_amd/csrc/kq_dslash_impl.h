@@ -600,6 +600,8 @@ template <class LF, class LL, typename SR>
 void launch_dslash_p(DslashArgs<LF, LL, SR> a, CgmState<SR> *st, const c2_t<SR> *r, Vec<SR> pnew, Vec<SR> x,
                      const double *part, uint32_t npart, double *shist, hipStream_t stream)
 {
+    if (a.nrhs != 1 || dslash_split_waves(std::is_same<SR, double>::value, a.g, 1, 1) != 8)
+        throw std::logic_error("dslash: the direction update needs one system and the split term of 8 waves");
     a.nblk = dslash_grid(a.g.Vh, 64);
     hipLaunchKernelGGL((k_dslash_split_p<LF, LL, SR>), dim3(a.nblk + 1), dim3(512), 0, stream, a, st, r, pnew, x,
                        part, npart, shist);

@@ -360,9 +360,9 @@ public:
     // 64 sites per CU. Reference solves with 4 shifts, separate update -> in the hopping term: FP64
     // 8^4 3.52 -> 3.24 ms, 12^3x8 4.05 -> 3.49, 12^4 4.32 -> 3.89, 16x12^3 4.57 -> 4.37, 16^2x12^2 (18432
     // sites) 5.91 -> 5.90, 16^4 7.00 -> 7.16; FP32 8^4 2.22 -> 1.92, 12^4 2.36 -> 1.97, 16x12^3
-    // 2.45 -> 2.09, 16^2x12^2 2.57 -> 2.51, 16^4 2.82 -> 2.88. (Where the split term is used with 8
-    // waves in both precisions, which the launch relies on.)
+    // 2.45 -> 2.09, 16^2x12^2 2.57 -> 2.51, 16^4 2.82 -> 2.88.
     static constexpr uint32_t kHopDirectionSites = 16384;
+    static_assert(kHopDirectionSites <= kSplitSites64 && kHopDirectionSites <= kSplitSites32, "launch_dslash_p");
 
     // Register a system; it starts at the next run() step. shifts: reference
     // convention (absolute shifts[0], shifts[k>=1] relative to it); tolk: absolute
@@ -378,6 +378,9 @@ public:
             throw std::runtime_error("solver: vector pool exhausted");
         if (x0 && (!reliable_ || nshift != 1))
             throw std::invalid_argument("solver: an initial guess needs the reliable single-shift mode");
+        // the hopping terms update only p_0 and x_0 of a system that is not deferred (launch_dslash_p)
+        if (p1_ && nshift > 1 && dslot_used_ >= ndslot_)
+            throw std::logic_error("solver: several shifts without deferred updates on a small lattice");
         const int sys = nsys_++;
         off_h_[sys] = pool_used_ * n3_;
         pool_used_ += nshift;

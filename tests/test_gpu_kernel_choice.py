@@ -119,6 +119,15 @@ def test_the_staged_kernel_is_the_one_tested(kq):
         assert kq.hop_kernel(lat, 2, 2, 256, fp64=True) == 1 and kq.hop_kernel(lat, 2, 1, 256, fp64=True) == 0
 
 
+@pytest.mark.parametrize("lat", [(2, 1, 1, 1), (6, 5, 4, 3), (8, 8, 8, 8), (32, 32, 16, 2), (16, 16, 16, 8)])
+def test_lattices_of_the_direction_update_take_eight_waves(kq, lat):
+    """Up to 16384 sites of one parity the solvers of one system update its direction inside the hopping
+    term, whose kernel has 8 waves per 64 sites."""
+    for fp64 in (False, True):
+        for nt in (64, 256):
+            assert kq.hop_kernel(lat, 1, 1, nt, fp64=fp64) == 8
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("lat", STAGED)
 @pytest.mark.parametrize("mode,tol", [(2, 1e-5), (3, 3e-3), (4, 5e-4)])
