@@ -44,6 +44,16 @@ constexpr int kMinDslashNT = 64;
 // workgroups of 64; 24^4 62 against 59.5); above, 256 is 1-3 % faster (32^4 176 against 181 us).
 inline int repro_nt(uint32_t Vh) { return Vh < 200000u ? 64 : 256; }
 
+// Blockings and block sizes that exist; others are refused on every lattice, also where the kernel
+// that runs has a block size of its own
+inline void check_blocking(int nr, int nt)
+{
+    if (nr != 1 && nr != 2 && nr != 3 && nr != 4 && nr != 8)
+        throw std::runtime_error("dslash: unsupported RHS blocking " + std::to_string(nr));
+    if (nt != 64 && nt != 128 && nt != 256)
+        throw std::runtime_error("dslash: unsupported block size " + std::to_string(nt));
+}
+
 // Launch D over all sites of parity dst_parity for every right-hand side.
 // nr = right-hand sides handled per thread (1, 2, 3, 4 or 8), nt = threads per block,
 // cap = at most this many wavefronts per SIMD (0: as many as the registers allow). The

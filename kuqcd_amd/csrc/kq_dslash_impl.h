@@ -763,11 +763,9 @@ static void launch_nt(const DslashArgs<LF, LL, SR> &a, int kernel, int nt, int c
     case 128:
         hipLaunchKernelGGL((k_dslash<LF, LL, SR, NR, EPI, 128>), grid, dim3(128), lds, st, a);
         break;
-    case 256:
+    default:
         hipLaunchKernelGGL((k_dslash<LF, LL, SR, NR, EPI, 256>), grid, dim3(256), lds, st, a);
         break;
-    default:
-        throw std::runtime_error("dslash: unsupported block size " + std::to_string(nt));
     }
     KQ_HIP_CHECK(hipGetLastError());
 }
@@ -912,6 +910,7 @@ uint32_t launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStr
 {
     if (a.g.Vh == 0 || a.nrhs <= 0)
         return 0;
+    check_blocking(nr, nt);
     switch (nr) {
     case 1:
         return launch_epi<LF, LL, SR, 1>(a, epi, nt, cap, st);
@@ -921,10 +920,8 @@ uint32_t launch_dslash(DslashArgs<LF, LL, SR> a, int epi, int nr, int nt, hipStr
         return launch_epi<LF, LL, SR, 3>(a, epi, nt, cap, st);
     case 4:
         return launch_epi<LF, LL, SR, 4>(a, epi, nt, cap, st);
-    case 8:
-        return launch_epi<LF, LL, SR, 8>(a, epi, nt, cap, st);
     default:
-        throw std::runtime_error("dslash: unsupported RHS blocking " + std::to_string(nr));
+        return launch_epi<LF, LL, SR, 8>(a, epi, nt, cap, st);
     }
 }
 

@@ -675,6 +675,10 @@ KuQCDStatus solve_extended(int slot, int nrhs, void **x, void **b, KuQCDInvertPa
         set_error("no preconditioner weights: call kq_ptnet_set_weights or kq_learned_train first");
         return KUQCD_ERR_UNSUPPORTED;
     }
+    // before any work: a launch that refuses its blocking while a chunk is captured leaves the stream
+    // in the capture
+    if (o.mode == KQ_MODE_FP64 || o.mode == KQ_MODE_REFERENCE || is_mixed_mode(o.mode))
+        check_blocking(o.nr > 0 ? o.nr : 1, o.nt > 0 ? o.nt : 64);
     Problem P;
     P.slot = slot;
     P.parity = (p.matpc_type == KUQCD_EVEN_EVEN) ? 0 : 1;
