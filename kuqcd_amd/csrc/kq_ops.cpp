@@ -271,13 +271,15 @@ std::pair<int, int> tuned_launch(int slot, int mode, int nrhs)
     static const int kNr[5] = {1, 2, 3, 4, 8}, kNt[3] = {64, 128, 256}, kCap[5] = {0, 5, 4, 3, 2};
     if (small_lattice(g)) {
         // Groups of a small lattice share the chip, so the blockings are timed on all nrhs systems
-        // (8 FP32 systems at 8^4: one group of 8 11.5 us, 8 groups of 1 about half), without caps
+        // (8 FP32 systems at 8^4: one group of 8 11.5 us, 8 groups of 1 about half), without caps; on at
+        // most 32, which fill the chip several times over: the vectors timed are allocated
+        const int ntime = std::min(std::max(nrhs, 1), 32);
         double best = 1e30, bs = 0.0;
         std::pair<int, int> pick{1, dslash_staged(g, 2, 256) ? 256 : 64};
         for (int nr : kNr) {
             if (nr > 1 && (nr >= 2 * nrhs || (mode == KQ_MODE_FP64 && nr > 2)))
                 continue;
-            const double t = time_mode(slot, mode, nrhs, nr, pick.second, 6, &bs);
+            const double t = time_mode(slot, mode, ntime, nr, pick.second, 6, &bs);
             if (t < best) {
                 best = t;
                 pick.first = nr;

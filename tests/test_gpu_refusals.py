@@ -1,4 +1,6 @@
 """Launch options that are refused, or accepted, whatever kernel the lattice runs on."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -32,3 +34,18 @@ def test_blocking_options_that_no_kernel_has(gpu, lat):
         opt = kq.default_options(mode=mode, rel_tol=1e-6, nr=1, nt=128, verbose=0)
         assert kq.solve_batched(x, b, p, opt)[0] == 0, kq.last_error()
         assert kq.bench_dslash(mode, 1, 1, 128, 1)[0] == 0, kq.last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lat", [(6, 5, 4, 3), (16, 16, 16, 16)])
+def test_autotuning_for_any_number_of_vectors(gpu, lat):
+    """The blocking is timed on blocks, not on the caller's number of vectors: none, and more than the
+    card holds or a launch has blocks for, get an answer on any lattice."""
+    kq = gpu
+    _load(kq, lat)
+    for mode in (1, 2):
+        for nrhs in (0, 1, 1000000):
+            print("case", lat, mode, nrhs, flush=True)
+            nr, nt = C.c_int(), C.c_int()
+            assert kq.L.lib().kq_autotune_dslash(mode, nrhs, C.byref(nr), C.byref(nt)) == 0, kq.last_error()
+            assert nr.value in ((1, 2) if mode == 1 else (1, 2, 3, 4, 8)) and nt.value in (64, 128, 256)
