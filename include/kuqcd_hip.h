@@ -106,7 +106,8 @@ KQ_API KuQCDStatus kq_mdaggm(const void *src, void *dst, int parity, double sigm
 /* No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): kq_mdaggm in
  * KQ_MODE_REFERENCE (the loaded gauge's precision) without any allocation. src and dst are
- * device memory in the reference host layout (Vh*6 reals each, not overlapping). The intermediate
+ * device memory in the reference host layout (Vh*6 reals each, not overlapping), of the library's
+ * GPU or of one whose memory it has access to. The intermediate
  * D src is kept in the library's scratch for this call, one static device
  * array of KQ_NOALLOC_SCRATCH_BYTES per GPU (the FP64 operator up to 32^4 sites); a larger
  * lattice returns KUQCD_ERR_INVALID_PARAM. The work is queued on the library stream and not

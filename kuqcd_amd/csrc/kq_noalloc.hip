@@ -88,7 +88,8 @@ extern "C" KuQCDStatus kq_mdaggm_noalloc(const void *src, void *dst, int parity,
             return KUQCD_ERR_INVALID_PARAM;
         }
         const size_t bytes = real * 6 * (size_t)g.Vh;
-        if (!on_this_device(src) || !on_this_device(dst)) {
+        // another GPU's memory too: its owner has made it accessible to this one
+        if (!on_a_device(src) || !on_a_device(dst)) {
             set_error("kq_mdaggm_noalloc: src and dst must be device memory (kq_device_alloc / hipMalloc)");
             return KUQCD_ERR_INVALID_PARAM;
         }

@@ -24,7 +24,8 @@ void copy_to_host(void *h, const void *d, size_t bytes, hipStream_t st);
 // bytes from h (pageable host, pinned host or device memory) to device memory d, likewise
 void copy_from_host(void *d, const void *h, size_t bytes, hipStream_t st);
 
-// true for device memory of the current GPU (not host, managed or another GPU's memory)
+// true for device memory of any GPU (not host or managed memory), and of the current one
+bool on_a_device(const void *p);
 bool on_this_device(const void *p);
 // true where kernels can read or write a caller's array of `bytes` bytes with elements of `elem` bytes
 // themselves: aligned, in device memory of the current GPU and inside one allocation. Other arrays

@@ -154,15 +154,27 @@ bool in_place(const void *p, size_t bytes, size_t elem)
     return o <= size && bytes <= size - o;
 }
 
-bool on_this_device(const void *p)
+static bool device_memory(const void *p, int &device)
 {
     hipPointerAttribute_t a{};
-    int dev = 0;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return a.type == hipMemoryTypeDevice && hipGetDevice(&dev) == hipSuccess && a.device == dev;
+    device = a.device;
+    return a.type == hipMemoryTypeDevice;
+}
+
+bool on_a_device(const void *p)
+{
+    int at = 0;
+    return device_memory(p, at);
+}
+
+bool on_this_device(const void *p)
+{
+    int at = 0, dev = 0;
+    return device_memory(p, at) && hipGetDevice(&dev) == hipSuccess && at == dev;
 }
 
 void copy_to_host(void *h, const void *d, size_t bytes, hipStream_t st)
