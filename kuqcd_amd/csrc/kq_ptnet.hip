@@ -62,6 +62,13 @@ template <class T> __device__ __forceinline__ const T &first_arg()
 {
     return *(const T *)__builtin_amdgcn_kernarg_segment_ptr();
 }
+template <class F> struct FirstParam;
+template <class T, class... R> struct FirstParam<void (*)(T, R...)> {
+    using type = T;
+};
+// to stand beside each kernel that calls first_arg<T>(): T is its first parameter
+#define KQ_FIRST_ARG(T, ...) \
+    static_assert(std::is_same<FirstParam<decltype(&__VA_ARGS__)>::type, T>::value, "first_arg reads the first parameter")
 
 // The links of the four taps: every load is issued before any is used
 template <class LF, class LL>
@@ -216,6 +223,7 @@ __global__ void __launch_bounds__(kNT) k_pt_layer1(const PtLayerArgs a, LF fat, 
         a.out16[(size_t)w * a.g.Vh + sl] = u;
     }
 }
+KQ_FIRST_ARG(PtLayerArgs, k_pt_layer1<LinkF, LinkF>);
 
 // acc += sum over direction mu's taps of T_t( sum_c w2[c][t] in_c ). With bfloat16 channels one
 // 16-byte load brings the four channels of one colour, and the 12 gathers and the link loads are all
@@ -325,6 +333,7 @@ k_pt_layer2(const PtLayerArgs a, LF fat, LL lng)
         }
     }
 }
+KQ_FIRST_ARG(PtLayerArgs, k_pt_layer2<LinkF, LinkF, true>);
 
 // P[c][t] = sum over sites y of parity qo of <(T_t in)(y), b_c(y)> for the two (in, b) pairs of a
 // gradient (blockIdx.y); part[pair][blk][c*16 + t] (complex, FP64).
@@ -396,6 +405,7 @@ __global__ void __launch_bounds__(kNT) k_pt_wgrad(Geom g, int qo, LF fat, LL lng
         part[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * J + lane] = o;
     }
 }
+KQ_FIRST_ARG(Geom, k_pt_wgrad<LinkF, LinkF>);
 
 // out[y*gridDim.x + j] = sum over blocks b of part[(y*nblk + b)*stride + j], j = blockIdx.x,
 // y = blockIdx.y < 2; fixed summation order. For y = 2, j < 2: the sums over the nblk2 entries of
