@@ -56,6 +56,22 @@ Pinned<double> &host_scratch()
     return *c.scratch;
 }
 
+void settle() noexcept
+{
+    Context &c = ctx();
+    if (!c.device_ready)
+        return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c.stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+        hipGraph_t g = nullptr;
+        if (hipStreamEndCapture(c.stream, &g) == hipSuccess && g != nullptr)
+            (void)hipGraphDestroy(g);
+    }
+    (void)hipStreamSynchronize(c.stream);
+    (void)hipStreamSynchronize(c.copy_stream);
+    (void)hipGetLastError();
+}
+
 void log_info(const char *fmt, ...)
 {
     if (ctx().verbosity <= 0)
@@ -459,12 +475,15 @@ template <typename Fn> static KuQCDStatus guarded(Fn fn)
     try {
         return fn();
     } catch (const std::bad_alloc &) {
+        settle();
         set_error("out of memory");
         return KUQCD_ERR_NO_MEMORY;
     } catch (const std::exception &e) {
+        settle();
         set_error(e.what());
         return KUQCD_ERR_UNKNOWN_ERROR;
     } catch (...) {
+        settle();
         set_error("unknown exception");
         return KUQCD_ERR_UNKNOWN_ERROR;
     }

@@ -80,6 +80,9 @@ struct Context {
 
 Context &ctx();
 void ensure_device();
+// After an error: ends a capture that the failed call began and waits for the work it queued, since
+// kernels read and write the caller's arrays and the call returns before the caller knows of them
+void settle() noexcept;
 constexpr size_t kScratchDoubles = 2048;
 Pinned<double> &host_scratch();
 inline int slot_index(int order, int prec) { return (order == KUQCD_BATCH_ORDER ? 0 : 2) + (prec == KUQCD_DOUBLE ? 1 : 0); }

@@ -550,12 +550,15 @@ template <class Fn> KuQCDStatus guarded(Fn fn)
     try {
         return fn();
     } catch (const std::bad_alloc &) {
+        settle();
         set_error("out of memory");
         return KUQCD_ERR_NO_MEMORY;
     } catch (const std::invalid_argument &e) {
+        settle();
         set_error(e.what());
         return KUQCD_ERR_INVALID_PARAM;
     } catch (const std::exception &e) {
+        settle();
         set_error(e.what());
         return KUQCD_ERR_UNKNOWN_ERROR;
     }

@@ -353,9 +353,11 @@ KuQCDStatus kq_dslash(const void *src, void *dst, int dst_parity, int mode)
     try {
         return apply(1, src, dst, dst_parity, mode, 1, 256, false, 0.0);
     } catch (const std::bad_alloc &) {
+        settle();
         set_error("out of memory");
         return KUQCD_ERR_NO_MEMORY;
     } catch (const std::exception &e) {
+        settle();
         set_error(e.what());
         return KUQCD_ERR_UNKNOWN_ERROR;
     }
@@ -366,9 +368,11 @@ KuQCDStatus kq_dslash_batched(int nrhs, const void *src, void *dst, int dst_pari
     try {
         return apply(nrhs, src, dst, dst_parity, mode, nr, nt, false, 0.0);
     } catch (const std::bad_alloc &) {
+        settle();
         set_error("out of memory");
         return KUQCD_ERR_NO_MEMORY;
     } catch (const std::exception &e) {
+        settle();
         set_error(e.what());
         return KUQCD_ERR_UNKNOWN_ERROR;
     }
@@ -379,9 +383,11 @@ KuQCDStatus kq_mdaggm(const void *src, void *dst, int parity, double sigma, int 
     try {
         return apply(1, src, dst, parity, mode, 1, 256, true, sigma);
     } catch (const std::bad_alloc &) {
+        settle();
         set_error("out of memory");
         return KUQCD_ERR_NO_MEMORY;
     } catch (const std::exception &e) {
+        settle();
         set_error(e.what());
         return KUQCD_ERR_UNKNOWN_ERROR;
     }

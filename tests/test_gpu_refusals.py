@@ -120,3 +120,76 @@ def test_arrays_on_another_gpu_are_accepted(gpu, tmp_path):
     r = subprocess.run([sys.executable, "-c", _PEER.format(root=str(ROOT), shim=str(shim))], env=dict(os.environ),
                        capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+_FAILING_COPY = """
+#define __HIP_PLATFORM_AMD__ 1
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+int armed = 0, failed = 0;
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
+{
+    static hipError_t (*real)(void *, const void *, size_t, hipMemcpyKind, hipStream_t);
+    if (!real)
+        real = dlsym(dlopen("/opt/rocm/lib/libamdhip64.so.7", RTLD_LAZY), "hipMemcpyAsync");
+    if (!real)
+        return hipErrorNotFound;
+    if (armed && k == hipMemcpyDeviceToHost && n >= (1u << 20) && --armed == 0) {
+        ++failed;
+        return hipErrorOutOfMemory;
+    }
+    return real(d, s, n, k, st);
+}
+"""
+
+_AFTER_ERROR = """
+import ctypes as C, sys
+sys.path.insert(0, {root!r})
+shim = C.CDLL({shim!r}, mode=C.RTLD_GLOBAL)
+import numpy as np
+import kuqcd_amd.api as kq
+hip = C.CDLL("/opt/rocm/lib/libamdhip64.so.7")
+kq.set_verbosity(0)
+assert kq.kuqcd_init() == kq.KUQCD_SUCCESS
+lat, ns = (32, 32, 32, 32), 32
+fat, lng = kq.gen_gauge(lat, kind=kq.KQ_GEN_WEAK, eps=0.3)
+kq.load_gauge_pair(fat, lng, lat)
+L, b = kq.L.lib(), kq.gen_source(lat, 0, seed=9)
+bd, xd = L.kq_device_alloc(b.nbytes), [L.kq_device_alloc(b.nbytes) for _ in range(ns - 2)]
+assert L.kq_memcpy(bd, b.ctypes.data, b.nbytes) == 0
+first, last, got, want = (np.zeros_like(b) for _ in range(4))
+xp, bp = (C.c_void_p * ns)(first.ctypes.data, *xd, last.ctypes.data), (C.c_void_p * 1)(bd)
+p = kq.InvertParam(shifts=np.array([[0.1] * ns]), tol=1.0, max_iter=2, num_shift=ns)
+opt = kq.default_options(mode=1, rel_tol=1e-9, refine=0, verbose=0)
+def solve():
+    return L.kq_solve_multishift_batched(1, xp, bp, C.byref(p.struct()), C.byref(opt), None)
+assert solve() == 0, kq.last_error()
+assert L.kq_memcpy(want.ctypes.data, xd[-1], want.nbytes) == 0 and np.any(want)
+zero = np.zeros_like(b)
+for x in xd:
+    assert L.kq_memcpy(x, zero.ctypes.data, zero.nbytes) == 0
+# the first solution goes to the host in chunks of 8 MiB; the last one's first chunk fails
+C.c_int.in_dll(shim, "armed").value = -(-b.nbytes // (8 << 20)) + 1
+last_kib = C.c_void_p(got.ctypes.data), C.c_void_p(xd[-1] + b.nbytes - 1024), C.c_size_t(1024), 2
+st = solve()
+# on the null stream, which does not wait for the library's
+err = hip.hipMemcpy(*last_kib)
+assert err == 0 and st != 0 and C.c_int.in_dll(shim, "failed").value == 1
+assert np.array_equal(got.reshape(-1)[:128], want.reshape(-1)[-128:])
+assert solve() == 0, kq.last_error()
+kq.kuqcd_gauge_free()
+kq.kuqcd_end()
+"""
+
+
+@pytest.mark.gpu
+def test_nothing_runs_on_after_an_error(gpu, tmp_path):
+    """A solve whose last solution cannot be copied to the host (a shim fails that copy) has returned with
+    the device arrays of the others written: no kernel on the caller's memory is left running."""
+    src, shim = tmp_path / "shim.c", tmp_path / "libshim.so"
+    src.write_text(_FAILING_COPY)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-D_GNU_SOURCE", "-I/opt/rocm/include", str(src), "-o", str(shim), "-ldl"],
+                   check=True, timeout=60)
+    r = subprocess.run([sys.executable, "-c", _AFTER_ERROR.format(root=str(ROOT), shim=str(shim))], env=dict(os.environ),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
