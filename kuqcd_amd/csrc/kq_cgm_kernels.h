@@ -60,7 +60,6 @@ __host__ __device__ inline size_t hist_scalar_index(int dslot, int j, int field,
 
 struct CgmLaunch {
     uint32_t Vh;
-    uint32_t nblk;      // blocks of the BLAS site loops (= stride of part_b)
     uint32_t nblk_dsl = 0;  // blocks of the hopping-term launch (= stride of part_a)
     int nsys;           // system slots (k_cgm_begin scans all of them)
     int nlaunch;        // slots of the live list the per-system kernels cover (>= live systems)

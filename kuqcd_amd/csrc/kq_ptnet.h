@@ -101,7 +101,6 @@ void loss_scale(const double2 *part_loss, float2 *g, const float2 *r, size_t n, 
 uint32_t pt_layer_nblk(uint32_t Vh);
 
 // ---- FP32 vector helpers (n complex entries)
-void vf_axpy(float2 *y, const float2 *x, float2 a, size_t n, hipStream_t st);  // y += a x (complex a)
 void vf_lincomb(float2 *y, const float2 *x1, float2 a1, const float2 *x2, float2 a2, size_t n,
                 hipStream_t st);                                                   // y = a1 x1 + a2 x2
 // several complex dot products <x_i, y_i> (sum over n complex entries) in one launch; out: host

@@ -446,15 +446,6 @@ __global__ void __launch_bounds__(kNT) k_reduce_cols(const double2 *part, uint32
         *out = mk<double2>(lre[0], lim[0]);
 }
 
-__global__ void k_vf_axpy(float2 *y, const float2 *x, float2 a, size_t n)
-{
-    const size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
-    if (i < n) {
-        const float2 p = cmulf(a, x[i]);
-        y[i] = mk<float2>(y[i].x + p.x, y[i].y + p.y);
-    }
-}
-
 __global__ void k_vf_lincomb(float2 *y, const float2 *x1, float2 a1, const float2 *x2, float2 a2, size_t n)
 {
     const size_t i = (size_t)blockIdx.x * kNT + threadIdx.x;
@@ -797,14 +788,6 @@ PtWeights pt_effective(const PtWeights &w, const PtNorms &nu)
 }
 
 // ---------------------------------------------------------------- vector helpers
-void vf_axpy(float2 *y, const float2 *x, float2 a, size_t n, hipStream_t st)
-{
-    if (n == 0)
-        return;
-    hipLaunchKernelGGL(k_vf_axpy, dim3(grid_of(n)), dim3(kNT), 0, st, y, x, a, n);
-    KQ_HIP_CHECK(hipGetLastError());
-}
-
 void vf_lincomb(float2 *y, const float2 *x1, float2 a1, const float2 *x2, float2 a2, size_t n, hipStream_t st)
 {
     if (n == 0)

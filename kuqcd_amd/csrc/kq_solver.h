@@ -611,7 +611,6 @@ private:
     {
         CgmLaunch L;
         L.Vh = g_.Vh;
-        L.nblk = nblk_;
         L.nsys = max_sys_;
         L.nlaunch = std::min(std::max(nlaunch, 1), max_sys_);
         L.rlist = max_sys_ > 1 ? rlist() : nullptr;
