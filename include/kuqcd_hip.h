@@ -99,7 +99,11 @@ KQ_API KuQCDStatus kq_solve_multishift_batched(int nrhs, void **x, void **b, KuQ
  * src on parity 1-dst_parity, host buffers in the gauge precision;
  * mode picks the device link/vector format (KqMode; REFERENCE = as loaded). */
 KQ_API KuQCDStatus kq_dslash(const void *src, void *dst, int dst_parity, int mode);
-/* nrhs vectors back to back (host layout each); nr/nt as in KqSolveOptions */
+/* nrhs vectors back to back (host layout each); nr (1, 2, 3, 4 or 8) and nt (64, 128 or 256) as in
+ * KqSolveOptions, but not 0. They are the blocking and block size of the mixed modes' kernel where
+ * that has a choice. In the loaded precision they are hints: blocks of more than 2 FP64 vectors run as
+ * blocks of 2, blocks of 4 FP32 vectors out of more than 4 as blocks of 8 where that is faster, and the
+ * kernel has a block size of its own. The results differ by rounding at most. */
 KQ_API KuQCDStatus kq_dslash_batched(int nrhs, const void *src, void *dst, int dst_parity, int mode, int nr, int nt);
 /* dst = sigma*src - D D src on parity `parity` (the CGM operator A) */
 KQ_API KuQCDStatus kq_mdaggm(const void *src, void *dst, int parity, double sigma, int mode);
@@ -127,7 +131,9 @@ typedef struct {
 KQ_API KuQCDStatus kq_bench_dslash(int mode, int nrhs, int nr, int nt, int iters, KqBenchResult *out);
 /* plain device copy of `bytes` bytes (HBM reference point) */
 KQ_API KuQCDStatus kq_bench_copy(size_t bytes, int iters, KqBenchResult *out);
-/* pick nr, nt for (mode, nrhs) on the loaded lattice by timing; cached */
+/* pick nr, nt for (mode, nrhs) on the loaded lattice by timing; cached. This and kq_bench_dslash time
+ * the hopping term on the solvers' own vectors (colour planes), as the solvers and the mixed modes run
+ * it; kq_dslash_batched in the loaded precision works on the caller's layout with another kernel */
 KQ_API KuQCDStatus kq_autotune_dslash(int mode, int nrhs, int *nr, int *nt);
 
 /* ---- synthetic inputs (reference host layouts, double precision) */
