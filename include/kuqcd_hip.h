@@ -101,9 +101,9 @@ KQ_API KuQCDStatus kq_solve_multishift_batched(int nrhs, void **x, void **b, KuQ
 KQ_API KuQCDStatus kq_dslash(const void *src, void *dst, int dst_parity, int mode);
 /* nrhs vectors back to back (host layout each); nr (1, 2, 3, 4 or 8) and nt (64, 128 or 256) as in
  * KqSolveOptions, but not 0. They are the blocking and block size of the mixed modes' kernel where
- * that has a choice. In the loaded precision they are hints: blocks of more than 2 FP64 vectors run as
- * blocks of 2, blocks of 4 FP32 vectors out of more than 4 as blocks of 8 where that is faster, and the
- * kernel has a block size of its own. The results differ by rounding at most. */
+ * that has a choice. In the loaded precision they are hints: with nr above 2 FP64 vectors run in blocks
+ * of 2, 3, 4 or at most nr, whichever is fastest, blocks of 4 FP32 vectors out of more than 4 as blocks of 8 where
+ * that is, and the kernel has a block size of its own. The results differ by rounding at most. */
 KQ_API KuQCDStatus kq_dslash_batched(int nrhs, const void *src, void *dst, int dst_parity, int mode, int nr, int nt);
 /* dst = sigma*src - D D src on parity `parity` (the CGM operator A) */
 KQ_API KuQCDStatus kq_mdaggm(const void *src, void *dst, int parity, double sigma, int mode);

@@ -35,6 +35,9 @@ template <class LF, class LL, typename SR> struct DslashArgs {
 
 // block sizes launch_dslash accepts: 64, 128 and 256 threads
 constexpr int kMinDslashNT = 64;
+// Most sites of one parity (times the blocks of vectors) for which the split hopping term is the rule
+// (dslash_split_waves), in FP64 and FP32
+constexpr uint32_t kSplitSites64 = 49152, kSplitSites32 = 98304;
 // Block size of the hopping terms whose partial sums feed the reference method, the plain
 // FP64 solve and the FP64 verification. One partial per workgroup, added in a fixed order,
 // makes a reduction deterministic for a given block size; fixing the block size by the lattice
@@ -77,10 +80,31 @@ void launch_dslash_p(DslashArgs<LF, LL, SR> a, CgmState<SR> *st, const c2_t<SR> 
 // launch_dslash on vectors of the loaded gauge's precision in the caller's host layout (device memory,
 // aligned to their reals): lay LAY_HOST with EPI_STORE (D src, nr right-hand sides per block), or
 // the two terms of sigma0 src - D D src on one right-hand side, LAY_HOST_SRC with EPI_STORE and
-// LAY_HOST_DST with EPI_AXMY, whose intermediate is in colour planes. The vectors of one launch
+// LAY_HOST_DST with EPI_AXMY, whose intermediate is in colour planes; or, in FP64, LAY_HOST_DST with
+// EPI_STORE in blocks of 3, 4 or 8 (host_planes_block). The vectors of one launch
 // must not overlap, except that aux and dst may be the same vector.
 template <class LF, class LL, typename SR>
 void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int nr, hipStream_t st);
+
+// Block size for nrhs FP64 vectors in the host layout, of which the caller wants blocks of nr, if their
+// source is first converted to colour planes, or 0 if the split term reads it as it is, in blocks of 2.
+// Blocks of 3 and more would spill in the split form; with one thread per site they read the links
+// less often, which pays above the sizes that the split term is for. Calls in blocks of 2 -> this,
+// nr = 4 (nr = 8): 16^3x32 8 vectors 139 -> 113 us (104); 24^4 3 vectors 169 -> 124, 5 250 -> 218
+// (173), 8 342 -> 256 (247); 32^4 3 500 -> 326, 5 750 -> 600 (422), 8 1027 -> 704 (678); 48^4 8
+// 5450 -> 3521 (3353). Reading the host layout in blocks of 8 as well, without the conversion: 32^4 1287,
+// 48^4 6307. The block is the one of least weight over all vectors: 29, 33 and 55 per block of 3, 4 and 8
+// pick the faster one for 3 to 12 vectors at these sizes (padding costs less than its slots, since it
+// repeats a vector).
+inline int host_planes_block(const Geom &g, int nrhs, int nr)
+{
+    if (nr < 3 || nrhs < 3 || g.Vh <= kSplitSites64)
+        return 0;
+    const int c3 = (nrhs + 2) / 3 * 29, c4 = (nrhs + 3) / 4 * 33, c8 = (nrhs + 7) / 8 * 55;
+    if (nr == 8 && c8 < c3 && c8 < c4)
+        return 8;
+    return c3 < c4 ? 3 : 4;
+}
 
 // Workgroups of nt sites for Vh sites, rounded up to a multiple of the 8 XCDs so that tile_site can
 // give each XCD a contiguous range of sites on any lattice (the last ones may be empty)
@@ -133,7 +157,6 @@ inline bool dslash_staged(const Geom &g, int nr, int nt)
 // verification, whose results are the same in every process (repro_nt). Two or more FP64 vectors
 // run faster as pairs on either form (two vectors in single blocks -> a pair: 16^4 20.7 -> 13.1 us, 24^4
 // 115 -> 65, 32^4 354 -> 193, 48^4 1948 -> 1077; only at 8^4 4.4 -> 5.0), so the rule follows those.
-constexpr uint32_t kSplitSites64 = 49152, kSplitSites32 = 98304;
 inline int dslash_split_waves(bool fp64, const Geom &g, int nrhs, int nr)
 {
     if (fp64)

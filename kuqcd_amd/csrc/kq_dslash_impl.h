@@ -232,9 +232,17 @@ __device__ __forceinline__ void dslash_epilogue(const A &a, const R (&acc)[NR][6
             for (int j = 0; j < NR; ++j) {
                 // padding slots repeat the last live right-hand side, so the
                 // store is unconditional (same value to the same address)
+                V2 o[3];
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
-                    put<LF>(&dst[j][(size_t)c * Vh + s], mk<V2>((SR)acc[j][2 * c], (SR)acc[j][2 * c + 1]));
+                    o[c] = mk<V2>((SR)acc[j][2 * c], (SR)acc[j][2 * c + 1]);
+                if constexpr (AOS) {
+                    st_site(dst[j] + (size_t)3 * s, o);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c)
+                        put<LF>(&dst[j][(size_t)c * Vh + s], o[c]);
+                }
             }
         }
     } else if constexpr (EPI == EPI_AXMY) {
@@ -843,6 +851,16 @@ static void launch_host_nt(DslashArgs<LF, LL, SR> a, int lay, int epi, hipStream
     KQ_HIP_CHECK(hipGetLastError());
 }
 
+// Source in colour planes, destination in the host layout, one thread per site and block of NR vectors
+template <class LF, class LL, typename SR, int NR>
+static void launch_host_block(DslashArgs<LF, LL, SR> a, hipStream_t st)
+{
+    a.nblk = dslash_grid(a.g.Vh, 256);
+    hipLaunchKernelGGL((k_dslash<LF, LL, SR, NR, EPI_STORE, 256, LAY_HOST_DST>), dim3(a.nblk, (a.nrhs + NR - 1) / NR),
+                       dim3(256), 0, st, a);
+    KQ_HIP_CHECK(hipGetLastError());
+}
+
 template <class LF, class LL, typename SR>
 void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int nr, hipStream_t st)
 {
@@ -855,7 +873,7 @@ void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int n
         // strides. Per launch, one thread per site -> split: FP64, one right-hand side, 24^4
         // 67.6 -> 65 us, 32^4 206 -> 196, 48^4 1087 -> 1015; FP32, 8 right-hand sides in blocks of
         // 4, 24^4 110 -> 82, 48^4 1597 -> 1382; in one block of 8 (S = 4), 24^4 90 -> 63. FP64
-        // blocks above 2 spill, so larger ones run as blocks of 2.
+        // blocks above 2 spill, so larger ones run as blocks of 2 (or not here: host_planes_block).
         if constexpr (kDouble) {
             if (nr >= 2)
                 launch_host_split<LF, LL, SR, 2, 8>(a, lay, epi, st);
@@ -890,6 +908,17 @@ void launch_dslash_host(const DslashArgs<LF, LL, SR> &a, int lay, int epi, int n
             }
         }
         return;
+    }
+    if constexpr (kDouble) {
+        if (lay == LAY_HOST_DST && epi == EPI_STORE) {
+            if (nr == 3)
+                launch_host_block<LF, LL, SR, 3>(a, st);
+            else if (nr == 4)
+                launch_host_block<LF, LL, SR, 4>(a, st);
+            else
+                launch_host_block<LF, LL, SR, 8>(a, st);
+            return;
+        }
     }
     // One side in the host layout (A = sigma - D D, one right-hand side): split up to the size at
     // which one thread per site fills the chip, measured per term, one thread -> split: FP64

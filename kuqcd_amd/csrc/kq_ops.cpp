@@ -19,7 +19,8 @@ static bool overlap(const void *p, const void *q, size_t bytes)
 // In the loaded precision the hopping terms read and write the caller's host layout themselves, so
 // device arrays are used in place: converting them to colour planes and back cost two kernels,
 // two device-to-device copies and their gaps around every vector (A at 8^4 to 32^4: see
-// k_dslash_split; 8 FP32 right-hand sides at 24^4: 290 us for a 98 us kernel). Arrays that a kernel
+// k_dslash_split; 8 FP32 right-hand sides at 24^4: 290 us for a 98 us kernel).
+// Only FP64 blocks of 3 and more convert their source (host_planes_block). Arrays that a kernel
 // cannot use in place (host memory, another GPU's, addresses that are not a multiple of a real, a
 // source that overlaps the destination) go through a device buffer in the same layout.
 template <class LF, class LL, typename R>
@@ -51,7 +52,16 @@ static void apply_host(LF fat, LL lng, const Geom &g, int nrhs, const void *src,
         a.dst_parity = dst_parity;
         a.src = Vec<R>{reinterpret_cast<c2_t<R> *>(const_cast<R *>(from)), g.Vh, n3};
         a.dst = Vec<R>{reinterpret_cast<c2_t<R> *>(to), g.Vh, n3};
-        launch_dslash_host(a, LAY_HOST, EPI_STORE, nr, c.stream);
+        const int block = std::is_same<R, double>::value ? host_planes_block(g, nrhs, nr) : 0;
+        if (block > 0) {
+            t.alloc(bytes);
+            a.src.p = t.as<c2_t<R>>();
+            for (int r = 0; r < nrhs; ++r)
+                vec_host_to_soa<R, R>(from + 2 * n3 * (size_t)r, a.src, r, c.stream);
+            launch_dslash_host(a, LAY_HOST_DST, EPI_STORE, block, c.stream);
+        } else {
+            launch_dslash_host(a, LAY_HOST, EPI_STORE, nr, c.stream);
+        }
     }
     if (put_back)
         copy_to_host(dst, to, bytes, c.stream);

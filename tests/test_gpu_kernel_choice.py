@@ -1,4 +1,5 @@
 """Which kernel a hopping term runs on, and that what may not depend on that choice does not."""
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -192,3 +193,38 @@ def test_staged_rows_bitwise_equal_to_unstaged(gpu, tmp_path, lat):
                        timeout=100)
     assert r.returncode == 0, r.stderr[-2000:]
     assert np.array_equal(out, np.load(path))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("links", ["su3", "u3", "general"])
+def test_fp64_blocks_on_large_lattices(gpu, links):
+    """FP64 vectors in blocks of 3, 4 and 8 above the sizes of the split term run on colour planes of the
+    source, one thread per site, and write the caller's layout: whole, padded and single blocks against the
+    oracle (1e-13) and blocks of 2, from device arrays aligned to one real, host arrays, and a source that
+    overlaps the destination."""
+    kq, L, lat = gpu, gpu.L.lib(), (18, 18, 18, 18)
+    fat, lng = _load(kq, lat, u3=links == "u3", general=links == "general")
+    src = np.stack([kq.gen_source(lat, 0, seed=90 + r) for r in range(9)])
+    want = np.stack([oracle.dslash(fat, lng, v, lat, 1) for v in src])
+    base = L.kq_device_alloc(2 * src.nbytes + 64)
+    s, d = base + 8, base + 8 + src.nbytes
+    out = np.empty_like(src)
+    try:
+        for n in (1, 2, 3, 4, 5, 9):
+            for nr in (2, 3, 4, 8):
+                print("case", links, n, nr, flush=True)
+                assert L.kq_memcpy(s, src.ctypes.data, src.nbytes) == 0
+                size = n * src[0].nbytes
+                assert L.kq_dslash_batched(n, C.c_void_p(s), C.c_void_p(d), 1, 0, nr, 256) == 0, kq.last_error()
+                assert L.kq_memcpy(out.ctypes.data, d, size) == 0
+                assert all(rel_err(out[r], want[r]) <= 1e-13 for r in range(n))
+                host = np.full_like(src[:n], np.nan)
+                assert kq.dslash_batched(np.ascontiguousarray(src[:n]), host, 1, 0, nr, 256) == 0, kq.last_error()
+                assert np.array_equal(host, out[:n])
+                # over the source's second half (which is no longer its own afterwards)
+                at = s + size // 2
+                assert L.kq_dslash_batched(n, C.c_void_p(s), C.c_void_p(at), 1, 0, nr, 256) == 0, kq.last_error()
+                assert L.kq_memcpy(host.ctypes.data, at, size) == 0
+                assert np.array_equal(host, out[:n])
+    finally:
+        L.kq_device_free(base)
