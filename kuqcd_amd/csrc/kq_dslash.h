@@ -149,7 +149,7 @@ inline bool dslash_staged(const Geom &g, int nr, int nt)
 // 14.5 -> 12.6, 20^4 19.0 -> 16.4, 24^4 29.8 -> 31.2; blocks of 4: 16^4 21.8 -> 12.4, 16^3x32
 // 23.8 -> 21.1, but two groups of 4 there 33 -> 37, 24^4 50 -> 47 (47.6 in workgroups of 64).
 // Blocks of 8 FP32 right-hand sides leave the one-thread form one wave per SIMD, waiting for its
-// gathers: split into 4 waves (or 2, launch_epi) at every size, 16^4 41 -> 18, 24^4 82 -> 75, 48^4
+// gathers: split into 4 waves (or 2, hop_kernel) at every size, 16^4 41 -> 18, 24^4 82 -> 75, 48^4
 // 1316 -> 1118, except where the larger lattices stage rows in LDS (32^4: 174 staged, 203 split).
 //
 // The two forms add the 16 hops in different orders. The FP64 rule therefore counts blocks of 2
